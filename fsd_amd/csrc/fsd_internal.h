@@ -149,26 +149,33 @@ struct LubTable {
     float table_min, table_dr;
 };
 
-// Interpolate `ncol` resistance functions starting at column c0
+// Interpolate NCOL resistance functions starting at column C0
 // (Lubrication.cu:172-231); contact_row < 0 disables the r <= 2.001 clamp.
-__device__ inline void lub_lookup(const LubTable &t, float dist, int c0, int ncol, int contact_row, float *out)
+// C0 and NCOL are even and a row is 88 bytes, so a row is read as float2.
+template <int C0, int NCOL>
+__device__ __forceinline__ void lub_lookup(const LubTable &t, float dist, int contact_row, float *out)
 {
-    if ((double)dist <= 2.001 && contact_row >= 0) {
-        for (int c = 0; c < ncol; ++c) out[c] = t.vals[22 * contact_row + c0 + c];
-        return;
-    }
-    float arg = (float)(((double)dist - 2.0) / (double)t.table_min);
-    int ind = (int)(log10f(arg) / t.table_dr);
+    static_assert(C0 % 2 == 0 && NCOL % 2 == 0, "pairs of columns");
+    const bool contact = (double)dist <= 2.001 && contact_row >= 0;
+    const float arg = (float)(((double)dist - 2.0) / (double)t.table_min);
+    int ind = contact ? contact_row : (int)(log10f(arg) / t.table_dr);
     ind = ind < 0 ? 0 : ind;
-    if (ind >= 999) {  // r in [~3.99968, 4): the reference reads past the distance array; row 999 is zero
-        for (int c = 0; c < ncol; ++c) out[c] = t.vals[22 * 999 + c0 + c];
+    // r in [~3.99968, 4): the reference reads past the distance array; row 999 is zero
+    const bool flat = contact || ind >= 999;
+    ind = ind >= 999 ? 999 : ind;
+    const float2 *lo = reinterpret_cast<const float2 *>(t.vals + 22 * ind + C0);
+    if (flat) {
+#pragma unroll
+        for (int c = 0; c < NCOL / 2; ++c) { out[2 * c] = lo[c].x; out[2 * c + 1] = lo[c].y; }
         return;
     }
-    float dl = t.dist[ind], du = t.dist[ind + 1];
-    float fac = (dist - dl) / (du - dl);
-    for (int c = 0; c < ncol; ++c) {
-        float lo = t.vals[22 * ind + c0 + c], hi = t.vals[22 * (ind + 1) + c0 + c];
-        out[c] = lo + (hi - lo) * fac;
+    const float dl = t.dist[ind], du = t.dist[ind + 1];
+    const float fac = (dist - dl) / (du - dl);
+#pragma unroll
+    for (int c = 0; c < NCOL / 2; ++c) {
+        const float2 l = lo[c], h = lo[11 + c];
+        out[2 * c] = l.x + (h.x - l.x) * fac;
+        out[2 * c + 1] = l.y + (h.y - l.y) * fac;
     }
 }
 
@@ -216,11 +223,11 @@ struct fsd_ctx {
     int *d_nneigh = nullptr, *d_nlist = nullptr;
     int ncell[3] = {0, 0, 0}; int ncells = 0; bool use_cells = false;
     int *d_cell_of = nullptr, *d_cell_count = nullptr, *d_cell_start = nullptr, *d_cell_list = nullptr;
-    int *d_flags = nullptr;     // [0] nlist overflow, [1] lub overflow, [2] prune overflow, [4] nlist entries,
-                                // [5] lubrication pairs, [6] some particle moved r_buff / 2 since the list
+    int *d_flags = nullptr;     // [0] nlist overflow, [2] prune overflow, [4] nlist entries, [8] lub overflow,
+                                // [9] lubrication pairs
     float4 *d_pos_last = nullptr;   // positions the neighbour list was built at
     int64_t nlist_builds = 0;       // neighbour lists built by this context
-    int *h_flags = nullptr;     // pinned mirror
+    int *h_flags = nullptr;     // pinned mirror; [6] (host only) some particle moved r_buff / 2 since the list
     bool nlist_valid = false;
     int64_t nlist_total = 0;
 

@@ -194,7 +194,7 @@ __global__ void lp_edge_feat_kernel(int64_t E, const int *erow, const int *lcol,
     if ((double)dist <= 2.0 + (double)t.table_min) {
         for (int c = 0; c < 10; ++c) v[c] = t.vals[c];
     } else {
-        lub_lookup(t, dist, 0, 10, -1, v);
+        lub_lookup<0, 10>(t, dist, -1, v);
     }
     float *g = geo + e * 8;
     g[0] = dx / dist; g[1] = dy / dist; g[2] = dz / dist;

@@ -3,6 +3,7 @@
 // pair records turn every R_FU apply of the GMRES loop into a pure block
 // gather with no table lookups.
 #include "fsd_internal.h"
+#include "pair_scan.h"
 
 // ---------------------------------------------------------------- scans
 // single-workgroup exclusive scan (n up to a few 10^5); out[n] = total
@@ -40,22 +41,6 @@ __global__ void __launch_bounds__(1024) scan_excl_kernel(const int *in, int *out
         __syncthreads();
     }
     if (tid == 0) out[n] = carry;
-}
-
-// total of n ints into *out (single workgroup)
-__global__ void __launch_bounds__(1024) sum_int_kernel(const int *in, int n, int *out)
-{
-    __shared__ int part[16];
-    int s = 0;
-    for (int i = threadIdx.x; i < n; i += 1024) s += in[i];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < 16; ++w) t += part[w];
-        *out = t;
-    }
 }
 
 int scan_excl(fsd_ctx *ctx, const int *in, int *out, int n)
@@ -155,74 +140,108 @@ __global__ void cell_scatter_kernel(const int *cell_of, int N, const int *start,
     list[start[c] + slot] = i;
 }
 
-// deterministic order inside a cell: ascending particle index
-__global__ void cell_sort_kernel(const int *start, int ncells, int *list)
+// deterministic order inside a cell: ascending particle index, one wave per cell.  A cell of up to
+// 256 particles is held in registers (four per lane) and each key stored at its rank, the number of
+// smaller keys (the keys differ); a fuller one (spheres that overlap) is sorted by one lane.
+__global__ void __launch_bounds__(64) cell_sort_kernel(const int *start, int ncells, int *list)
 {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ncells) return;
-    int s = start[c], e = start[c + 1];
-    for (int a = s + 1; a < e; ++a) {
-        int key = list[a], q = a - 1;
-        while (q >= s && list[q] > key) { list[q + 1] = list[q]; --q; }
-        list[q + 1] = key;
+    __shared__ int keys[256];
+    const int s = start[blockIdx.x], n = start[blockIdx.x + 1] - s, lane = threadIdx.x;
+    if (n > 256) {
+        if (lane == 0)
+            for (int a = s + 1; a < s + n; ++a) {
+                int key = list[a], q = a - 1;
+                while (q >= s && list[q] > key) { list[q + 1] = list[q]; --q; }
+                list[q + 1] = key;
+            }
+        return;
+    }
+    for (int a = lane; a < n; a += 64) keys[a] = list[s + a];
+    __syncthreads();
+    for (int a = lane; a < n; a += 64) {
+        const int key = keys[a];
+        int rank = 0;
+        for (int q = 0; q < n; ++q) rank += keys[q] < key;
+        list[s + rank] = key;
     }
 }
 
-__global__ void nlist_cells_kernel(const float4 *pos, int N, BoxF b, int cx, int cy, int cz, const int *cell_of,
-                                   const int *start, const int *list, float rl2, int maxn, int *nneigh, int *nlist,
-                                   int *overflow)
+// One entry run [q0, q1) of the cell-sorted particles (list null: the particles q0 .. q1 - 1
+// themselves) tested against particle i by its 16 lanes; the neighbours are appended to its row in
+// the run's order.  Returns the new count (which may exceed maxn; entries beyond it are dropped).
+__device__ __forceinline__ int nlist_run(const float4 *pos, const BoxF &b, float4 pi, int i, const int *list, int q0,
+                                         int q1, int lane, float rl2, int maxn, int *row, int cnt)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
-    int c = cell_of[i];
-    int ix = c / (cy * cz), iy = (c / cz) % cy, iz = c % cz;
-    int cnt = 0;
-    for (int dx = -1; dx <= 1; ++dx) {
-        int jx = ix + dx; jx = jx < 0 ? jx + cx : (jx >= cx ? jx - cx : jx);
-        for (int dy = -1; dy <= 1; ++dy) {
-            int jy = iy + dy; jy = jy < 0 ? jy + cy : (jy >= cy ? jy - cy : jy);
-            for (int dz = -1; dz <= 1; ++dz) {
-                int jz = iz + dz; jz = jz < 0 ? jz + cz : (jz >= cz ? jz - cz : jz);
-                int cc = (jx * cy + jy) * cz + jz;
-                for (int q = start[cc]; q < start[cc + 1]; ++q) {
-                    int j = list[q];
-                    if (j == i) continue;
-                    float4 pj = pos[j];
-                    float ddx = pj.x - pi.x, ddy = pj.y - pi.y, ddz = pj.z - pi.z;
-                    box_min_image(b, ddx, ddy, ddz);
-                    if (dist2_nc(ddx, ddy, ddz) < rl2) {
-                        if (cnt < maxn) nlist[(int64_t)i * maxn + cnt] = j;
-                        ++cnt;
-                    }
-                }
+    const int first = (threadIdx.x & 63) & ~(PG - 1);
+    for (int k = q0; k < q1; k += PG) {
+        const bool in = k + lane < q1;
+        const int q = in ? k + lane : q0;
+        const int j = list ? list[q] : q;
+        const float4 pj = pos[j];
+        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+        box_min_image(b, dx, dy, dz);
+        const bool ok = in && j != i && dist2_nc(dx, dy, dz) < rl2;
+        const unsigned m = (unsigned)(__ballot(ok) >> first) & 0xffffu;
+        const int o = cnt + __popc(m & ((1u << lane) - 1u));
+        if (ok && o < maxn) row[o] = j;
+        cnt += __popc(m);
+    }
+    return cnt;
+}
+
+// 16 lanes per particle, particles in cell order.  Bound by the latency of its dependent loads (cell
+// start, particle, position); the three cells along z of a column are one run of the sorted particles,
+// two where the column wraps.
+__global__ void __launch_bounds__(PGB) nlist_cells_kernel(const float4 *pos, int N, BoxF b, int cx, int cy, int cz,
+                                                          const int *cell_of, const int *start, const int *list,
+                                                          float rl2, int maxn, int *nneigh, int *nlist, int *overflow,
+                                                          int *total)
+{
+    __shared__ int s_cnt[PGB / PG];
+    int lane;
+    const int i = pg_particle(N, list, lane);
+    int cnt = -1;
+    if (i >= 0) {
+        const float4 pi = pos[i];
+        const int c = cell_of[i];
+        const int ix = c / (cy * cz), iy = (c / cz) % cy, iz = c % cz;
+        int *row = nlist + (int64_t)i * maxn;
+        cnt = 0;
+        for (int o = 0; o < 9; ++o) {
+            int jx = ix + o / 3 - 1, jy = iy + o % 3 - 1;
+            jx = jx < 0 ? jx + cx : (jx >= cx ? jx - cx : jx);
+            jy = jy < 0 ? jy + cy : (jy >= cy ? jy - cy : jy);
+            const int *st = start + (jx * cy + jy) * cz;
+            if (iz == 0) {
+                cnt = nlist_run(pos, b, pi, i, list, st[cz - 1], st[cz], lane, rl2, maxn, row, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[0], st[2], lane, rl2, maxn, row, cnt);
+            } else if (iz == cz - 1) {
+                cnt = nlist_run(pos, b, pi, i, list, st[cz - 2], st[cz], lane, rl2, maxn, row, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[0], st[1], lane, rl2, maxn, row, cnt);
+            } else {
+                cnt = nlist_run(pos, b, pi, i, list, st[iz - 1], st[iz + 2], lane, rl2, maxn, row, cnt);
             }
         }
+        if (lane == 0) nneigh[i] = cnt < maxn ? cnt : maxn;
     }
-    if (cnt > maxn) atomicMax(overflow, cnt);
-    nneigh[i] = cnt < maxn ? cnt : maxn;
+    if (lane == 0) s_cnt[threadIdx.x / PG] = cnt;
+    pg_block_counts(s_cnt, maxn, overflow, total);
 }
 
 // small boxes (fewer than 3 cells along an axis): all pairs
-__global__ void nlist_allpairs_kernel(const float4 *pos, int N, BoxF b, float rl2, int maxn, int *nneigh, int *nlist,
-                                      int *overflow)
+__global__ void __launch_bounds__(PGB) nlist_allpairs_kernel(const float4 *pos, int N, BoxF b, float rl2, int maxn,
+                                                             int *nneigh, int *nlist, int *overflow, int *total)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
-    int cnt = 0;
-    for (int j = 0; j < N; ++j) {
-        if (j == i) continue;
-        float4 pj = pos[j];
-        float ddx = pj.x - pi.x, ddy = pj.y - pi.y, ddz = pj.z - pi.z;
-        box_min_image(b, ddx, ddy, ddz);
-        if (dist2_nc(ddx, ddy, ddz) < rl2) {
-            if (cnt < maxn) nlist[(int64_t)i * maxn + cnt] = j;
-            ++cnt;
-        }
+    __shared__ int s_cnt[PGB / PG];
+    int lane;
+    const int i = pg_particle(N, nullptr, lane);
+    int cnt = -1;
+    if (i >= 0) {
+        cnt = nlist_run(pos, b, pos[i], i, nullptr, 0, N, lane, rl2, maxn, nlist + (int64_t)i * maxn, 0);
+        if (lane == 0) nneigh[i] = cnt < maxn ? cnt : maxn;
     }
-    if (cnt > maxn) atomicMax(overflow, cnt);
-    nneigh[i] = cnt < maxn ? cnt : maxn;
+    if (lane == 0) s_cnt[threadIdx.x / PG] = cnt;
+    pg_block_counts(s_cnt, maxn, overflow, total);
 }
 
 // NeighborList::distanceCheck of HOOMD: some particle has moved at least r_buff / 2 (minimum
@@ -244,13 +263,16 @@ int k_update_nlist(fsd_ctx *ctx, const float4 *pos, bool *rebuilt)
     *rebuilt = false;
     if (ctx->nlist_valid) {
         const float half = 0.5f * ctx->p.r_buff;
-        FSD_HIP(hipMemsetAsync(ctx->d_flags + 6, 0, sizeof(int), ctx->stream));
+        // the kernel stores into the pinned host flag itself (a store per moved particle, none in the
+        // usual call): one launch where clearing, copying and reading a device flag were three.
+        // Nothing of this context is in flight on the flag: every call drains the stream.
+        volatile int *moved = ctx->h_flags + 6;
+        *moved = 0;
         hipLaunchKernelGGL(max_disp_kernel, dim3(nblk(ctx->N, 256)), dim3(256), 0, ctx->stream, pos, ctx->d_pos_last,
-                           ctx->N, ctx->box, half * half, ctx->d_flags + 6);
+                           ctx->N, ctx->box, half * half, ctx->h_flags + 6);
         FSD_HIP(hipGetLastError());
-        FSD_HIP(hipMemcpyAsync(ctx->h_flags + 6, ctx->d_flags + 6, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FSD_HIP(hipStreamSynchronize(ctx->stream));
-        if (!ctx->h_flags[6]) return 0;
+        if (!*moved) return 0;
     }
     *rebuilt = true;
     return k_build_nlist(ctx, pos);
@@ -273,17 +295,16 @@ int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
             FSD_HIP(hipMemsetAsync(ctx->d_cell_count, 0, sizeof(int) * ctx->ncells, ctx->stream));
             hipLaunchKernelGGL(cell_scatter_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, ctx->d_cell_of, N,
                                ctx->d_cell_start, ctx->d_cell_count, ctx->d_cell_list);
-            hipLaunchKernelGGL(cell_sort_kernel, dim3(nblk(ctx->ncells, 128)), dim3(128), 0, ctx->stream,
+            hipLaunchKernelGGL(cell_sort_kernel, dim3(ctx->ncells), dim3(64), 0, ctx->stream,
                                ctx->d_cell_start, ctx->ncells, ctx->d_cell_list);
-            hipLaunchKernelGGL(nlist_cells_kernel, dim3(nblk(N, 128)), dim3(128), 0, ctx->stream, pos, N, ctx->box,
+            hipLaunchKernelGGL(nlist_cells_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
                                ctx->ncell[0], ctx->ncell[1], ctx->ncell[2], ctx->d_cell_of, ctx->d_cell_start,
-                               ctx->d_cell_list, rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags);
+                               ctx->d_cell_list, rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags, ctx->d_flags + 4);
         } else {
-            hipLaunchKernelGGL(nlist_allpairs_kernel, dim3(nblk(N, 128)), dim3(128), 0, ctx->stream, pos, N, ctx->box,
-                               rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags);
+            hipLaunchKernelGGL(nlist_allpairs_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
+                               rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags, ctx->d_flags + 4);
         }
         FSD_HIP(hipGetLastError());
-        hipLaunchKernelGGL(sum_int_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->d_nneigh, N, ctx->d_flags + 4);
         FSD_HIP(hipMemcpyAsync(ctx->h_flags, ctx->d_flags, 8 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FSD_HIP(hipStreamSynchronize(ctx->stream));
         int need = ctx->h_flags[0];
@@ -307,55 +328,74 @@ int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
 }
 
 // -------------------------------------------------- lubrication records
-// One thread per particle: select neighbours with 0 < r^2 < rlub^2, store
-// the pair record and accumulate the particle's 6x6 self block
-// (Lubrication.cu:147-296 split into j- and i-side terms).
-__global__ void lub_pairs_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn,
-                                 LubTable t, float rl2, int maxlub, int *lub_n, int *lub_j, float4 *lub_a,
-                                 float4 *lub_b, float *lub_self, int *overflow)
+// Neighbours with 0 < r^2 < rlub^2: the pair records in list order, and the
+// particle's 6x6 self block (Lubrication.cu:147-296 split into j- and i-side
+// terms), a sum over its pairs of 17 terms (r r, the identity and eps.r times
+// their resistance functions), summed over the 16 lanes by DPP.
+__global__ void __launch_bounds__(PGB) lub_pairs_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                        const int *nlist, int maxn, LubTable t, float rl2, int maxlub,
+                                                        int *lub_n, int *lub_j, float4 *lub_a, float4 *lub_b,
+                                                        float *lub_self, int *overflow, int *total, const int *order)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
-    float S[36];
-    for (int q = 0; q < 36; ++q) S[q] = 0.f;
-    int cnt = 0;
-    const int nn = nneigh[i];
-    for (int k = 0; k < nn; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
-        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        box_min_image(b, dx, dy, dz);
-        float d2 = dist2_nc(dx, dy, dz);
-        if (!(d2 < rl2 && d2 > 0.f)) continue;
-        float dist = sqrtf(d2);
-        float v[10];
-        lub_lookup(t, dist, 0, 10, 232, v);
-        float rx = dx / dist, ry = dy / dist, rz = dz / dist;
-        if (cnt < maxlub) {
-            int64_t o = (int64_t)i * maxlub + cnt;
-            lub_j[o] = j;
-            lub_a[o] = make_float4(rx, ry, rz, v[1] - v[3]);
-            lub_b[o] = make_float4(v[3], v[5], v[7] - v[9], v[9]);
+    __shared__ PairRing ring;
+    __shared__ int s_cnt[PGB / PG];
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    const int grp = threadIdx.x / PG;
+    if (i >= 0) {
+        // sums of (XA11 - YA11) r r and YA11, YB11 r, (XC11 - YC11) r r and YC11
+        float s[17];
+#pragma unroll
+        for (int q = 0; q < 17; ++q) s[q] = 0.f;
+        const int64_t base = (int64_t)i * maxlub;
+        const int cnt = pg_pairs(
+            ring, pos, b, pos[i], nlist + (int64_t)i * maxn, nneigh[i], lane,
+            [&](float d2) { return d2 < rl2 && d2 > 0.f; },
+            [&](int q, int j, float4 d) {
+                const float dist = sqrtf(d.w);
+                float v[10];
+                lub_lookup<0, 10>(t, dist, 232, v);
+                const float rx = d.x / dist, ry = d.y / dist, rz = d.z / dist;
+                if (q < maxlub) {
+                    lub_j[base + q] = j;
+                    lub_a[base + q] = make_float4(rx, ry, rz, v[1] - v[3]);
+                    lub_b[base + q] = make_float4(v[3], v[5], v[7] - v[9], v[9]);
+                }
+                const float da = v[0] - v[2], dc = v[6] - v[8];
+                s[0] += da * (rx * rx); s[1] += da * (rx * ry); s[2] += da * (rx * rz);
+                s[3] += da * (ry * ry); s[4] += da * (ry * rz); s[5] += da * (rz * rz);
+                s[6] += v[2];
+                s[7] += v[4] * rx; s[8] += v[4] * ry; s[9] += v[4] * rz;
+                s[10] += dc * (rx * rx); s[11] += dc * (rx * ry); s[12] += dc * (rx * rz);
+                s[13] += dc * (ry * ry); s[14] += dc * (ry * rz); s[15] += dc * (rz * rz);
+                s[16] += v[8];
+            });
+#pragma unroll
+        for (int q = 0; q < 17; ++q) s[q] = group_sum<PG>(s[q]);
+        float *S = reinterpret_cast<float *>(ring.d[grp]);   // the ring is done with: 36 of its floats
+        if (lane == 0) {
+            // E v = eps.r.v  (Lubrication.cu:243-254): E = ((0, rz, -ry), (-rz, 0, rx), (ry, -rx, 0))
+            const float A[9] = {s[0] + s[6], s[1], s[2], s[1], s[3] + s[6], s[4], s[2], s[4], s[5] + s[6]};
+            const float C[9] = {s[10] + s[16], s[11], s[12], s[11], s[13] + s[16], s[14], s[12], s[14], s[15] + s[16]};
+            const float B[9] = {0.f, s[9], -s[8], -s[9], 0.f, s[7], s[8], -s[7], 0.f};
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    S[a * 6 + c] = A[3 * a + c];
+                    S[a * 6 + 3 + c] = -B[3 * a + c];
+                    S[(3 + a) * 6 + c] = B[3 * a + c];
+                    S[(3 + a) * 6 + 3 + c] = C[3 * a + c];
+                }
+            lub_n[i] = cnt < maxlub ? cnt : maxlub;
+            s_cnt[grp] = cnt;
         }
-        ++cnt;
-        const float r[3] = {rx, ry, rz};
-        // E v = eps.r.v  (Lubrication.cu:243-254)
-        const float E[3][3] = {{0.f, rz, -ry}, {-rz, 0.f, rx}, {ry, -rx, 0.f}};
-        const float XA11 = v[0], YA11 = v[2], YB11 = v[4], XC11 = v[6], YC11 = v[8];
-        for (int a = 0; a < 3; ++a)
-            for (int c = 0; c < 3; ++c) {
-                float rr = r[a] * r[c];
-                float del = (a == c) ? 1.f : 0.f;
-                S[a * 6 + c] += (XA11 - YA11) * rr + YA11 * del;
-                S[a * 6 + 3 + c] += -YB11 * E[a][c];
-                S[(3 + a) * 6 + c] += YB11 * E[a][c];
-                S[(3 + a) * 6 + 3 + c] += (XC11 - YC11) * rr + YC11 * del;
-            }
+        wave_lds_fence();
+        for (int q = lane; q < 36; q += PG) lub_self[(int64_t)i * 36 + q] = S[q];
+    } else if (lane == 0) {
+        s_cnt[grp] = -1;
     }
-    if (cnt > maxlub) atomicMax(overflow, cnt);
-    lub_n[i] = cnt < maxlub ? cnt : maxlub;
-    for (int q = 0; q < 36; ++q) lub_self[(int64_t)i * 36 + q] = S[q];
+    pg_block_counts(s_cnt, maxlub, overflow, total);
 }
 
 int k_build_lub_pairs(fsd_ctx *ctx, const float4 *pos)
@@ -365,16 +405,17 @@ int k_build_lub_pairs(fsd_ctx *ctx, const float4 *pos)
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     const float rl2 = ctx->p.rlub * ctx->p.rlub;
     for (int attempt = 0; attempt < 2; ++attempt) {
-        FSD_HIP(hipMemsetAsync(ctx->d_flags + 1, 0, sizeof(int), ctx->stream));
-        hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(N, 128)), dim3(128), 0, ctx->stream, pos, N, ctx->box,
+        // flags 8 (most pairs of a particle, when more than maxlub) and 9 (pairs in all)
+        FSD_HIP(hipMemsetAsync(ctx->d_flags + 8, 0, 2 * sizeof(int), ctx->stream));
+        hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
                            ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, rl2, ctx->maxlub, ctx->d_lub_n, ctx->d_lub_j,
-                           ctx->d_lub_a, ctx->d_lub_b, ctx->d_lub_self, ctx->d_flags + 1);
+                           ctx->d_lub_a, ctx->d_lub_b, ctx->d_lub_self, ctx->d_flags + 8, ctx->d_flags + 9,
+                           cell_order(ctx));
         FSD_HIP(hipGetLastError());
-        hipLaunchKernelGGL(sum_int_kernel, dim3(1), dim3(1024), 0, ctx->stream, ctx->d_lub_n, N, ctx->d_flags + 5);
-        FSD_HIP(hipMemcpyAsync(ctx->h_flags + 1, ctx->d_flags + 1, 5 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        FSD_HIP(hipMemcpyAsync(ctx->h_flags + 8, ctx->d_flags + 8, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         FSD_HIP(hipStreamSynchronize(ctx->stream));
-        ctx->lub_total = ctx->h_flags[5];
-        int need = ctx->h_flags[1];
+        ctx->lub_total = ctx->h_flags[9];
+        int need = ctx->h_flags[8];
         if (need == 0) break;
         if (attempt == 1) { ctx->err = "lubrication pair capacity exceeded"; return FSD_E_CAPACITY; }
         int nm = ((need + 16) / 16) * 16 + 16;
@@ -397,9 +438,9 @@ int k_lub_pairs_into(fsd_ctx *ctx, const float4 *pos, int maxlub, int *lub_n, in
     if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     const float rl2 = ctx->p.rlub * ctx->p.rlub;
-    hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(ctx->N, 128)), dim3(128), 0, ctx->stream, pos, ctx->N, ctx->box,
-                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, rl2, maxlub, lub_n, lub_j, lub_a, lub_b, lub_self,
-                       overflow);
+    hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N,
+                       ctx->box, ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, rl2, maxlub, lub_n, lub_j, lub_a, lub_b,
+                       lub_self, overflow, (int *)nullptr, cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }
@@ -512,30 +553,37 @@ __device__ inline void strain_block(const EParams &ep, int k, float E[3][3])
     E[2][0] = E[0][2]; E[2][1] = E[1][2]; E[2][2] = (-1.0f / 3.0f) * (e[0] + e[4]);
 }
 
-// Lubrication_RFE_kernel (Lubrication.cu:350-608): F += R_FE : E
-__global__ void rfe_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn, LubTable t,
-                           float rl2, EParams ep, float *F)
+// o[lane] += sign * v[lane] for the first M lanes (without indexing registers by the lane)
+template <int M>
+__device__ __forceinline__ void pg_add(float *o, int lane, const float *v, float sign)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
+    float f = v[0];
+#pragma unroll
+    for (int q = 1; q < M; ++q) f = (lane == q) ? v[q] : f;
+    if (lane < M) o[lane] += sign * f;
+}
+
+// Lubrication_RFE_kernel (Lubrication.cu:350-608): F += R_FE : E
+__global__ void __launch_bounds__(PGB) rfe_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                  const int *nlist, int maxn, LubTable t, float rl2, EParams ep,
+                                                  float *F, const int *order)
+{
+    __shared__ PairRing ring;
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    if (i < 0) return;
     float Ei[3][3];
     strain_block(ep, i, Ei);
     float acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int k = 0; k < nneigh[i]; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
-        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        box_min_image(b, dx, dy, dz);
-        float d2 = dist2_nc(dx, dy, dz);
-        if (!(d2 < rl2)) continue;
+    pg_pairs(ring, pos, b, pos[i], nlist + (int64_t)i * maxn, nneigh[i], lane, [&](float d2) { return d2 < rl2; },
+             [&](int, int j, float4 d) {
         float Ej[3][3];
         strain_block(ep, j, Ej);
-        float dist = sqrtf(d2);
+        const float dist = sqrtf(d.w);
         float v[6];
-        lub_lookup(t, dist, 10, 6, 232, v);
+        lub_lookup<10, 6>(t, dist, 232, v);
         const float XG11 = v[0], XG12 = v[1], YG11 = v[2], YG12 = v[3], YH11 = v[4], YH12 = v[5];
-        const float r[3] = {dx / dist, dy / dist, dz / dist};
+        const float r[3] = {d.x / dist, d.y / dist, d.z / dist};
         float Ei_r[3], Ej_r[3];
         for (int a = 0; a < 3; ++a) {
             Ei_r[a] = Ei[a][0] * r[0] + Ei[a][1] * r[1] + Ei[a][2] * r[2];
@@ -551,74 +599,75 @@ __global__ void rfe_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, 
                       + 2.0f * YG21 * (-Ej_r[a]);
             acc[3 + a] += YH11 * (2.0f * eEi[a]) + YH21 * (2.0f * eEj[a]);
         }
-    }
-    for (int a = 0; a < 6; ++a) F[6 * (int64_t)i + a] += acc[a];
+    });
+#pragma unroll
+    for (int a = 0; a < 6; ++a) acc[a] = group_sum<PG>(acc[a]);
+    pg_add<6>(F + 6 * (int64_t)i, lane, acc, 1.f);
 }
 
 // Lubrication_RSU_kernel (Lubrication.cu:650-911): S -= R_SU U
-__global__ void rsu_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn, LubTable t,
-                           float rl2, const float *U, float *S)
+__global__ void __launch_bounds__(PGB) rsu_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                  const int *nlist, int maxn, LubTable t, float rl2, const float *U,
+                                                  float *S, const int *order)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
-    const float *ui = U + 6 * (int64_t)i, *wi = U + 6 * (int64_t)i + 3;
+    __shared__ PairRing ring;
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    if (i < 0) return;
+    float ui[3], wi[3];
+    for (int a = 0; a < 3; ++a) { ui[a] = U[6 * (int64_t)i + a]; wi[a] = U[6 * (int64_t)i + 3 + a]; }
     float si[5] = {0, 0, 0, 0, 0};
-    const int ca[5] = {0, 0, 0, 1, 1}, cb[5] = {0, 1, 2, 2, 1};
-    for (int k = 0; k < nneigh[i]; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
-        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        box_min_image(b, dx, dy, dz);
-        float d2 = dist2_nc(dx, dy, dz);
-        if (!(d2 < rl2)) continue;
-        float dist = sqrtf(d2);
+    pg_pairs(ring, pos, b, pos[i], nlist + (int64_t)i * maxn, nneigh[i], lane, [&](float d2) { return d2 < rl2; },
+             [&](int, int j, float4 d) {
+        constexpr int ca[5] = {0, 0, 0, 1, 1}, cb[5] = {0, 1, 2, 2, 1};
+        float uj[3], wj[3];
+        for (int a = 0; a < 3; ++a) { uj[a] = U[6 * (int64_t)j + a]; wj[a] = U[6 * (int64_t)j + 3 + a]; }
+        const float dist = sqrtf(d.w);
         float v[6];
-        lub_lookup(t, dist, 10, 6, 232, v);
+        lub_lookup<10, 6>(t, dist, 232, v);
         const float XG11 = v[0], XG12 = v[1], YG11 = v[2], YG12 = v[3], YH11 = v[4], YH12 = v[5];
-        const float r[3] = {dx / dist, dy / dist, dz / dist};
-        const float *uj = U + 6 * (int64_t)j, *wj = U + 6 * (int64_t)j + 3;
+        const float r[3] = {d.x / dist, d.y / dist, d.z / dist};
         float rdui = r[0] * ui[0] + r[1] * ui[1] + r[2] * ui[2];
         float rduj = r[0] * uj[0] + r[1] * uj[1] + r[2] * uj[2];
         float ewi[3] = {r[2] * wi[1] - r[1] * wi[2], -r[2] * wi[0] + r[0] * wi[2], r[1] * wi[0] - r[0] * wi[1]};
         float ewj[3] = {r[2] * wj[1] - r[1] * wj[2], -r[2] * wj[0] + r[0] * wj[2], r[1] * wj[0] - r[0] * wj[1]};
+#pragma unroll
         for (int c = 0; c < 5; ++c) {
-            int a = ca[c], bb = cb[c];
+            const int a = ca[c], bb = cb[c];
             float third = (a == bb) ? (1.0f / 3.0f) : 0.f;
             si[c] += XG11 * (r[a] * r[bb] - third) * rdui + XG12 * (r[a] * r[bb] - third) * rduj
                      + YG11 * (ui[a] * r[bb] + r[a] * ui[bb] - 2.0f * r[a] * r[bb] * rdui)
                      + YG12 * (uj[a] * r[bb] + r[a] * uj[bb] - 2.0f * r[a] * r[bb] * rduj);
             si[c] += YH11 * (r[a] * ewi[bb] + ewi[a] * r[bb]) + YH12 * (r[a] * ewj[bb] + ewj[a] * r[bb]);
         }
-    }
-    for (int c = 0; c < 5; ++c) S[5 * (int64_t)i + c] -= si[c];
+    });
+#pragma unroll
+    for (int c = 0; c < 5; ++c) si[c] = group_sum<PG>(si[c]);
+    pg_add<5>(S + 5 * (int64_t)i, lane, si, -1.f);
 }
 
 // Lubrication_RSE_kernel (Lubrication.cu:953-1211): S += R_SE : E, cutoff r^2 < 16
-__global__ void rse_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn, LubTable t,
-                           EParams ep, float *S)
+__global__ void __launch_bounds__(PGB) rse_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                  const int *nlist, int maxn, LubTable t, EParams ep, float *S,
+                                                  const int *order)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
+    __shared__ PairRing ring;
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    if (i < 0) return;
     float Ei[3][3];
     strain_block(ep, i, Ei);
     float Si[5] = {0, 0, 0, 0, 0};
-    const int ca[5] = {0, 0, 0, 1, 1}, cb[5] = {0, 1, 2, 2, 1};
-    for (int k = 0; k < nneigh[i]; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
-        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        box_min_image(b, dx, dy, dz);
-        float d2 = dist2_nc(dx, dy, dz);
-        if (!((double)d2 < 16.0)) continue;
+    pg_pairs(ring, pos, b, pos[i], nlist + (int64_t)i * maxn, nneigh[i], lane, [&](float d2) { return d2 < 16.0f; },
+             [&](int, int j, float4 d) {
+        constexpr int ca[5] = {0, 0, 0, 1, 1}, cb[5] = {0, 1, 2, 2, 1};
         float Ej[3][3];
         strain_block(ep, j, Ej);
-        float dist = sqrtf(d2);
+        const float dist = sqrtf(d.w);
         float v[6];
-        lub_lookup(t, dist, 16, 6, 232, v);
+        lub_lookup<16, 6>(t, dist, 232, v);
         const float XM11 = v[0], XM12 = v[1], YM11 = v[2], YM12 = v[3], ZM11 = v[4], ZM12 = v[5];
-        const float r[3] = {dx / dist, dy / dist, dz / dist};
+        const float r[3] = {d.x / dist, d.y / dist, d.z / dist};
         float Ei_r[3], Ej_r[3];
         for (int a = 0; a < 3; ++a) {
             Ei_r[a] = Ei[a][0] * r[0] + Ei[a][1] * r[1] + Ei[a][2] * r[2];
@@ -626,8 +675,9 @@ __global__ void rse_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, 
         }
         float rEi = r[0] * Ei_r[0] + r[1] * Ei_r[1] + r[2] * Ei_r[2];
         float rEj = r[0] * Ej_r[0] + r[1] * Ej_r[1] + r[2] * Ej_r[2];
+#pragma unroll
         for (int c = 0; c < 5; ++c) {
-            int a = ca[c], bb = cb[c];
+            const int a = ca[c], bb = cb[c];
             float third = (a == bb) ? (1.0f / 3.0f) : 0.f;
             float del = (a == bb) ? 1.f : 0.f;
             Si[c] += 1.5f * XM11 * (r[a] * r[bb] - third) * rEi + 1.5f * XM12 * (r[a] * r[bb] - third) * rEj
@@ -636,8 +686,10 @@ __global__ void rse_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, 
                      + 0.5f * ZM11 * (2.f * Ei[a][bb] + (del + r[a] * r[bb]) * rEi - 2.0f * r[a] * Ei_r[bb] - 2.0f * r[bb] * Ei_r[a])
                      + 0.5f * ZM12 * (2.f * Ej[a][bb] + (del + r[a] * r[bb]) * rEj - 2.0f * r[a] * Ej_r[bb] - 2.0f * r[bb] * Ej_r[a]);
         }
-    }
-    for (int c = 0; c < 5; ++c) S[5 * (int64_t)i + c] += Si[c];
+    });
+#pragma unroll
+    for (int c = 0; c < 5; ++c) Si[c] = group_sum<PG>(Si[c]);
+    pg_add<5>(S + 5 * (int64_t)i, lane, Si, 1.f);
 }
 
 static EParams make_ep(fsd_ctx *ctx, float shear_rate, const float *ori)
@@ -653,9 +705,9 @@ static EParams make_ep(fsd_ctx *ctx, float shear_rate, const float *ori)
 int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
-    hipLaunchKernelGGL(rfe_kernel, dim3(nblk(ctx->N, 128)), dim3(128), 0, ctx->stream, pos, ctx->N, ctx->box,
+    hipLaunchKernelGGL(rfe_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
                        ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, ctx->p.rlub * ctx->p.rlub,
-                       make_ep(ctx, shear_rate, ori), F);
+                       make_ep(ctx, shear_rate, ori), F, cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }
@@ -663,8 +715,9 @@ int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, f
 int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
-    hipLaunchKernelGGL(rsu_kernel, dim3(nblk(ctx->N, 128)), dim3(128), 0, ctx->stream, pos, ctx->N, ctx->box,
-                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, ctx->p.rlub * ctx->p.rlub, U, S);
+    hipLaunchKernelGGL(rsu_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
+                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, ctx->p.rlub * ctx->p.rlub, U, S,
+                       cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }
@@ -672,25 +725,30 @@ int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S)
 int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
-    hipLaunchKernelGGL(rse_kernel, dim3(nblk(ctx->N, 128)), dim3(128), 0, ctx->stream, pos, ctx->N, ctx->box,
-                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, make_ep(ctx, shear_rate, ori), S);
+    hipLaunchKernelGGL(rse_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
+                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, make_ep(ctx, shear_rate, ori), S,
+                       cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }
 
 // ------------------------------------------------------------ force law
 // Stokes_SetForce_manually_kernel (Helper_Stokes.cu:65-172)
-__global__ void force_law_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn,
-                                 float ndsr, float k_n, float kappa, float beta, float epsq, float T_ext, float *F)
+__global__ void __launch_bounds__(PGB) force_law_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                        const int *nlist, int maxn, float ndsr, float k_n, float kappa,
+                                                        float beta, float epsq, float T_ext, float *F,
+                                                        const int *order)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    if (i < 0) return;
+    const float4 pi = pos[i];
     const float h_rough = sqrtf(epsq), rcol = 2.0f + 1.0f * h_rough, F0 = 1.0f / ndsr, Ham = F0 * beta;
     float fx = 0.f, fy = 0.f, fz = 0.f;
-    for (int k = 0; k < nneigh[i]; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
+    const int nn = nneigh[i];
+    for (int k = lane; k < nn; k += PG) {
+        const int j = nlist[(int64_t)i * maxn + k];
+        const float4 pj = pos[j];
         float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
         box_min_image(b, dx, dy, dz);
         float dist = sqrtf(dist2_nc(dx, dy, dz));
@@ -700,15 +758,19 @@ __global__ void force_law_kernel(const float4 *pos, int N, BoxF b, const int *nn
         if (gap < 0.f) mag = Ham / (12.f * epsq) - F0 - k_n * fabsf(gap);
         fx += mag * (dx / dist); fy += mag * (dy / dist); fz += mag * (dz / dist);
     }
-    F[6 * (int64_t)i] = fx; F[6 * (int64_t)i + 1] = fy; F[6 * (int64_t)i + 2] = fz;
-    F[6 * (int64_t)i + 3] = 0.f; F[6 * (int64_t)i + 4] = 0.f; F[6 * (int64_t)i + 5] = T_ext;
+    const float f[6] = {group_sum<PG>(fx), group_sum<PG>(fy), group_sum<PG>(fz), 0.f, 0.f, T_ext};
+    float v = f[0];
+#pragma unroll
+    for (int q = 1; q < 6; ++q) v = (lane == q) ? f[q] : v;
+    if (lane < 6) F[6 * (int64_t)i + lane] = v;
 }
 
 int k_force_law(fsd_ctx *ctx, const float4 *pos, float T_ext, float *F)
 {
     const fsd_params &p = ctx->p;
-    hipLaunchKernelGGL(force_law_kernel, dim3(nblk(ctx->N, 128)), dim3(128), 0, ctx->stream, pos, ctx->N, ctx->box,
-                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, p.ndsr, p.k_n, p.kappa, p.beta_AF, p.epsq, T_ext, F);
+    hipLaunchKernelGGL(force_law_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
+                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, p.ndsr, p.k_n, p.kappa, p.beta_AF, p.epsq, T_ext, F,
+                       cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }

@@ -12,51 +12,50 @@
 // solves run both sweeps in one single-workgroup launch on a static
 // schedule (sweep_plan.h), or one launch per level where LDS is too small.
 #include "fsd_internal.h"
+#include "pair_scan.h"
 
 // ----------------------------------------------------------- pruning
 // Precondition_GetPrunedNneigh/GetPrunedNlist (Precondition.cu:70-242):
 // neighbours with r^2 < rp^2 (r = x_i - x_j), self included, ascending.
-__global__ void prune_kernel(const float4 *pos, int N, BoxF b, const int *nneigh, const int *nlist, int maxn,
-                             float rp2, int *pn, int *plist, int *pless, int *overflow)
+__global__ void __launch_bounds__(PGB) prune_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
+                                                    const int *nlist, int maxn, float rp2, int *pn, int *plist,
+                                                    int *pless, int *overflow, const int *order)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    float4 pi = pos[i];
-    int A[FSD_PSTRIDE];
-    int cnt = 1;
-    A[0] = i;
-    for (int k = 0; k < nneigh[i]; ++k) {
-        int j = nlist[(int64_t)i * maxn + k];
-        float4 pj = pos[j];
-        float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-        box_min_image(b, dx, dy, dz);
-        if (dist2_nc(dx, dy, dz) < rp2) {
-            if (cnt < FSD_PSTRIDE) A[cnt] = j;
-            ++cnt;
+    static_assert(FSD_PSTRIDE == PG, "one lane per entry of a pruned list");
+    __shared__ PairRing ring;
+    __shared__ int s_list[PGB / PG][FSD_PSTRIDE];
+    int lane;
+    const int i = pg_particle(N, order, lane);
+    if (i < 0) return;
+    int *A = s_list[threadIdx.x / PG];
+    if (lane == 0) A[0] = i;
+    int cnt = 1 + pg_pairs(ring, pos, b, pos[i], nlist + (int64_t)i * maxn, nneigh[i], lane,
+                           [&](float d2) { return d2 < rp2; },
+                           [&](int q, int j, float4) { if (q + 1 < FSD_PSTRIDE) A[q + 1] = j; });
+    if (cnt > FSD_PSTRIDE) {
+        if (lane == 0) atomicMax(overflow, cnt);
+        cnt = FSD_PSTRIDE;
+    }
+    // ascending: every lane stores its entry at its rank
+    if (lane < cnt) {
+        const int key = A[lane];
+        int rank = 0;
+        for (int q = 0; q < cnt; ++q) rank += A[q] < key;
+        plist[(int64_t)i * FSD_PSTRIDE + rank] = key;
+        if (lane == 0) {   // A[0] = i
+            pn[i] = cnt;
+            pless[i] = rank;
         }
     }
-    if (cnt > FSD_PSTRIDE) { atomicMax(overflow, cnt); cnt = FSD_PSTRIDE; }
-    for (int a = 1; a < cnt; ++a) {
-        int key = A[a], q = a - 1;
-        while (q >= 0 && A[q] > key) { A[q + 1] = A[q]; --q; }
-        A[q + 1] = key;
-    }
-    int nl = 0;
-    for (int a = 0; a < cnt; ++a) {
-        plist[(int64_t)i * FSD_PSTRIDE + a] = A[a];
-        nl += (A[a] < i);
-    }
-    pn[i] = cnt;
-    pless[i] = nl;
 }
 
 int k_prune(fsd_ctx *ctx, const float4 *pos)
 {
     const int N = ctx->N;
     FSD_HIP(hipMemsetAsync(ctx->d_flags + 2, 0, sizeof(int), ctx->stream));
-    hipLaunchKernelGGL(prune_kernel, dim3(nblk(N, 128)), dim3(128), 0, ctx->stream, pos, N, ctx->box, ctx->d_nneigh,
-                       ctx->d_nlist, ctx->maxn, ctx->p.rp * ctx->p.rp, ctx->d_pn, ctx->d_plist, ctx->d_pless,
-                       ctx->d_flags + 2);
+    hipLaunchKernelGGL(prune_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
+                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, ctx->p.rp * ctx->p.rp, ctx->d_pn, ctx->d_plist,
+                       ctx->d_pless, ctx->d_flags + 2, cell_order(ctx));
     FSD_HIP(hipGetLastError());
     return 0;
 }
@@ -90,7 +89,7 @@ __global__ void blocks_kernel(const float4 *pos, int N, BoxF b, const int *pn, c
         if ((double)dist <= 2.0 + (double)t.table_min) {
             for (int c = 0; c < 10; ++c) v[c] = t.vals[c];     // contact clamp: table row 0
         } else {
-            lub_lookup(t, dist, 0, 10, -1, v);
+            lub_lookup<0, 10>(t, dist, -1, v);
         }
         const float XA11 = v[0], XA12 = v[1], YA11 = v[2], YA12 = v[3], YB11 = v[4], YB12 = v[5];
         const float XC11 = v[6], XC12 = v[7], YC11 = v[8], YC12 = v[9];

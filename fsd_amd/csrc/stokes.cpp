@@ -184,9 +184,9 @@ static int alloc_all(fsd_ctx *ctx)
         CK(hipMalloc(&ctx->d_cell_start, sizeof(int) * (ctx->ncells + 1)));
         CK(hipMalloc(&ctx->d_cell_list, sizeof(int) * N));
     }
-    CK(hipMalloc(&ctx->d_flags, sizeof(int) * 8));
+    CK(hipMalloc(&ctx->d_flags, sizeof(int) * 16));
     CK(hipMalloc(&ctx->d_pos_last, sizeof(float4) * (size_t)N));
-    CK(hipHostMalloc((void **)&ctx->h_flags, sizeof(int) * 8, hipHostMallocDefault));
+    CK(hipHostMalloc((void **)&ctx->h_flags, sizeof(int) * 16, hipHostMallocDefault));
     // lubrication records
     ctx->maxlub = 48;
     CK(hipMalloc(&ctx->d_lub_n, sizeof(int) * N));
