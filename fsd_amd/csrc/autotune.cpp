@@ -71,7 +71,7 @@ int autotune_run(fsd_ctx *ctx, const float4 *pos)
     RC(time_us(ctx, s, wave, &best));
     const bool can_spread2 = ctx->tile == 8 && ctx->pse.P == 6;
     const bool can_contract_tiled = ctx->contract_lds > 0;
-    const bool can_fx = ctx->fx_B > 0 && ctx->plan_fwd2 && ctx->plan_inv2;
+    const bool can_fx = ctx->fft_lds;
     int *knobs[3] = {&t.spread, &t.contract, &t.xpass};
     const bool alt[3] = {can_spread2, can_contract_tiled, can_fx};   // the default (0) is a real choice
     for (int k = 0; k < 3; ++k) {

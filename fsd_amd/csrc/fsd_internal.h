@@ -19,6 +19,7 @@
 #include <vector>
 #include "fsd.h"
 #include "precond_plan.h"
+#include "fft_small.h"
 
 #define FSD_MAXP 14        // pruned neighbours incl. self (kissing number 12 + self + 1)
 #define FSD_PSTRIDE 16     // stride of the pruned list
@@ -195,7 +196,7 @@ struct fsd_tuning {
     int spread = 0;          // 0: spread_tile2_kernel (tile 8, P 6), 1: spread_kernel (one workgroup per tile)
     int contract = 0;        // 0: tile contraction (contract_tile2/contract_tile, when it fits in LDS),
                              // 1: one wave per particle (contract_kernel)
-    int xpass = 0;           // 0: x transforms fused with the Green's function (when built), 1: 3-D rocFFT
+    int xpass = 0;           // 0: the transforms of k_fft.hip (when the grid fits them), 1: 3-D rocFFT
     int real_g = 16, real_blk = 256;   // real-space sum: lanes per particle (4, 8, 16), workgroup size
     int rfu_g = 8, rfu_blk = 256;      // R_FU product: lanes per particle (8, 16), workgroup size
     int tuned = 0;
@@ -246,10 +247,11 @@ struct fsd_ctx {
     float2 *d_spec = nullptr;     // 11*Mh complex
     float4 *d_gridk = nullptr;    // Mh
     rocfft_plan plan_fwd = nullptr, plan_inv = nullptr;
-    // 2-D (y, z) transforms batched over the fields and x planes; the x direction and the Green's
-    // function then run in one kernel (fx_B: Nx / 8, 0 when the 3-D plans are used instead)
-    rocfft_plan plan_fwd2 = nullptr, plan_inv2 = nullptr;
-    int fx_B = 0;
+    // this library's transforms (k_fft.hip), used unless the grid does not fit them
+    bool fft_lds = false;
+    FftAxis fft_axis[3];
+    float2 *d_fft_tw = nullptr;
+    unsigned short *d_fft_loc = nullptr;
     rocfft_execution_info info_fwd = nullptr, info_inv = nullptr;
     void *d_fftwork = nullptr; size_t fftwork_size = 0;
     int tiles[3] = {0, 0, 0}; int ntiles = 0; int tile = 8;
@@ -416,7 +418,14 @@ int k_normals(fsd_ctx *ctx, int64_t n, uint32_t step, uint32_t stream, float sd,
 int k_ff_noise(fsd_ctx *ctx, const float *noise, float fac);
 int k_wave_to_general(fsd_ctx *ctx, float *out);
 int k_shift_wrap(fsd_ctx *ctx, const float4 *pos, const float *psi6, float scale, float4 *out);
-int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool inverse_yz = false);
+int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done = false);
+// transforms of the grids (k_fft.hip; the 3-D library plans in stokes.cpp)
+int fft_init(fsd_ctx *ctx);
+int fft_plans_3d(fsd_ctx *ctx);
+int k_fft_yz_forward(fsd_ctx *ctx);
+int k_fft_x(fsd_ctx *ctx, bool green);
+int k_fft_yz_inverse(fsd_ctx *ctx);
+inline bool use_fft_lds(const fsd_ctx *ctx) { return ctx->fft_lds && ctx->tune.xpass == 0; }
 int k_precond_apply2(fsd_ctx *ctx, const float *b0, const float *b1, float *y0, float *y1, int n_rhs);
 int k_export_csr(fsd_ctx *ctx, const float4 *pos, int32_t *h_rowptr, int32_t *h_col, float *h_val,
                  int32_t *h_prow, int32_t *h_pcol, float *h_L, int64_t cap);

@@ -1,13 +1,14 @@
 // PSE far-field grand mobility on MI355X.
 //
 //   wave space:  particle records -> tile-gather spreading (no global atomics)
-//                -> rocFFT R2C (11 batched fields) -> Green's-function scaling on
-//                the half spectrum -> rocFFT C2R -> per-particle contraction;
+//                -> real-to-complex transform (11 fields, k_fft.hip), Green's function
+//                on the half spectrum and back -> per-particle contraction;
 //   real space:  table-interpolated FTS pair sum, 16 lanes per particle, with an
 //                epilogue that adds the wave-space result, converts the velocity
 //                gradient to (W, E) and writes the generalised velocity.
 // Restates Mobility.cu:131-1542 and Helper_Mobility.cu:88-410.
 #include "fsd_internal.h"
+#include "green.h"
 
 #define FSD_TILE 8
 
@@ -448,71 +449,6 @@ __global__ void __launch_bounds__(512) spread_tile2_kernel(SpreadGeom g, const f
 }
 
 // ------------------------------------------------------------ Green kernel
-// Mobility_WaveSpace_Green_kernel (Mobility.cu:315-479) on the half spectrum.
-// Field order: Fx Fy Fz | C_xx C_xy C_xz C_yz C_yy C_yx C_zx C_zy.
-__device__ inline void green_apply(const float4 tk, bool origin, const float2 v[11], float2 o[11])
-{
-#pragma unroll
-    for (int c = 0; c < 11; ++c) o[c] = make_float2(0.f, 0.f);
-    if (origin) return;
-    const float k[3] = {tk.x, tk.y, tk.z};
-    const float ksq = k[0] * k[0] + k[1] * k[1] + k[2] * k[2];
-    const float kk = sqrtf(ksq);
-    // couplet matrix rows (x, y, z)
-    const float2 Cm[3][3] = {{v[3], v[4], v[5]}, {v[8], v[7], v[6]}, {v[9], v[10], make_float2(-(v[3].x + v[7].x), -(v[3].y + v[7].y))}};
-    float2 kdF;
-    kdF.x = (k[0] * v[0].x + k[1] * v[1].x + k[2] * v[2].x) / ksq;
-    kdF.y = (k[0] * v[0].y + k[1] * v[1].y + k[2] * v[2].y) / ksq;
-    float2 Cdk[3];
-    for (int a = 0; a < 3; ++a) {
-        Cdk[a].x = Cm[a][0].x * k[0] + Cm[a][1].x * k[1] + Cm[a][2].x * k[2];
-        Cdk[a].y = Cm[a][0].y * k[0] + Cm[a][1].y * k[1] + Cm[a][2].y * k[2];
-    }
-    float2 kCk;
-    kCk.x = (Cdk[0].x * k[0] + Cdk[1].x * k[1] + Cdk[2].x * k[2]) / ksq;
-    kCk.y = (Cdk[0].y * k[0] + Cdk[1].y * k[1] + Cdk[2].y * k[2]) / ksq;
-    const float sk = sinf(kk), ck = cosf(kk);
-    const float j0 = sk / kk;
-    const float jt = 3.0f * (sk - kk * ck) / (ksq * kk);
-    const float Buf = tk.w * j0 * j0;
-    const float Buc = -tk.w * j0 * jt;        // UC (imaginary coupling)
-    const float Bdf = tk.w * j0 * jt;         // DF (imaginary coupling)
-    const float q = (sk - kk * ck) / (ksq * kk);
-    const float Bdc = tk.w * 9.0f * q * q;    // DC
-    for (int a = 0; a < 3; ++a) {
-        float2 ff = v[a];
-        float2 u;
-        u.x = (ff.x - k[a] * kdF.x) * Buf;
-        u.y = (ff.y - k[a] * kdF.y) * Buf;
-        // + i (Cdk_a - k_a kCk) Buc
-        u.x += -(Cdk[a].y - k[a] * kCk.y) * Buc;
-        u.y += (Cdk[a].x - k[a] * kCk.x) * Buc;
-        o[a] = u;
-    }
-    // gradient slots in field order: (x,x) (x,y) (x,z) (y,z) (y,y) (y,x) (z,x) (z,y)
-    const int sa[8] = {0, 0, 0, 1, 1, 1, 2, 2}, sc[8] = {0, 1, 2, 2, 1, 0, 0, 1};
-#pragma unroll
-    for (int s = 0; s < 8; ++s) {
-        const int a = sa[s], c = sc[s];
-        const float kk_ac = k[a] * k[c];
-        float2 z;
-        z.x = v[a].x * k[c] - kk_ac * kdF.x;
-        z.y = v[a].y * k[c] - kk_ac * kdF.y;
-        float2 d;
-        d.x = -z.y * Bdf + (Cdk[a].x * k[c] - kk_ac * kCk.x) * Bdc;
-        d.y = z.x * Bdf + (Cdk[a].y * k[c] - kk_ac * kCk.y) * Bdc;
-        o[3 + s] = d;
-    }
-}
-
-struct GreenGeom {
-    int Nx, Ny, Nz;
-    BoxF b;
-    float xi, eta, twopi_k;
-};
-
-// the spread grid is real, so its spectrum at the conjugate mode is conj(v);
-// modes with a Nyquist index get the Hermitian part of the two outputs
 __global__ void green_kernel(float2 *spec, const float4 *gk, int64_t Mh, GreenGeom g)
 {
     int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -522,235 +458,9 @@ __global__ void green_kernel(float2 *spec, const float4 *gk, int64_t Mh, GreenGe
     float2 v[11];
 #pragma unroll
     for (int c = 0; c < 11; ++c) v[c] = spec[c * Mh + id];
-    float2 o[11];
-    green_apply(gk[id], id == 0, v, o);
-    if (has_nyquist(i, j, k, g.Nx, g.Ny, g.Nz)) {
-        const int ic = (g.Nx - i) % g.Nx, jc = (g.Ny - j) % g.Ny, kc = (g.Nz - k) % g.Nz;
-        const float4 tkc = gridk_value(ic, jc, kc, g.Nx, g.Ny, g.Nz, g.b, g.xi, g.eta, g.twopi_k);
-        float2 vc[11], oc[11];
+    green_update(g, gk, i, j, k, v);
 #pragma unroll
-        for (int c = 0; c < 11; ++c) vc[c] = make_float2(v[c].x, -v[c].y);
-        green_apply(tkc, false, vc, oc);
-#pragma unroll
-        for (int c = 0; c < 11; ++c) o[c] = make_float2(0.5f * (o[c].x + oc[c].x), 0.5f * (o[c].y - oc[c].y));
-    }
-#pragma unroll
-    for (int c = 0; c < 11; ++c) spec[c * Mh + id] = o[c];
-}
-
-// The x direction of the 3-D transform with the Green's function between its
-// forward and inverse halves, on the half spectrum after the (y, z) transforms:
-// element (c, x, ky, kz) at c Mh + (x Ny + ky) Nzh + kz.  One workgroup takes one
-// ky and FX_KC consecutive kz for all 11 fields, so every mode it holds after the
-// forward transform has all 11 fields in LDS and green_kernel's update applies
-// point by point; the inverse brings the columns back to x.  Nx = 8 B: forward,
-// an 8-point DFT over n1 for each n2 (x = B n1 + n2), the twiddle W^(n2 k1), then a
-// B-point DFT over n2 for each k1 (fx_dft8, fx_dftB), leaving mode k1 + 8 k2 at
-// B k1 + k2; the inverse
-// runs the same stages backwards with conjugate twiddles (unnormalised, as the
-// library's transforms).  W = exp(-2 pi i / Nx) from an LDS table built in FP64.
-// small DFTs of the x pass (INV: the conjugate kernel, unnormalised): 8 points by radix 2,
-// 9 points as 3 x 3, other lengths directly from the table wB[j] = W_B^j
-__device__ __forceinline__ float2 fx_mul_i(float2 v, bool inv)   // v * (inv ? i : -i)
-{
-    return inv ? make_float2(-v.y, v.x) : make_float2(v.y, -v.x);
-}
-template <bool INV>
-__device__ __forceinline__ void fx_dft4(const float2 c[4], float2 y[4])
-{
-    const float2 t0 = make_float2(c[0].x + c[2].x, c[0].y + c[2].y), t1 = make_float2(c[0].x - c[2].x, c[0].y - c[2].y);
-    const float2 t2 = make_float2(c[1].x + c[3].x, c[1].y + c[3].y);
-    const float2 t3 = fx_mul_i(make_float2(c[1].x - c[3].x, c[1].y - c[3].y), INV);
-    y[0] = make_float2(t0.x + t2.x, t0.y + t2.y); y[2] = make_float2(t0.x - t2.x, t0.y - t2.y);
-    y[1] = make_float2(t1.x + t3.x, t1.y + t3.y); y[3] = make_float2(t1.x - t3.x, t1.y - t3.y);
-}
-template <bool INV>
-__device__ __forceinline__ void fx_dft8(const float2 x[8], float2 y[8])
-{
-    constexpr float R = 0.70710678118654752f;
-    float2 a[4], b[4], e[4], o[4];
-#pragma unroll
-    for (int n = 0; n < 4; ++n) {
-        a[n] = make_float2(x[n].x + x[n + 4].x, x[n].y + x[n + 4].y);
-        b[n] = make_float2(x[n].x - x[n + 4].x, x[n].y - x[n + 4].y);
-    }
-    // b_n W8^(-+n): W8 = R (1 -+ i), W8^2 = -+i, W8^3 = R (-1 -+ i)
-    b[1] = INV ? make_float2(R * (b[1].x - b[1].y), R * (b[1].x + b[1].y))
-               : make_float2(R * (b[1].x + b[1].y), R * (b[1].y - b[1].x));
-    b[2] = fx_mul_i(b[2], INV);
-    b[3] = INV ? make_float2(-R * (b[3].x + b[3].y), R * (b[3].x - b[3].y))
-               : make_float2(R * (b[3].y - b[3].x), -R * (b[3].x + b[3].y));
-    fx_dft4<INV>(a, e);
-    fx_dft4<INV>(b, o);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) { y[2 * k] = e[k]; y[2 * k + 1] = o[k]; }
-}
-template <bool INV>
-__device__ __forceinline__ void fx_dft3(float2 a, float2 b, float2 c, float2 &X0, float2 &X1, float2 &X2)
-{
-    constexpr float H = 0.86602540378443865f;   // sqrt(3) / 2
-    const float2 sm = make_float2(b.x + c.x, b.y + c.y), d = make_float2(b.x - c.x, b.y - c.y);
-    const float2 t = fx_mul_i(make_float2(H * d.x, H * d.y), INV);
-    const float2 m = make_float2(a.x - 0.5f * sm.x, a.y - 0.5f * sm.y);
-    X0 = make_float2(a.x + sm.x, a.y + sm.y);
-    X1 = make_float2(m.x + t.x, m.y + t.y);
-    X2 = make_float2(m.x - t.x, m.y - t.y);
-}
-template <int B, bool INV>
-__device__ __forceinline__ void fx_dftB(const float2 x[B], float2 X[B], const float2 wB[B])
-{
-    auto mul = [](float2 a, float2 w) {   // a * w, or a * conj(w) for the inverse
-        return INV ? make_float2(a.x * w.x + a.y * w.y, a.y * w.x - a.x * w.y)
-                   : make_float2(a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x);
-    };
-    if constexpr (B == 9) {   // n = 3 m1 + m2, k = k1 + 3 k2
-        float2 u[3][3];
-#pragma unroll
-        for (int m2 = 0; m2 < 3; ++m2) {
-            fx_dft3<INV>(x[m2], x[3 + m2], x[6 + m2], u[0][m2], u[1][m2], u[2][m2]);
-#pragma unroll
-            for (int k1 = 1; k1 < 3; ++k1)
-                if (m2 > 0) u[k1][m2] = mul(u[k1][m2], wB[m2 * k1]);
-        }
-#pragma unroll
-        for (int k1 = 0; k1 < 3; ++k1) fx_dft3<INV>(u[k1][0], u[k1][1], u[k1][2], X[k1], X[k1 + 3], X[k1 + 6]);
-    } else {
-#pragma unroll
-        for (int k = 0; k < B; ++k) {
-            float2 acc = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int n = 0; n < B; ++n) {
-                const float2 p = mul(x[n], wB[(n * k) % B]);
-                acc.x += p.x; acc.y += p.y;
-            }
-            X[k] = acc;
-        }
-    }
-}
-
-#define FX_KC 4
-template <int B>
-__global__ void __launch_bounds__(256) fft_x_green_kernel(float2 *spec, const float4 *gk, int64_t Mh, GreenGeom g)
-{
-    constexpr int NX = 8 * B;
-    __shared__ float2 buf[11 * NX * FX_KC];   // [field][x][kz in the chunk]
-    __shared__ float2 tw[NX];
-    const int tid = threadIdx.x;
-    const int Nzh = g.Nz / 2 + 1;
-    const int nchunk = (Nzh + FX_KC - 1) / FX_KC;
-    // the chunks of a ky row share cache lines (a chunk is FX_KC of the row's Nzh modes): a contiguous
-    // range of rows per XCD keeps every line's readers and writers on one L2
-    const int blk = xcd_remap(blockIdx.x, gridDim.x);
-    const int ky = blk / nchunk, kz0 = (blk % nchunk) * FX_KC;
-    const int kc = min(FX_KC, Nzh - kz0);
-    if (tid < NX) {
-        double sn, cs;
-        sincospi(-2.0 * (double)tid / (double)NX, &sn, &cs);
-        tw[tid] = make_float2((float)cs, (float)sn);
-    }
-    const int nload = 11 * NX * kc;
-    for (int i = tid; i < nload; i += 256) {
-        const int c = i / (NX * kc), r = i - c * (NX * kc), x = r / kc, z = r - x * kc;
-        buf[(c * NX + x) * FX_KC + z] = spec[c * Mh + ((int64_t)x * g.Ny + ky) * Nzh + kz0 + z];
-    }
-    __syncthreads();
-    const int ncol = 11 * kc;
-    // W_B^j = W^(8 j)
-    float2 wB[B];
-#pragma unroll
-    for (int j = 0; j < B; ++j) wB[j] = tw[8 * j];
-    auto at = [&](int col, int x) -> float2 & { return buf[((col / kc) * NX + x) * FX_KC + col % kc]; };
-    auto cmul = [](float2 a, float2 b) { return make_float2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x); };
-    auto cmulc = [](float2 a, float2 b) { return make_float2(a.x * b.x + a.y * b.y, a.y * b.x - a.x * b.y); };
-    // forward stage A: 8-point DFTs, then the twiddles
-    for (int task = tid; task < ncol * B; task += 256) {
-        const int col = task / B, n2 = task - col * B;
-        float2 xs[8], y[8];
-#pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) xs[n1] = at(col, B * n1 + n2);
-        fx_dft8<false>(xs, y);
-#pragma unroll
-        for (int k1 = 0; k1 < 8; ++k1) at(col, B * k1 + n2) = cmul(y[k1], tw[n2 * k1]);
-    }
-    __syncthreads();
-    // forward stage B: B-point DFTs
-    for (int task = tid; task < ncol * 8; task += 256) {
-        const int col = task >> 3, k1 = task & 7;
-        float2 ys[B], X[B];
-#pragma unroll
-        for (int n2 = 0; n2 < B; ++n2) ys[n2] = at(col, B * k1 + n2);
-        fx_dftB<B, false>(ys, X, wB);
-#pragma unroll
-        for (int k2 = 0; k2 < B; ++k2) at(col, B * k1 + k2) = X[k2];
-    }
-    __syncthreads();
-    // Green's function (green_kernel's update) at every mode of the block
-    for (int pt = tid; pt < NX * kc; pt += 256) {
-        const int kx = pt / kc, z = pt - kx * kc;
-        const int pos = B * (kx & 7) + (kx >> 3);
-        const int k = kz0 + z;
-        const int64_t id = ((int64_t)kx * g.Ny + ky) * Nzh + k;
-        float2 v[11], o[11];
-#pragma unroll
-        for (int c = 0; c < 11; ++c) v[c] = buf[(c * NX + pos) * FX_KC + z];
-        green_apply(gk[id], id == 0, v, o);
-        if (has_nyquist(kx, ky, k, g.Nx, g.Ny, g.Nz)) {
-            const int ic = (g.Nx - kx) % g.Nx, jc = (g.Ny - ky) % g.Ny, kcj = (g.Nz - k) % g.Nz;
-            const float4 tkc = gridk_value(ic, jc, kcj, g.Nx, g.Ny, g.Nz, g.b, g.xi, g.eta, g.twopi_k);
-            float2 vc[11], oc[11];
-#pragma unroll
-            for (int c = 0; c < 11; ++c) vc[c] = make_float2(v[c].x, -v[c].y);
-            green_apply(tkc, false, vc, oc);
-#pragma unroll
-            for (int c = 0; c < 11; ++c) o[c] = make_float2(0.5f * (o[c].x + oc[c].x), 0.5f * (o[c].y - oc[c].y));
-        }
-#pragma unroll
-        for (int c = 0; c < 11; ++c) buf[(c * NX + pos) * FX_KC + z] = o[c];
-    }
-    __syncthreads();
-    // inverse stage B, then the conjugate twiddles
-    for (int task = tid; task < ncol * 8; task += 256) {
-        const int col = task >> 3, k1 = task & 7;
-        float2 Xs[B], y[B];
-#pragma unroll
-        for (int k2 = 0; k2 < B; ++k2) Xs[k2] = at(col, B * k1 + k2);
-        fx_dftB<B, true>(Xs, y, wB);
-#pragma unroll
-        for (int n2 = 0; n2 < B; ++n2) at(col, B * k1 + n2) = cmulc(y[n2], tw[n2 * k1]);
-    }
-    __syncthreads();
-    // inverse stage A: 8-point DFTs back to x
-    for (int task = tid; task < ncol * B; task += 256) {
-        const int col = task / B, n2 = task - col * B;
-        float2 ys[8], x[8];
-#pragma unroll
-        for (int k1 = 0; k1 < 8; ++k1) ys[k1] = at(col, B * k1 + n2);
-        fx_dft8<true>(ys, x);
-#pragma unroll
-        for (int n1 = 0; n1 < 8; ++n1) at(col, B * n1 + n2) = x[n1];
-    }
-    __syncthreads();
-    for (int i = tid; i < nload; i += 256) {
-        const int c = i / (NX * kc), r = i - c * (NX * kc), x = r / kc, z = r - x * kc;
-        spec[c * Mh + ((int64_t)x * g.Ny + ky) * Nzh + kz0 + z] = buf[(c * NX + x) * FX_KC + z];
-    }
-}
-
-// launch of fft_x_green_kernel for Nx = 8 B (B in 5..11, so the block fits in 64 KiB of LDS); false
-// for other sizes
-static bool launch_fft_x_green(fsd_ctx *ctx, const GreenGeom &gg)
-{
-    const int Nzh = ctx->pse.Nz / 2 + 1;
-    const dim3 grid(ctx->pse.Ny * ((Nzh + FX_KC - 1) / FX_KC)), blk(256);
-    float2 *spec = ctx->d_spec;
-    const float4 *gk = ctx->d_gridk;
-    const int64_t Mh = ctx->Mh;
-    switch (ctx->fx_B) {
-#define FX_CASE(b) case b: hipLaunchKernelGGL(fft_x_green_kernel<b>, grid, blk, 0, ctx->stream, spec, gk, Mh, gg); return true;
-        FX_CASE(5) FX_CASE(6) FX_CASE(7) FX_CASE(8) FX_CASE(9) FX_CASE(10) FX_CASE(11)
-#undef FX_CASE
-        default: return false;
-    }
+    for (int c = 0; c < 11; ++c) spec[c * Mh + id] = v[c];
 }
 
 // ------------------------------------------------------------ contraction
@@ -1210,9 +920,9 @@ __global__ void __launch_bounds__(256) realspace_kernel(RealParams rp, const flo
 }
 
 // inverse transform of the 11 half spectra in d_spec and contraction of the
-// grids at the particles into d_wave (u and the velocity gradient); with
-// inverse_yz only the (y, z) part of the inverse remains (x has been done)
-int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool inverse_yz)
+// grids at the particles into d_wave (u and the velocity gradient); with x_done
+// only the (y, z) part of the inverse remains
+int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
 {
     const int N = ctx->N;
     const fsd_pse_info &ps = ctx->pse;
@@ -1228,11 +938,16 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool inverse_yz)
     g.prefac = ps.prefac; g.expfac = ps.expfac;
     hipEvent_t ev;
     prof_begin(ctx, PROF_FFT, &ev);
-    {
+    if (use_fft_lds(ctx)) {
+        int rc = x_done ? 0 : k_fft_x(ctx, false);
+        if (!rc) rc = k_fft_yz_inverse(ctx);
+        if (rc) return rc;
+    } else {
         void *in[1] = {ctx->d_spec};
         void *out[1] = {ctx->d_grid};
-        if (rocfft_execute(inverse_yz ? ctx->plan_inv2 : ctx->plan_inv, in, out, ctx->info_inv) !=
-            rocfft_status_success) {
+        const int rc = fft_plans_3d(ctx);
+        if (rc) return rc;
+        if (rocfft_execute(ctx->plan_inv, in, out, ctx->info_inv) != rocfft_status_success) {
             ctx->err = "rocfft inverse failed";
             return FSD_E_HIP;
         }
@@ -1288,22 +1003,28 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
                                (int64_t)ctx->M);
         FSD_HIP(hipGetLastError());
         prof_end(ctx, PROF_SPREAD, ev);
-        const bool fx = ctx->tune.xpass == 0 && ctx->fx_B > 0 && ctx->plan_fwd2 && ctx->plan_inv2;
+        const bool fx = use_fft_lds(ctx);
         prof_begin(ctx, PROF_FFT, &ev);
-        {
+        if (fx) {
+            const int rc = k_fft_yz_forward(ctx);
+            if (rc) return rc;
+        } else {
             void *in[1] = {ctx->d_grid};
             void *out[1] = {ctx->d_spec};
-            if (rocfft_execute(fx ? ctx->plan_fwd2 : ctx->plan_fwd, in, out, ctx->info_fwd) != rocfft_status_success) {
+            const int rc = fft_plans_3d(ctx);
+            if (rc) return rc;
+            if (rocfft_execute(ctx->plan_fwd, in, out, ctx->info_fwd) != rocfft_status_success) {
                 ctx->err = "rocfft forward failed";
                 return FSD_E_HIP;
             }
         }
         prof_end(ctx, PROF_FFT, ev);
         prof_begin(ctx, PROF_GREEN, &ev);
-        GreenGeom gg{ps.Nx, ps.Ny, ps.Nz, ctx->box, ctx->p.xi, ps.eta, k_twopi(ctx)};
         if (fx) {   // x transforms and the Green's function in one pass
-            if (!launch_fft_x_green(ctx, gg)) { ctx->err = "no x-transform kernel for this grid"; return FSD_E_PARAM; }
+            const int rc = k_fft_x(ctx, true);
+            if (rc) return rc;
         } else {
+            GreenGeom gg{ps.Nx, ps.Ny, ps.Nz, ctx->box, ctx->p.xi, ps.eta, k_twopi(ctx)};
             hipLaunchKernelGGL(green_kernel, dim3(nblk(ctx->Mh, 256)), dim3(256), 0, ctx->stream, ctx->d_spec,
                                ctx->d_gridk, (int64_t)ctx->Mh, gg);
         }

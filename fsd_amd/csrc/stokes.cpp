@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -166,6 +167,38 @@ static void cell_dims(fsd_ctx *ctx)
         if (r_ < 0) return r_;                                                                      \
     } while (0)
 
+// the 3-D library plans (batched over the 11 fields), made on the first use: grids that do not fit
+// the LDS transforms, and the autotuner's comparison with them
+int fft_plans_3d(fsd_ctx *ctx)
+{
+    if (ctx->plan_fwd && ctx->plan_inv) return 0;
+    static std::mutex mu;   // contexts may step from several threads
+    std::lock_guard<std::mutex> lk(mu);
+    const fsd_pse_info &ps = ctx->pse;
+    size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
+    if (rocfft_plan_create(&ctx->plan_fwd, rocfft_placement_notinplace, rocfft_transform_type_real_forward,
+                           rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success ||
+        rocfft_plan_create(&ctx->plan_inv, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
+                           rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success) {
+        ctx->err = "rocfft_plan_create failed";
+        return FSD_E_HIP;
+    }
+    size_t w1 = 0, w2 = 0;
+    rocfft_plan_get_work_buffer_size(ctx->plan_fwd, &w1);
+    rocfft_plan_get_work_buffer_size(ctx->plan_inv, &w2);
+    ctx->fftwork_size = std::max(w1, w2);
+    if (ctx->fftwork_size) CK(hipMalloc(&ctx->d_fftwork, ctx->fftwork_size));
+    rocfft_execution_info_create(&ctx->info_fwd);
+    rocfft_execution_info_create(&ctx->info_inv);
+    rocfft_execution_info_set_stream(ctx->info_fwd, ctx->stream);
+    rocfft_execution_info_set_stream(ctx->info_inv, ctx->stream);
+    if (ctx->fftwork_size) {
+        rocfft_execution_info_set_work_buffer(ctx->info_fwd, ctx->d_fftwork, ctx->fftwork_size);
+        rocfft_execution_info_set_work_buffer(ctx->info_inv, ctx->d_fftwork, ctx->fftwork_size);
+    }
+    return 0;
+}
+
 static int alloc_all(fsd_ctx *ctx)
 {
     const int N = ctx->N;
@@ -225,47 +258,11 @@ static int alloc_all(fsd_ctx *ctx)
     CK(hipMalloc(&ctx->d_wave, sizeof(float) * 11 * (size_t)N));
     CK(hipMalloc(&ctx->d_rec, sizeof(float4) * 3 * (size_t)N));
     {
-        size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
-        if (rocfft_plan_create(&ctx->plan_fwd, rocfft_placement_notinplace, rocfft_transform_type_real_forward,
-                               rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success ||
-            rocfft_plan_create(&ctx->plan_inv, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
-                               rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success) {
-            ctx->err = "rocfft_plan_create failed";
-            return FSD_E_HIP;
-        }
-        size_t w1 = 0, w2 = 0;
-        rocfft_plan_get_work_buffer_size(ctx->plan_fwd, &w1);
-        rocfft_plan_get_work_buffer_size(ctx->plan_inv, &w2);
-        ctx->fftwork_size = std::max(w1, w2);
-        // the mobility's transforms: (y, z) by rocFFT, batched over the 11 fields and the x planes (the
-        // layout of the 3-D half spectrum), x and the Green's function in one kernel when Nx = 8 B,
-        // 5 <= B <= 11.  FSD_FFT_3D=1 keeps the 3-D plans and the separate Green's function.
+        // transforms: this library's kernels when the grid fits (k_fft.hip); FSD_FFT_3D=1 keeps the
+        // 3-D library plans and the separate Green's function
         const char *f3 = getenv("FSD_FFT_3D");
-        const int B = ps.Nx / 8;
-        if (!(f3 && f3[0] == '1') && ps.Nx % 8 == 0 && B >= 5 && B <= 11) {
-            size_t len2[2] = {(size_t)ps.Nz, (size_t)ps.Ny};
-            const size_t batch = 11 * (size_t)ps.Nx;
-            if (rocfft_plan_create(&ctx->plan_fwd2, rocfft_placement_notinplace, rocfft_transform_type_real_forward,
-                                   rocfft_precision_single, 2, len2, batch, nullptr) != rocfft_status_success ||
-                rocfft_plan_create(&ctx->plan_inv2, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
-                                   rocfft_precision_single, 2, len2, batch, nullptr) != rocfft_status_success) {
-                ctx->err = "rocfft_plan_create (2-D) failed";
-                return FSD_E_HIP;
-            }
-            rocfft_plan_get_work_buffer_size(ctx->plan_fwd2, &w1);
-            rocfft_plan_get_work_buffer_size(ctx->plan_inv2, &w2);
-            ctx->fftwork_size = std::max(ctx->fftwork_size, std::max(w1, w2));
-            ctx->fx_B = B;
-        }
-        if (ctx->fftwork_size) CK(hipMalloc(&ctx->d_fftwork, ctx->fftwork_size));
-        rocfft_execution_info_create(&ctx->info_fwd);
-        rocfft_execution_info_create(&ctx->info_inv);
-        rocfft_execution_info_set_stream(ctx->info_fwd, ctx->stream);
-        rocfft_execution_info_set_stream(ctx->info_inv, ctx->stream);
-        if (ctx->fftwork_size) {
-            rocfft_execution_info_set_work_buffer(ctx->info_fwd, ctx->d_fftwork, ctx->fftwork_size);
-            rocfft_execution_info_set_work_buffer(ctx->info_inv, ctx->d_fftwork, ctx->fftwork_size);
-        }
+        if (!(f3 && f3[0] == '1')) RC(fft_init(ctx));
+        if (!ctx->fft_lds) RC(fft_plans_3d(ctx));
     }
     // Ewald table
     ctx->ewald_nR = ps.ewald_n + 1;
@@ -369,7 +366,7 @@ static void free_all(fsd_ctx *ctx)
                     ctx->d_x64, ctx->d_r64, ctx->d_ybot64, ctx->d_norm64, ctx->d_refx32, ctx->d_refy32,
                     ctx->d_refr32, ctx->d_refd,
                     ctx->d_Z, ctx->d_lanV, ctx->d_lanw, ctx->d_lany0, ctx->d_lan_h, ctx->d_noise, ctx->d_posp,
-                    ctx->d_rfd_rhs, ctx->d_rfd_sol};
+                    ctx->d_rfd_rhs, ctx->d_rfd_sol, ctx->d_fft_tw, ctx->d_fft_loc};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (ctx->h_flags) hipHostFree(ctx->h_flags);
@@ -379,8 +376,6 @@ static void free_all(fsd_ctx *ctx)
     if (ctx->h_lan) hipHostFree(ctx->h_lan);
     if (ctx->plan_fwd) rocfft_plan_destroy(ctx->plan_fwd);
     if (ctx->plan_inv) rocfft_plan_destroy(ctx->plan_inv);
-    if (ctx->plan_fwd2) rocfft_plan_destroy(ctx->plan_fwd2);
-    if (ctx->plan_inv2) rocfft_plan_destroy(ctx->plan_inv2);
     if (ctx->info_fwd) rocfft_execution_info_destroy(ctx->info_fwd);
     if (ctx->info_inv) rocfft_execution_info_destroy(ctx->info_inv);
     for (auto &s : ctx->slots)
