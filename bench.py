@@ -46,7 +46,7 @@ HBM_PEAK_GBS = 8000.0
 GUESS_TEXT = {"previous": "previous solution", "extrapolate": "linear extrapolation of the last two solutions",
               "quadratic": "quadratic extrapolation of the last three solutions"}
 # kernel-class name -> kernel name in rocprofv3 traces
-KERNEL_NAMES = {"spread": "spread_tile2_kernel<8, 6>", "green": "x_green_kernel<4, 256, true>", "contract": "contract_tile2_kernel<13, 6>",
+KERNEL_NAMES = {"spread": "spread_mfma_kernel<6>", "green": "x_green_kernel<4, 256, true>", "contract": "contract_tile2_kernel<13, 6>",
                 "realspace": "realspace_kernel<16>", "rfu": "rfu_apply_kernel<8>", "sweep": "tp_sweep1_kernel",
                 "ichol": "ichol_level_kernel", "gmres_vec": "multidot_partial4_kernel", "ljit": "lj_fwd_kernel",
                 "jacobi": "jac_fwd_kernel"}

@@ -6,7 +6,7 @@
 //   lubrication per-pair records (neighbour, unit vector, five "12" resistance
 //               functions) + one symmetric 6x6 self block per particle,
 //               built once per step and reused by every R_FU apply;
-//   PSE grids   11 real fields [11][M] (M = Nx*Ny*Nz, z fastest) and their
+//   PSE grids   11 real fields [11][Nx][Ny][pitch] (z fastest; grid_pitch) and their
 //               half spectra [11][Nx*Ny*(Nz/2+1)] (rocFFT R2C/C2R);
 //   IC(0)       block-sparse lower factor on the RCM-permuted particle graph:
 //               per permuted particle a dense 6x6 diagonal block and one 6x6
@@ -193,7 +193,7 @@ struct ProfSlot {
 // Launch shapes chosen by the autotuner (fsd_autotune): each knob selects one of the
 // kernels or launch shapes that compute the same operator.
 struct fsd_tuning {
-    int spread = 0;          // 0: spread_tile2_kernel (tile 8, P 6), 1: spread_kernel (one workgroup per tile)
+    int spread = 0;          // 0: spread_mfma_kernel (P 6), 1: spread_kernel (one workgroup per tile)
     int contract = 0;        // 0: tile contraction (contract_tile2/contract_tile, when it fits in LDS),
                              // 1: one wave per particle (contract_kernel)
     int xpass = 0;           // 0: the transforms of k_fft.hip (when the grid fits them), 1: 3-D rocFFT
@@ -243,7 +243,7 @@ struct fsd_ctx {
 
     // PSE
     int M = 0, Mh = 0;
-    float *d_grid = nullptr;      // 11*M real
+    float *d_grid = nullptr;      // 11 real grids, rows of grid_pitch floats
     float2 *d_spec = nullptr;     // 11*Mh complex
     float4 *d_gridk = nullptr;    // Mh
     rocfft_plan plan_fwd = nullptr, plan_inv = nullptr;
@@ -426,6 +426,9 @@ int k_fft_yz_forward(fsd_ctx *ctx);
 int k_fft_x(fsd_ctx *ctx, bool green);
 int k_fft_yz_inverse(fsd_ctx *ctx);
 inline bool use_fft_lds(const fsd_ctx *ctx) { return ctx->fft_lds && ctx->tune.xpass == 0; }
+// row length of the grids in memory: whole float4s for this library's transforms (16-byte stores
+// and loads for odd lengths too), Nz for the 3-D plans
+inline int grid_pitch(const fsd_ctx *ctx) { return use_fft_lds(ctx) ? (ctx->pse.Nz + 3) / 4 * 4 : ctx->pse.Nz; }
 int k_precond_apply2(fsd_ctx *ctx, const float *b0, const float *b1, float *y0, float *y1, int n_rhs);
 int k_export_csr(fsd_ctx *ctx, const float4 *pos, int32_t *h_rowptr, int32_t *h_col, float *h_val,
                  int32_t *h_prow, int32_t *h_pcol, float *h_L, int64_t cap);

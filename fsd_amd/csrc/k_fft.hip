@@ -26,6 +26,7 @@ namespace {
 struct YzArgs {
     FftAxis y, z;
     int Nx, Ny, Nz, Nzh, zpairs;   // zpairs: pairs of y rows
+    int pz;                        // floats of a grid row in memory, a multiple of 4
 };
 
 // LDS: the plane, row y at y Nzh complex (rows 2p, 2p + 1 share 2 Nzh places while they are one
@@ -36,7 +37,7 @@ __device__ __forceinline__ void load_tables(const FftAxis &y, const FftAxis &z, 
     for (int i = threadIdx.x; i < z.n; i += blockDim.x) { tw[y.n + i] = z.tw[i]; loc[y.n + i] = z.loc[i]; }
 }
 
-constexpr int YZ_LOADS = 8;        // global loads a thread has in flight
+constexpr int YZ_LOADS = 4;        // global loads of 16 bytes a thread has in flight
 
 // most (row pair, kz) tasks of a thread in the real unpacking: bounds the plane to NT YZ_HOLD pairs of modes
 template <int NT>
@@ -73,23 +74,26 @@ __global__ void __launch_bounds__(NT) yz_forward_kernel(YzArgs a, const float *g
     unsigned short *loc = reinterpret_cast<unsigned short *>(tw + Ny + Nz);
     load_tables(a.y, a.z, tw, loc);
     // real rows 2p and 2p + 1 as the real and imaginary part of one row
-    const int np = Ny * Nz;
-    const float *in = grid + (int64_t)blockIdx.x * np;
-    const fft::FastDiv by_z(Nz);
+    const int p4 = a.pz / 4, np = Ny * p4;
+    const float4 *in = reinterpret_cast<const float4 *>(grid + (int64_t)blockIdx.x * Ny * a.pz);
+    const fft::FastDiv by_z(p4);
     float *fb = reinterpret_cast<float *>(buf);
     for (int i0 = 0; i0 < np; i0 += NT * YZ_LOADS) {
-        float v[YZ_LOADS];
+        float4 v[YZ_LOADS];
 #pragma unroll
-        for (int u = 0; u < YZ_LOADS; ++u) {
-            const int i = i0 + u * NT + threadIdx.x;
-            v[u] = i < np ? in[i] : 0.f;
-        }
+        for (int u = 0; u < YZ_LOADS; ++u) v[u] = in[min(i0 + u * NT + (int)threadIdx.x, np - 1)];
 #pragma unroll
         for (int u = 0; u < YZ_LOADS; ++u) {
             const int i = i0 + u * NT + threadIdx.x;
             int z;
             const int y = by_z(i, z);
-            if (i < np) fb[2 * ((y >> 1) * row + z) + (y & 1)] = v[u];
+            if (i < np) {
+                float *o = fb + 2 * ((y >> 1) * row + 4 * z) + (y & 1);
+                const float w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (4 * z + k < Nz) o[2 * k] = w[k];
+            }
         }
     }
     if (Ny & 1)   // the last row's missing partner
@@ -152,18 +156,19 @@ __global__ void __launch_bounds__(NT) yz_inverse_kernel(YzArgs a, const float2 *
     const fft::FastDiv by_h(Nzh);
     if (Ny & 1)
         for (int k = threadIdx.x; k < Nzh; k += NT) buf[Ny * Nzh + k] = make_float2(0.f, 0.f);
-    for (int i0 = 0; i0 < nh; i0 += NT * YZ_LOADS) {
-        float2 v[YZ_LOADS];
-        unsigned short r[YZ_LOADS];
+    constexpr int LOADS = 2 * YZ_LOADS;
+    for (int i0 = 0; i0 < nh; i0 += NT * LOADS) {
+        float2 v[LOADS];
+        unsigned short r[LOADS];
 #pragma unroll
-        for (int u = 0; u < YZ_LOADS; ++u) {
+        for (int u = 0; u < LOADS; ++u) {
             const int i = i0 + u * NT + threadIdx.x;
             int k;
             v[u] = i < nh ? in[i] : make_float2(0.f, 0.f);
             r[u] = i < nh ? a.y.loc[by_h(i, k)] : 0;
         }
 #pragma unroll
-        for (int u = 0; u < YZ_LOADS; ++u) {
+        for (int u = 0; u < LOADS; ++u) {
             const int i = i0 + u * NT + threadIdx.x;
             int k;
             by_h(i, k);
@@ -205,14 +210,17 @@ __global__ void __launch_bounds__(NT) yz_inverse_kernel(YzArgs a, const float2 *
         __syncthreads();
     }
     fft::transform<true, NT>(buf, a.z, pairs, [&](int tasks) { return ZRows(tasks, row); }, 1, tw + Ny);
-    const int np = Ny * Nz;
-    float *out = grid + (int64_t)blockIdx.x * np;
+    // rows of pz floats; the padding repeats the row's end
+    const int p4 = a.pz / 4, np = Ny * p4;
+    float4 *out = reinterpret_cast<float4 *>(grid + (int64_t)blockIdx.x * Ny * a.pz);
     const float *fb = reinterpret_cast<const float *>(buf);
-    const fft::FastDiv by_z(Nz);
+    const fft::FastDiv by_z(p4);
     for (int i = threadIdx.x; i < np; i += NT) {
         int z;
         const int y = by_z(i, z);
-        out[i] = fb[2 * ((y >> 1) * row + z) + (y & 1)];
+        const float *v = fb + 2 * ((y >> 1) * row) + (y & 1);
+        z *= 4;
+        out[i] = make_float4(v[2 * z], v[2 * min(z + 1, Nz - 1)], v[2 * min(z + 2, Nz - 1)], v[2 * min(z + 3, Nz - 1)]);
     }
 }
 
@@ -372,6 +380,7 @@ static YzArgs yz_args(const fsd_ctx *ctx)
     a.Nx = ctx->pse.Nx; a.Ny = ctx->pse.Ny; a.Nz = ctx->pse.Nz;
     a.Nzh = a.Nz / 2 + 1;
     a.zpairs = (a.Ny + 1) / 2;
+    a.pz = grid_pitch(ctx);
     return a;
 }
 

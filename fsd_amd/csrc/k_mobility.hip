@@ -129,9 +129,23 @@ __global__ void fc_records_kernel(const float *gF, int N, float4 *rec)
 // ------------------------------------------------------------ spreading
 struct SpreadGeom {
     int Nx, Ny, Nz, P, tile, tnx, tny, tnz;
+    int pz;                    // row length of the grids in memory (grid_pitch)
     float hx, hy, hz, Lx2, Ly2, Lz2, xy;
     float prefac, expfac;
 };
+
+static SpreadGeom spread_geom(const fsd_ctx *ctx)
+{
+    const fsd_pse_info &ps = ctx->pse;
+    SpreadGeom g;
+    g.Nx = ps.Nx; g.Ny = ps.Ny; g.Nz = ps.Nz; g.P = ps.P; g.tile = ctx->tile;
+    g.tnx = ctx->tiles[0]; g.tny = ctx->tiles[1]; g.tnz = ctx->tiles[2];
+    g.pz = grid_pitch(ctx);
+    g.hx = ps.gridh_x; g.hy = ps.gridh_y; g.hz = ps.gridh_z;
+    g.Lx2 = ctx->box.Lx / 2.0f; g.Ly2 = ctx->box.Ly / 2.0f; g.Lz2 = ctx->box.Lz / 2.0f; g.xy = ctx->box.xy;
+    g.prefac = ps.prefac; g.expfac = ps.expfac;
+    return g;
+}
 
 // The origin cells whose stencils reach a tile [t0, t0 + tile) on one axis are
 // t0 - P + 1 .. t0 + tile - 1 (wrapped): `halo_axis` lists them once each
@@ -255,85 +269,79 @@ __global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const float4 
         }
     }
     if (inside) {
-        const int64_t id = ((int64_t)gx * g.Ny + gy) * g.Nz + gz;
+        const int64_t id = ((int64_t)gx * g.Ny + gy) * g.pz + gz;
 #pragma unroll
         for (int c = 0; c < 11; ++c) grid[c * M + id] = acc[c];
     }
 }
 
-// Spreading for the usual stencil (P = 6, tile 8) with the work of a grid
-// point limited to its own stencil window.  The tile's H^3 halo of origin
-// cells (H = tile + P - 1) is counted and scanned in LDS, its particles are
-// staged in LDS in (x, y, z) halo-cell order, and a point at local (lx, ly,
-// lz) visits, for each of its 36 halo columns (lx + a, ly + b), the
-// consecutive staged particles of cells lz .. lz + P - 1: exactly the
-// particles whose stencil covers it.  A tile whose halo holds more than
-// SP2_CAP particles reads them from global memory instead (about 190 are staged
-// at volume fraction 0.45; the cap keeps the LDS at 50 KB, three workgroups per
-// CU).  Same weights and accumulation as spread_kernel (each point sums its
-// particles in the same cell order, and writes once).
-#define SP2_CAP 512
-// contribution of one particle (origin o, position p, records r) to grid point (gx, gy, gz)
-__device__ __forceinline__ void spread_point_add(const SpreadGeom &g, int gx, int gy, int gz, int o0, int o1, int o2,
-                                                 float p0, float p1, float p2, float4 r0, float4 r1, float4 r2,
-                                                 float *acc)
+// Spreading for the usual stencil (P = 6) on the matrix cores: one workgroup per tile of 8^3
+// nodes, one wave per 4 x 4 columns by 4 nodes along z.
+//
+// A node lies in the stencils of ~19 spheres at volume fraction 0.45 and each adds 11
+// products.  For the 16 columns of a wave and one z that is a matrix product,
+//   grid[field, column] = sum over spheres rec[field, sphere] (e[sphere, column] w[sphere, z]),
+// with e the Gaussian along x and y (zero outside the sphere's stencil) and w its factor along
+// z: mfma 16x16x4 in FP32 takes four spheres at a time, fields (11 of 16 rows) by columns.  A
+// lane forms one e per step and multiplies it by the four w, so the four products of a step
+// share it and the records.  Per node this takes 64 spheres (those that reach any of the 4 x 4
+// x 4 nodes), of which 19 count, at twice the VALU's rate.  The same sums on the VALU were bound
+// by lanes that waited for the longest of 36 short runs of spheres (34.6 us per product at N =
+// 32768) or, with those runs merged, by LDS bank conflicts (each lane its own sphere: 34.6 us).
+// The tile's halo of 13^3 origin cells is staged in LDS.  Its spheres are in the order of buckets
+// (x, third of z, y): a wave of the lower nodes needs the first two thirds, one of the upper
+// nodes the last two, so its spheres are 18 runs of nine buckets each, which it lists.  A halo of
+// more than SP2_CAP spheres is staged in parts.  Every node sums its spheres in bucket order and is
+// written once (no atomics).
+#define SP2_CAP 256
+typedef float mfma_f4 __attribute__((ext_vector_type(4)));
+template <int PP>
+__global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const float4 *pos, const int *orig,
+                                                             const float4 *rec, const int *ostart, const int *olist,
+                                                             float *grid, int64_t M)
 {
-    int tx = gx - o0; tx += (tx < 0) ? g.Nx : 0; tx -= (tx >= g.Nx) ? g.Nx : 0;
-    int ty = gy - o1; ty += (ty < 0) ? g.Ny : 0; ty -= (ty >= g.Ny) ? g.Ny : 0;
-    int tz = gz - o2; tz += (tz < 0) ? g.Nz : 0; tz -= (tz >= g.Nz) ? g.Nz : 0;
-    const float uy = g.hy * (float)(o1 + ty) - g.Ly2;
-    const float dx = g.hx * (float)(o0 + tx) - g.Lx2 + g.xy * uy - p0;
-    const float dy = uy - p1;
-    const float dz = g.hz * (float)(o2 + tz) - g.Lz2 - p2;
-    const float w = g.prefac * __expf(-g.expfac * (dx * dx + dy * dy + dz * dz));
-    acc[0] += w * r0.x; acc[1] += w * r0.y; acc[2] += w * r0.z;
-    acc[3] += w * r0.w; acc[4] += w * r1.x; acc[5] += w * r1.y; acc[6] += w * r1.z;
-    acc[7] += w * r1.w; acc[8] += w * r2.x; acc[9] += w * r2.y; acc[10] += w * r2.z;
-}
-
-template <int TILE, int PP>
-__global__ void __launch_bounds__(512) spread_tile2_kernel(SpreadGeom g, const float4 *pos, const int *orig,
-                                                           const float4 *rec, const int *ostart, const int *olist,
-                                                           float *grid, int64_t M)
-{
-    constexpr int H = TILE + PP - 1;
-    constexpr int NQ = H * H * H;                // halo cells
-    constexpr int PER = (NQ + 511) / 512;
-    __shared__ int s_beg[NQ];                    // first olist entry of each halo cell
-    __shared__ int s_base[NQ + 1];               // exclusive scan of the cells' counts
-    __shared__ int s_wsum[8];
-    // staged particle: the offsets (cx, cy, cy - py, cz) of its stencil in the tile's frame and its
-    // records scaled by the Gaussian's prefactor
-    __shared__ float4 s_c[SP2_CAP];
-    __shared__ float4 s_r[SP2_CAP][3];
+    constexpr int T = 8, BL = 4, H = T + PP - 1, HB = BL + PP - 1, NT = 512, NW = NT / 64;
+    constexpr int ZP[4] = {0, H - HB, HB, H};     // thirds of the halo's z cells: 4, 5 and 4 of them
+    constexpr int NB = 3 * H * H;                 // buckets
+    static_assert(NB <= NT && SP2_CAP <= NT, "a bucket and a staged sphere per thread");
+    __shared__ int s_base[NB + 1];                // exclusive scan of the buckets' counts
+    __shared__ int s_beg[2][NB];                  // olist position of a bucket's two pieces (z may wrap) ...
+    __shared__ int s_first[NB];                   // ... and the count of the first
+    __shared__ int s_wsum[NW];
+    __shared__ float4 s_c[SP2_CAP];               // scaled offsets of the tile's first column (x, y), its columns
+    __shared__ float4 s_z[SP2_CAP][2];            // factors along z
+    __shared__ float s_r[SP2_CAP * 12 + 4];       // records; rows 12 to 15 of a product read past a sphere's 12
+    __shared__ unsigned short s_list[NW][SP2_CAP + 8];
 
     const int tile_id = xcd_remap(blockIdx.x, gridDim.x);
     const int tz_i = tile_id % g.tnz, ty_i = (tile_id / g.tnz) % g.tny, tx_i = tile_id / (g.tnz * g.tny);
-    const int x0 = tx_i * TILE, y0 = ty_i * TILE, z0 = tz_i * TILE;
-    const int lt = threadIdx.x;
-    // counts of the halo cells, PER consecutive cells per thread
-    int cnt[PER];
-    int sum = 0;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int q = lt * PER + k;
-        cnt[k] = 0;
-        if (q < NQ) {
-            const int hx = q / (H * H), hy = (q / H) % H, hz = q % H;
-            int x = x0 - (PP - 1) + hx, y = y0 - (PP - 1) + hy, z = z0 - (PP - 1) + hz;
-            x += (x < 0) ? g.Nx : 0; x -= (x >= g.Nx) ? g.Nx : 0; x -= (x >= g.Nx) ? g.Nx : 0;
-            y += (y < 0) ? g.Ny : 0; y -= (y >= g.Ny) ? g.Ny : 0; y -= (y >= g.Ny) ? g.Ny : 0;
-            z += (z < 0) ? g.Nz : 0; z -= (z >= g.Nz) ? g.Nz : 0; z -= (z >= g.Nz) ? g.Nz : 0;
-            const int c = (x * g.Ny + y) * g.Nz + z;
-            const int b = ostart[c];
-            s_beg[q] = b;
-            cnt[k] = ostart[c + 1] - b;
-        }
-        sum += cnt[k];
+    const int x0 = tx_i * T, y0 = ty_i * T, z0 = tz_i * T;
+    const int lt = threadIdx.x, lane = lt & 63, wv = lt >> 6;
+    auto wrap = [](int v, int n) {
+        v += (v < 0) ? n : 0;
+        v -= (v >= n) ? n : 0;
+        return v - ((v >= n) ? n : 0);
+    };
+    // a third's cells: n0 from cell za on, the others from cell 0 on (grids have at least 8 points)
+    auto third = [&](int p, int &za, int &n0) {
+        za = wrap(z0 - (PP - 1) + ZP[p], g.Nz);
+        n0 = min(ZP[p + 1] - ZP[p], g.Nz - za);
+    };
+    int cnt = 0;
+    if (lt < NB) {
+        const int hx = lt / (3 * H), r = lt - hx * (3 * H), p = r / H, hy = r - p * H;
+        const int c = (wrap(x0 - (PP - 1) + hx, g.Nx) * g.Ny + wrap(y0 - (PP - 1) + hy, g.Ny)) * g.Nz;
+        int za, n0;
+        third(p, za, n0);
+        const int nz = ZP[p + 1] - ZP[p];
+        const int b0 = ostart[c + za], e0 = ostart[c + za + n0];
+        const int b1 = n0 < nz ? ostart[c] : 0, e1 = n0 < nz ? ostart[c + nz - n0] : 0;
+        s_beg[0][lt] = b0;
+        s_beg[1][lt] = b1;
+        s_first[lt] = e0 - b0;
+        cnt = (e0 - b0) + (e1 - b1);
     }
-    // exclusive scan over the threads: wave inclusive scan, then wave offsets
-    const int lane = lt & 63, wv = lt >> 6;
-    int inc = sum;
+    int inc = cnt;
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const int v = __shfl_up(inc, o, 64);
@@ -341,111 +349,135 @@ __global__ void __launch_bounds__(512) spread_tile2_kernel(SpreadGeom g, const f
     }
     if (lane == 63) s_wsum[wv] = inc;
     __syncthreads();
-    int woff = 0;
-    for (int w = 0; w < wv; ++w) woff += s_wsum[w];
-    int run = woff + inc - sum;
+    int before = 0, total = 0;
 #pragma unroll
-    for (int k = 0; k < PER; ++k) {
-        const int q = lt * PER + k;
-        if (q < NQ) s_base[q] = run;
-        run += cnt[k];
+    for (int w = 0; w < NW; ++w) {
+        before += w < wv ? s_wsum[w] : 0;
+        total += s_wsum[w];
     }
-    int total = 0;
-    for (int w = 0; w < 8; ++w) total += s_wsum[w];
-    if (lt == 0) s_base[NQ] = total;
-    const bool staged = total <= SP2_CAP;
+    if (lt < NB) s_base[lt] = before + inc - cnt;
+    if (lt == 0) s_base[NB] = total;
     __syncthreads();
-    if (staged) {
-        // staged slots sl = lt and lt + 512 (at most SP2_CAP of them): the halo cell holding the
-        // slot by binary search over the scan (the last cell whose base is <= sl is non-empty and
-        // holds it), then the particle's index and records; the loads of both slots overlap
-        static_assert(SP2_CAP <= 2 * 512, "two staged slots per thread");
-        int q2[2], sl2[2];
+
+    // lengths in units in which the Gaussian is 2^-(d^2)
+    const float unit = sqrtf(g.expfac * 1.44269504088896341f);
+    const int col = lane & 15, quad = lane >> 4;
+    const int bx = (wv >> 1 & 1) * BL, by = (wv & 1) * BL, half = wv >> 2;   // the wave's nodes
+    const int lx = bx + col / BL, ly = by + col % BL;
+    const float ay = unit * (g.hy * (float)ly);
+    const float ax = unit * (g.hx * (float)lx) + g.xy * ay;
+    const unsigned here = (1u << lx) | (1u << (T + ly));
+    mfma_f4 acc[4];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int sl = lt + h * 512;
-            int lo = 0, hi = NQ - 1;
-            while (lo < hi) {
+    for (int k = 0; k < 4; ++k) acc[k] = mfma_f4{0.f, 0.f, 0.f, 0.f};
+
+    for (int base = 0; base < total; base += SP2_CAP) {
+        if (base) __syncthreads();                // the part before is done with
+        const int p = base + lt;
+        if (lt < SP2_CAP && p < total) {
+            // the bucket by binary search over the scan (the last one whose base is not above the position
+            // holds it), then the index and the records
+            int lo = 0, hi = NB - 1;
+#pragma unroll
+            for (int step = 0; step < 9; ++step) {   // 2^9 > NB
                 const int mid = (lo + hi + 1) >> 1;
-                if (s_base[mid] <= sl) lo = mid; else hi = mid - 1;
+                const bool right = lo < hi && s_base[mid] <= p;
+                hi = (lo < hi && !right) ? mid - 1 : hi;
+                lo = right ? mid : lo;
             }
-            q2[h] = lo;
-            sl2[h] = sl;
-        }
-        int i2[2];
+            const int o = p - s_base[lo], n1 = s_first[lo];
+            const bool second = o >= n1;
+            const int i = olist[second ? s_beg[1][lo] + (o - n1) : s_beg[0][lo] + o];
+            const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
+            const float4 q = pos[i];
+            const float4 r0 = rec[3 * (int64_t)i], r1 = rec[3 * (int64_t)i + 1], r2 = rec[3 * (int64_t)i + 2];
+            // the sphere's origin is the halo cell (hc) up to the period, so a node at local (lx, ly, lz)
+            // of its stencil is node o + (P - 1) - hc + l: with the node's position
+            // h (o + P - 1 - hc) - L/2 + h l, its offset from the sphere is c + h l
+            const int hxc = lo / (3 * H), rb = lo - hxc * (3 * H), zp = rb / H, hyc = rb - zp * H;
+            int za, n0;
+            third(zp, za, n0);
+            const int wz = ((oz % g.Nz) + g.Nz) % g.Nz;
+            const int hzc = ZP[zp] + (second ? n0 + wz : wz - za);
+            const float cy = g.hy * (float)(oy + (PP - 1) - hyc) - g.Ly2;
+            const float cx = g.hx * (float)(ox + (PP - 1) - hxc) - g.Lx2 - q.x + g.xy * cy;
+            const float cz = g.hz * (float)(oz + (PP - 1) - hzc) - g.Lz2 - q.z;
+            float w[T];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const bool ok = sl2[h] < total;
-            i2[h] = olist[ok ? s_beg[q2[h]] + (sl2[h] - s_base[q2[h]]) : 0];
-        }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int sl = sl2[h], i = i2[h];
-            if (sl < total) {
-                // the particle's origin is the halo cell (hc) up to the period, so a point at local
-                // (lx, ly, lz) of its stencil is node o + (P - 1) - hc + l: with the node's position
-                // h (o + P - 1 - hc) - L/2 + h l, its offset from the particle is c + h l
-                const int q = q2[h];
-                const int hxc = q / (H * H), hyc = (q / H) % H, hzc = q % H;
-                const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
-                const float4 p = pos[i];
-                const float cx = g.hx * (float)(ox + (PP - 1) - hxc) - g.Lx2 - p.x;
-                const float cy = g.hy * (float)(oy + (PP - 1) - hyc) - g.Ly2;
-                const float cz = g.hz * (float)(oz + (PP - 1) - hzc) - g.Lz2 - p.z;
-                s_c[sl] = make_float4(cx, cy, cy - p.y, cz);
-                const float4 r0 = rec[3 * (int64_t)i], r1 = rec[3 * (int64_t)i + 1], r2 = rec[3 * (int64_t)i + 2];
-                const float f = g.prefac;
-                s_r[sl][0] = make_float4(f * r0.x, f * r0.y, f * r0.z, f * r0.w);
-                s_r[sl][1] = make_float4(f * r1.x, f * r1.y, f * r1.z, f * r1.w);
-                s_r[sl][2] = make_float4(f * r2.x, f * r2.y, f * r2.z, 0.f);
+            for (int k = 0; k < T; ++k) {
+                const float dz = unit * (cz + g.hz * (float)k);
+                const int s = k + (PP - 1) - hzc;     // node of the stencil
+                w[k] = (s >= 0 && s < PP) ? g.prefac * __builtin_amdgcn_exp2f(-(dz * dz)) : 0.f;
             }
+            // columns of the tile inside the stencil: hc - P + 1 .. hc along each axis
+            const unsigned six = (1u << PP) - 1u;
+            const unsigned mx = ((six << hxc) >> (PP - 1)) & 0xffu, my = ((six << hyc) >> (PP - 1)) & 0xffu;
+            s_c[lt] = make_float4(unit * cx, unit * (cy - q.y), __uint_as_float(mx | (my << T)), 0.f);
+            s_z[lt][0] = make_float4(w[0], w[1], w[2], w[3]);
+            s_z[lt][1] = make_float4(w[4], w[5], w[6], w[7]);
+            float4 *r = reinterpret_cast<float4 *>(s_r + 12 * lt);
+            r[0] = r0;
+            r[1] = r1;
+            r[2] = r2;
+        }
+        // this wave's spheres of the part: lane k < 18 lists run k
+        unsigned short *list = s_list[wv];
+        int len = 0;
+        {
+            int b = 0, n = 0;
+            if (lane < 2 * HB) {
+                const int q = ((bx + (lane >> 1)) * 3 + half + (lane & 1)) * H + by;
+                b = max(s_base[q] - base, 0);
+                n = max(min(s_base[q + HB] - base, SP2_CAP) - b, 0);
+            }
+            int at = n;
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) {
+                const int v = __shfl_up(at, o, 64);
+                if (lane >= o) at += v;
+            }
+            len = __shfl(at, 31, 64);
+            at -= n;
+            for (int k = 0; k < n; ++k) list[at + k] = (unsigned short)(b + k);
+            if (lane < 8) list[len + lane] = 0;   // idle spheres of the last step
+        }
+        __syncthreads();
+        for (int t0 = 0; t0 < len; t0 += 8) {
+            const int t = t0 + quad, sa = list[t], sb = list[t + 4];
+            const float4 ca = s_c[sa], cb = s_c[sb], za = s_z[sa][half], zb = s_z[sb][half];
+            const float ra = s_r[12 * sa + col], rb = s_r[12 * sb + col];
+            const float dxa = ca.x + ax, dya = ca.y + ay, dxb = cb.x + ax, dyb = cb.y + ay;
+            const bool ina = (__float_as_uint(ca.z) & here) == here && t < len;
+            const bool inb = (__float_as_uint(cb.z) & here) == here && t + 4 < len;
+            const float ea = ina ? __builtin_amdgcn_exp2f(-(dxa * dxa + dya * dya)) : 0.f;
+            const float eb = inb ? __builtin_amdgcn_exp2f(-(dxb * dxb + dyb * dyb)) : 0.f;
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra, ea * za.x, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra, ea * za.y, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra, ea * za.z, acc[2], 0, 0, 0);
+            acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(ra, ea * za.w, acc[3], 0, 0, 0);
+            acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb, eb * zb.x, acc[0], 0, 0, 0);
+            acc[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb, eb * zb.y, acc[1], 0, 0, 0);
+            acc[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb, eb * zb.z, acc[2], 0, 0, 0);
+            acc[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(rb, eb * zb.w, acc[3], 0, 0, 0);
         }
     }
-    __syncthreads();
-    const int lx = lt / (TILE * TILE), ly = (lt / TILE) % TILE, lz = lt % TILE;
-    const int gx = x0 + lx, gy = y0 + ly, gz = z0 + lz;
-    if (lt >= TILE * TILE * TILE || gx >= g.Nx || gy >= g.Ny || gz >= g.Nz) return;
-    float acc[11];
+    // a lane holds fields 4 quad .. 4 quad + 3 of its column
+    const int gx = x0 + lx, gy = y0 + ly, gz = z0 + 4 * half;
+    if (gx >= g.Nx || gy >= g.Ny || gz >= g.Nz) return;
+    const int64_t id = ((int64_t)gx * g.Ny + gy) * g.pz + gz;
 #pragma unroll
-    for (int c = 0; c < 11; ++c) acc[c] = 0.f;
-    // one loop per source (separate code, so the staged loop reads LDS only)
-    if (staged) {
-        // offsets of this point in the tile's frame; a staged particle's are added to them
-        const float ax = g.hx * (float)lx, ay = g.hy * (float)ly, az = g.hz * (float)lz;
-        const float nexp = -g.expfac;
-        for (int a = 0; a < PP; ++a)
-            for (int b = 0; b < PP; ++b) {
-                const int q0 = ((lx + a) * H + (ly + b)) * H + lz;
-                const int s1 = s_base[q0 + PP];
-                for (int sl = s_base[q0]; sl < s1; ++sl) {
-                    const float4 c = s_c[sl];
-                    const float uy = c.y + ay;
-                    const float dx = c.x + ax + g.xy * uy, dy = c.z + ay, dz = c.w + az;
-                    const float e = __expf(nexp * (dx * dx + dy * dy + dz * dz));
-                    const float4 r0 = s_r[sl][0], r1 = s_r[sl][1], r2 = s_r[sl][2];
-                    acc[0] += e * r0.x; acc[1] += e * r0.y; acc[2] += e * r0.z;
-                    acc[3] += e * r0.w; acc[4] += e * r1.x; acc[5] += e * r1.y; acc[6] += e * r1.z;
-                    acc[7] += e * r1.w; acc[8] += e * r2.x; acc[9] += e * r2.y; acc[10] += e * r2.z;
-                }
-            }
-    } else {
-        for (int a = 0; a < PP; ++a)
-            for (int b = 0; b < PP; ++b) {
-                const int q0 = ((lx + a) * H + (ly + b)) * H + lz;
-                for (int q = q0; q < q0 + PP; ++q) {
-                    const int beg = s_beg[q], n = s_base[q + 1] - s_base[q];
-                    for (int m = 0; m < n; ++m) {
-                        const int i = olist[beg + m];
-                        const float4 p = pos[i];
-                        spread_point_add(g, gx, gy, gz, orig[3 * i], orig[3 * i + 1], orig[3 * i + 2], p.x, p.y, p.z,
-                                         rec[3 * (int64_t)i], rec[3 * (int64_t)i + 1], rec[3 * (int64_t)i + 2], acc);
-                    }
-                }
-            }
+    for (int q = 0; q < 4; ++q) {
+        const int f = 4 * quad + q;
+        if (f >= 11) break;
+        float *o = grid + (int64_t)f * M + id;
+        if (g.pz % 4 == 0) {                       // 16-byte aligned rows; the padding takes the rest
+            *reinterpret_cast<float4 *>(o) = make_float4(acc[0][q], acc[1][q], acc[2][q], acc[3][q]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (gz + k < g.Nz) o[k] = acc[k][q];
+        }
     }
-    const int64_t id = ((int64_t)gx * g.Ny + gy) * g.Nz + gz;
-#pragma unroll
-    for (int c = 0; c < 11; ++c) grid[c * M + id] = acc[c];
 }
 
 // ------------------------------------------------------------ Green kernel
@@ -493,7 +525,7 @@ __global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float
             const float dx = g.hx * (float)x - g.Lx2 + g.xy * uy - p.x;
             x = ((x % g.Nx) + g.Nx) % g.Nx;
             const float w = quadw_prefac * __expf(-g.expfac * (dx * dx + dy * dy + dz * dz));
-            const int64_t id = ((int64_t)x * g.Ny + y) * g.Nz + z;
+            const int64_t id = ((int64_t)x * g.Ny + y) * g.pz + z;
 #pragma unroll
             for (int c = 0; c < 11; ++c) acc[c] += w * grid[c * M + id];
         }
@@ -546,7 +578,7 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
         x -= (x >= g.Nx) ? g.Nx : 0; x -= (x >= g.Nx) ? g.Nx : 0;
         y -= (y >= g.Ny) ? g.Ny : 0; y -= (y >= g.Ny) ? g.Ny : 0;
         z -= (z >= g.Nz) ? g.Nz : 0; z -= (z >= g.Nz) ? g.Nz : 0;
-        s_g[idx] = grid[c * M + ((int64_t)x * g.Ny + y) * g.Nz + z];
+        s_g[idx] = grid[c * M + ((int64_t)x * g.Ny + y) * g.pz + z];
     }
     __syncthreads();
     if (lt == 0) {
@@ -603,20 +635,27 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
 // The tile contraction for the usual stencil (P = 6, tile 8, S = 13) with
 // compile-time sizes, the 11 fields split over two workgroups per tile
 // (fields [0, 6) and [6, 11)) so that three workgroups share a CU and one's
-// halo load overlaps another's arithmetic.  Same arithmetic per output as
-// contract_tile_kernel.
+// halo load overlaps another's arithmetic.
+//
+// Bound by VALU and LDS issue, not by HBM (18.8 MB at N = 32768 take 4 us).  So a
+// particle has 16 lanes, not a wave: 12 of them each sum 18 of its 216 nodes (one z,
+// three y, all x) and the sums over lanes are four DPP steps inside a row of 16, for
+// four particles at once (a wave per particle kept 36 lanes busy and spent more on the
+// sums than on the nodes).  The LDS block is node-major, six fields to a node, so a node
+// is three 8-byte reads; lanes of consecutive z are six words apart, which conflicts
+// nowhere inside a particle.  The block is loaded by 16 lanes per row of 13 nodes: the
+// wrapped row offsets come from a table and z is fixed per lane.
 #define CT_NF 6
 #define CT_PCAP 128   // particles of a tile staged in LDS (about 45 in an 8^3 tile at volume fraction 0.45)
 template <int S, int PP>
-__global__ void __launch_bounds__(512) contract_tile2_kernel(SpreadGeom g, const float4 *pos, const int *orig,
+__global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, const float4 *pos, const int *orig,
                                                              const int *ostart, const int *olist, const float *grid,
                                                              int64_t M, float quadw_prefac, float *wave)
 {
-    constexpr int S3 = S * S * S;
-    constexpr int TILE = S - PP + 1;
-    extern __shared__ float s_g[];           // [CT_NF][S][S][S]
+    constexpr int S2 = S * S, TILE = S - PP + 1, NT = 512, RL = 16;   // RL: lanes of a particle
+    static_assert(TILE * TILE == 64 && PP == 6 && CT_NF % 2 == 0, "a wave scans the tile's columns");
+    extern __shared__ float s_g[];           // [S][S][S][CT_NF]
     __shared__ int s_run_beg[TILE * TILE], s_run_off[TILE * TILE + 1];
-    __shared__ int s_w[3][S];                // wrapped grid index of each halo offset
     __shared__ int s_pi[CT_PCAP], s_pb[CT_PCAP];      // staged particles: index, local origin (bytes)
     __shared__ float4 s_pc[CT_PCAP];                  //   and offsets from the particle
     const int item = xcd_remap(blockIdx.x, gridDim.x);   // a slab of tiles per XCD: halos shared in its L2
@@ -624,59 +663,26 @@ __global__ void __launch_bounds__(512) contract_tile2_kernel(SpreadGeom g, const
     const int f0 = grp ? CT_NF : 0, nf = grp ? 11 - CT_NF : CT_NF;
     const int tz_i = tile_id % g.tnz, ty_i = (tile_id / g.tnz) % g.tny, tx_i = tile_id / (g.tnz * g.tny);
     const int x0 = tx_i * TILE, y0 = ty_i * TILE, z0 = tz_i * TILE;
-    const int lt = threadIdx.x;
+    const int lt = threadIdx.x, lane16 = lt % RL;
     const int xe = min(x0 + TILE, g.Nx), ye = min(y0 + TILE, g.Ny), z1 = min(z0 + TILE, g.Nz);
-    const int ncx = xe - x0, ncy = ye - y0;
-    if (lt < ncx * ncy) {
-        const int x = x0 + lt / ncy, y = y0 + lt % ncy;
-        const int cb = (x * g.Ny + y) * g.Nz;
-        const int b0 = ostart[cb + z0], b1 = ostart[cb + z1];
-        s_run_beg[lt] = b0;
-        s_run_off[lt + 1] = b1 - b0;
-    }
-    if (lt < 3 * S) {
-        const int ax = lt / S, o = lt - ax * S;
-        const int n = ax == 0 ? g.Nx : (ax == 1 ? g.Ny : g.Nz);
-        int v = (ax == 0 ? x0 : (ax == 1 ? y0 : z0)) + o;
+    const int ncx = xe - x0, ncy = ye - y0, nruns = ncx * ncy;
+    auto wrap = [](int v, int n) {           // v < 3 n (the halo may pass a short axis twice)
         v -= (v >= n) ? n : 0;
-        v -= (v >= n) ? n : 0;
-        s_w[ax][o] = v;
-    }
-    __syncthreads();
-    // grid block of this workgroup's fields, wrapped: the loads of a thread are issued in
-    // batches (the launch has 512 threads), so their latencies overlap
-    {
-        constexpr int NT = 512, ITER = (CT_NF * S3 + NT - 1) / NT, BATCH = 13;
-#pragma unroll
-        for (int b0 = 0; b0 < ITER; b0 += BATCH) {
-            float v[BATCH];
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
-                const int idx = lt + (b0 + u) * NT;
-                const int c = idx / S3, r = idx - c * S3;
-                const int ax = r / (S * S), ay = (r / S) % S, az = r % S;
-                const bool ok = b0 + u < ITER && idx < nf * S3;
-                const int64_t off = ok ? (f0 + c) * M + ((int64_t)s_w[0][ax] * g.Ny + s_w[1][ay]) * g.Nz + s_w[2][az]
-                                       : 0;
-                v[u] = grid[off];
-            }
-#pragma unroll
-            for (int u = 0; u < BATCH; ++u) {
-                const int idx = lt + (b0 + u) * NT;
-                if (b0 + u < ITER && idx < nf * S3) s_g[idx] = v[u];
-            }
+        return v - ((v >= n) ? n : 0);
+    };
+    // Wave 0 finds and stages the tile's particles (three dependent loads: column bounds, index,
+    // position) while the other waves load the grid block, every load of a thread in flight at once.
+    const bool scout = lt < 64;
+    int run_n = 0;
+    if (scout) {
+        if (lt < nruns) {
+            const int x = x0 + lt / ncy, y = y0 + lt % ncy;
+            const int cb = (x * g.Ny + y) * g.Nz;
+            const int b0 = ostart[cb + z0];
+            run_n = ostart[cb + z1] - b0;
+            s_run_beg[lt] = b0;
         }
     }
-    if (lt == 0) {
-        s_run_off[0] = 0;
-        for (int q = 0; q < ncx * ncy; ++q) s_run_off[q + 1] += s_run_off[q];
-    }
-    __syncthreads();
-    const int nruns = ncx * ncy;
-    const int total = s_run_off[nruns];
-    const int wv = lt >> 6, lane = lt & 63, nw = blockDim.x >> 6;
-    // fields XX XY XZ YZ YY YX ZX ZY (grid order 3..10) -> slots {XX, YX, ZX, ZY, YY, XY, XZ, YZ}
-    constexpr int slot_of[11] = {0, 1, 2, 3, 8, 9, 10, 7, 4, 5, 6};
     // olist entry of the tile's q-th particle (runs are the tile's (x, y) cell columns)
     auto entry = [&](int q) {
         int lo = 0, hi = nruns - 1;
@@ -686,10 +692,10 @@ __global__ void __launch_bounds__(512) contract_tile2_kernel(SpreadGeom g, const
         }
         return s_run_beg[lo] + (q - s_run_off[lo]);
     };
-    // the tile's particles staged in LDS by one thread each, so the contraction loop below issues no
-    // global load (a tile with more than CT_PCAP particles reads the rest from global memory): the
-    // index, the stencil origin in the block's local frame (packed bytes) and the offsets
-    // (h o - L/2 - p) of the stencil's first node from the particle, y also without p_y
+    // a staged particle (so the contraction loop below issues no global load; a tile with more than
+    // CT_PCAP particles reads the rest from global memory): the index, the stencil origin in the
+    // block's local frame (packed bytes) and the offsets (h o - L/2 - p) of the stencil's first node
+    // from the particle, y also without p_y
     auto stage = [&](int i, int &bpk, float4 &c) {
         const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
         const float4 p = pos[i];
@@ -700,22 +706,65 @@ __global__ void __launch_bounds__(512) contract_tile2_kernel(SpreadGeom g, const
         const float cy = g.hy * (float)oy - g.Ly2;
         c = make_float4(g.hx * (float)ox - g.Lx2 - p.x, cy, cy - p.y, g.hz * (float)oz - g.Lz2 - p.z);
     };
-    const int nst = min(total, CT_PCAP);
-    if (lt < nst) {
-        const int i = olist[entry(lt)];
-        int bpk;
-        float4 c;
-        stage(i, bpk, c);
-        s_pi[lt] = i;
-        s_pb[lt] = bpk;
-        s_pc[lt] = c;
+    if (scout) {
+        int inc = run_n;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int v = __shfl_up(inc, o, 64);
+            if (lt >= o) inc += v;
+        }
+        s_run_off[lt + 1] = inc;             // runs past nruns are empty
+        if (lt == 0) s_run_off[0] = 0;
+        const int nst = min(__shfl(inc, 63, 64), CT_PCAP);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        for (int q = lt; q < nst; q += 64) {
+            const int i = olist[entry(q)];
+            int bpk;
+            float4 c;
+            stage(i, bpk, c);
+            s_pi[q] = i;
+            s_pb[q] = bpk;
+            s_pc[q] = c;
+        }
+    } else {
+        // node e of the block: its grid offset serves every field, whose base address is uniform
+        constexpr int PER = (S2 * S + NT - 64 - 1) / (NT - 64);
+        int e[PER], off[PER];
+        float v[PER][CT_NF];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            e[u] = min(lt - 64 + u * (NT - 64), S2 * S - 1);   // past the end: the last node again
+            const int r = e[u] / S, az = e[u] - r * S, ax = r / S, ay = r - ax * S;
+            off[u] = (wrap(x0 + ax, g.Nx) * g.Ny + wrap(y0 + ay, g.Ny)) * g.pz + wrap(z0 + az, g.Nz);
+        }
+#pragma unroll
+        for (int c = 0; c < CT_NF; ++c) {
+            // the second group's sixth field repeats its fifth and is not written out
+            const float *gc = grid + (int64_t)(f0 + min(c, nf - 1)) * M;
+#pragma unroll
+            for (int u = 0; u < PER; ++u) v[u][c] = gc[off[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            float2 *o = reinterpret_cast<float2 *>(s_g + e[u] * CT_NF);
+#pragma unroll
+            for (int c = 0; c < CT_NF; c += 2) o[c / 2] = make_float2(v[u][c], v[u][c + 1]);
+        }
     }
     __syncthreads();
-    // this lane's stencil column (ty, tz) and its offsets
-    const int ty = lane / PP, tz = lane - PP * (lane / PP);
-    const float aty = g.hy * (float)ty, atz = g.hz * (float)tz;
+    const int total = s_run_off[TILE * TILE];
+    // fields XX XY XZ YZ YY YX ZX ZY (grid order 3..10) -> slots {XX, YX, ZX, ZY, YY, XY, XZ, YZ}
+    constexpr int slot_of[11] = {0, 1, 2, 3, 8, 9, 10, 7, 4, 5, 6};
+    // this lane's nodes: z = tz, y = ty0 .. ty0 + 2, every x; lanes 12 to 15 of a particle have none
+    const bool active = lane16 < 2 * PP;
+    const int tz = active ? lane16 % PP : 0, ty0 = active ? lane16 / PP * (PP / 2) : 0;
+    const float atz = g.hz * (float)tz;
     const float gq = __expf(-2.0f * g.expfac * g.hx * g.hx);
-    for (int q = wv; q < total; q += nw) {
+    int slot = 0;
+#pragma unroll
+    for (int f = 0; f < CT_NF; ++f)
+        slot = (lane16 == f) ? (grp ? slot_of[CT_NF + (f < 11 - CT_NF ? f : 0)] : slot_of[f]) : slot;
+    for (int q = lt / RL; q < total; q += NT / RL) {
         int i, bpk;
         float4 c;
         if (q < CT_PCAP) {
@@ -727,46 +776,38 @@ __global__ void __launch_bounds__(512) contract_tile2_kernel(SpreadGeom g, const
             stage(i, bpk, c);
         }
         const int bx = bpk & 0xff, by = (bpk >> 8) & 0xff, bz = bpk >> 16;
+        const float *node = s_g + ((bx * S + by + ty0) * S + bz + tz) * CT_NF;
         float acc[CT_NF];
 #pragma unroll
-        for (int c2 = 0; c2 < CT_NF; ++c2) acc[c2] = 0.f;
-        if (lane < PP * PP) {
-            const float uy = c.y + aty, dy = c.z + aty, dz = c.w + atz;
-            const float dyz = dy * dy + dz * dz;
+        for (int f = 0; f < CT_NF; ++f) acc[f] = 0.f;
+        const float dz = c.w + atz;
+#pragma unroll
+        for (int ty = 0; ty < PP / 2; ++ty) {
+            const float ay = g.hy * (float)(ty0 + ty);
+            const float uy = c.y + ay, dy = c.z + ay;
             const float dx0 = c.x + g.xy * uy;
-            const int rb = (bx * S + by + ty) * S + bz + tz;
             // the weights along x by the fast-Gaussian-gridding recurrence (Greengard and Lee,
             // SIAM Rev. 2004): w(tx + 1) = w(tx) r(tx), r(tx + 1) = r(tx) q with
-            // r(0) = exp(-a hx (2 dx0 + hx)) and q = exp(-2 a hx^2): two exponentials per lane
-            float w = __expf(-g.expfac * (dx0 * dx0 + dyz));
+            // r(0) = exp(-a hx (2 dx0 + hx)) and q = exp(-2 a hx^2)
+            float w = __expf(-g.expfac * (dx0 * dx0 + (dy * dy + dz * dz)));
             float r = __expf(-g.expfac * g.hx * (2.0f * dx0 + g.hx));
 #pragma unroll
             for (int tx = 0; tx < PP; ++tx) {
-                const int ro = rb + tx * S * S;
-#pragma unroll
-                for (int c2 = 0; c2 < CT_NF; ++c2)
-                    if (c2 < nf) acc[c2] += w * s_g[c2 * S3 + ro];
+                const float2 *v = reinterpret_cast<const float2 *>(node + (tx * S2 + ty * S) * CT_NF);
+                const float2 v0 = v[0], v1 = v[1], v2 = v[2];
+                acc[0] += w * v0.x; acc[1] += w * v0.y; acc[2] += w * v1.x;
+                acc[3] += w * v1.y; acc[4] += w * v2.x; acc[5] += w * v2.y;
                 w *= r;
                 r *= gq;
             }
         }
-        // wave sums: rows of 16 by DPP, then the three rows that hold the 36 lanes.  Lane c < nf
-        // writes field c and every other lane writes field 0 again (the same value to the same
-        // address): one store that every lane issues, with no branch around it
-        const int ce = lane < nf ? lane : 0;
         float mine = 0.f;
-        int slot = 0;
 #pragma unroll
         for (int f = 0; f < CT_NF; ++f) {
-            const float r = group_sum<16>(acc[f]);
-            const float t = quadw_prefac *
-                            (__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), 0)) +
-                             __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), 16)) +
-                             __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, r), 32)));
-            mine = (ce == f) ? t : mine;
-            slot = (ce == f) ? (f0 ? slot_of[CT_NF + (f < 11 - CT_NF ? f : 0)] : slot_of[f]) : slot;
+            const float t = group_sum<RL>(active ? acc[f] : 0.f);
+            mine = (lane16 == f) ? t : mine;
         }
-        wave[11 * (int64_t)i + slot] = mine;
+        if (lane16 < nf) wave[11 * (int64_t)i + slot] = quadw_prefac * mine;
     }
 }
 
@@ -930,12 +971,8 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
         const int rc = k_setup_spread(ctx, pos);
         if (rc) return rc;
     }
-    SpreadGeom g;
-    g.Nx = ps.Nx; g.Ny = ps.Ny; g.Nz = ps.Nz; g.P = ps.P; g.tile = ctx->tile;
-    g.tnx = ctx->tiles[0]; g.tny = ctx->tiles[1]; g.tnz = ctx->tiles[2];
-    g.hx = ps.gridh_x; g.hy = ps.gridh_y; g.hz = ps.gridh_z;
-    g.Lx2 = ctx->box.Lx / 2.0f; g.Ly2 = ctx->box.Ly / 2.0f; g.Lz2 = ctx->box.Lz / 2.0f; g.xy = ctx->box.xy;
-    g.prefac = ps.prefac; g.expfac = ps.expfac;
+    const SpreadGeom g = spread_geom(ctx);
+    const int64_t Mp = (int64_t)ps.Nx * ps.Ny * g.pz;   // grid field stride
     hipEvent_t ev;
     prof_begin(ctx, PROF_FFT, &ev);
     if (use_fft_lds(ctx)) {
@@ -957,15 +994,15 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
     const bool tiled = ctx->tune.contract == 0 && ctx->contract_lds;
     if (tiled && ctx->contract_split)
         hipLaunchKernelGGL((contract_tile2_kernel<13, 6>), dim3(2 * ctx->ntiles), dim3(512), ctx->contract_lds,
-                           ctx->stream, g, pos, ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, (int64_t)ctx->M,
+                           ctx->stream, g, pos, ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp,
                            ps.quadW * ps.prefac, ctx->d_wave);
     else if (tiled)
         hipLaunchKernelGGL(contract_tile_kernel, dim3(ctx->ntiles), dim3(512), ctx->contract_lds, ctx->stream, g, pos,
-                           ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, (int64_t)ctx->M,
+                           ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp,
                            ps.quadW * ps.prefac, ctx->d_wave);
     else
         hipLaunchKernelGGL(contract_kernel, dim3(nblk((int64_t)N * 64, 256)), dim3(256), 0, ctx->stream, g, pos,
-                           ctx->d_porig, ctx->d_grid, (int64_t)ctx->M, N, ps.quadW * ps.prefac, ctx->d_wave);
+                           ctx->d_porig, ctx->d_grid, Mp, N, ps.quadW * ps.prefac, ctx->d_wave);
     FSD_HIP(hipGetLastError());
     prof_end(ctx, PROF_CONTRACT, ev);
     return 0;
@@ -980,12 +1017,8 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
     float4 *rec = ctx->d_rec;
     hipLaunchKernelGGL(fc_records_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, gF, N, rec);
     FSD_HIP(hipGetLastError());
-    SpreadGeom g;
-    g.Nx = ps.Nx; g.Ny = ps.Ny; g.Nz = ps.Nz; g.P = ps.P; g.tile = ctx->tile;
-    g.tnx = ctx->tiles[0]; g.tny = ctx->tiles[1]; g.tnz = ctx->tiles[2];
-    g.hx = ps.gridh_x; g.hy = ps.gridh_y; g.hz = ps.gridh_z;
-    g.Lx2 = ctx->box.Lx / 2.0f; g.Ly2 = ctx->box.Ly / 2.0f; g.Lz2 = ctx->box.Lz / 2.0f; g.xy = ctx->box.xy;
-    g.prefac = ps.prefac; g.expfac = ps.expfac;
+    const SpreadGeom g = spread_geom(ctx);
+    const int64_t Mp = (int64_t)ps.Nx * ps.Ny * g.pz;   // grid field stride
     const float *wave = nullptr;
     if (parts & 2) {
         if (!ctx->spread_valid || ctx->spread_pos != (const float *)pos) {
@@ -995,12 +1028,12 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
         hipEvent_t ev;
         prof_begin(ctx, PROF_SPREAD, &ev);
         if (ctx->tile == 8 && ctx->pse.P == 6 && ctx->tune.spread == 0)
-            hipLaunchKernelGGL((spread_tile2_kernel<8, 6>), dim3(ctx->ntiles), dim3(512), 0, ctx->stream, g, pos,
-                               ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid, (int64_t)ctx->M);
+            hipLaunchKernelGGL(spread_mfma_kernel<6>, dim3(ctx->ntiles), dim3(512), 0, ctx->stream, g, pos,
+                               ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp);
         else
             hipLaunchKernelGGL(spread_kernel, dim3(ctx->ntiles), dim3(ctx->tile * ctx->tile * ctx->tile), 0,
                                ctx->stream, g, pos, ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid,
-                               (int64_t)ctx->M);
+                               Mp);
         FSD_HIP(hipGetLastError());
         prof_end(ctx, PROF_SPREAD, ev);
         const bool fx = use_fft_lds(ctx);

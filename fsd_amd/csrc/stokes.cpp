@@ -231,7 +231,7 @@ static int alloc_all(fsd_ctx *ctx)
     const fsd_pse_info &ps = ctx->pse;
     ctx->M = ps.Nx * ps.Ny * ps.Nz;
     ctx->Mh = ps.Nx * ps.Ny * (ps.Nz / 2 + 1);
-    CK(hipMalloc(&ctx->d_grid, sizeof(float) * 11 * (size_t)ctx->M));
+    CK(hipMalloc(&ctx->d_grid, sizeof(float) * 11 * (size_t)ps.Nx * ps.Ny * ((ps.Nz + 3) / 4 * 4)));
     CK(hipMalloc(&ctx->d_spec, sizeof(float2) * 11 * (size_t)ctx->Mh));
     CK(hipMalloc(&ctx->d_gridk, sizeof(float4) * (size_t)ctx->Mh));
     ctx->tile = 8;
