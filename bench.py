@@ -48,8 +48,8 @@ GUESS_TEXT = {"previous": "previous solution", "extrapolate": "linear extrapolat
 # kernel-class name -> kernel name in rocprofv3 traces
 KERNEL_NAMES = {"spread": "spread_mfma_kernel<6>", "green": "x_green_kernel<4, 256, true>", "contract": "contract_tile2_kernel<13, 6>",
                 "realspace": "realspace_kernel<16>", "rfu": "rfu_apply_kernel<8>", "sweep": "tp_sweep1_kernel",
-                "ichol": "ichol_level_kernel", "gmres_vec": "multidot_partial4_kernel", "ljit": "lj_fwd_kernel",
-                "jacobi": "jac_fwd_kernel"}
+                "ichol": "ichol_level_kernel", "gmres_vec": "multidot_partial4_kernel", "ljit": "bj_iter_kernel<false>",
+                "jacobi": "bj_iter_kernel<false>"}
 
 
 def algorithmic_bytes(cls, N, info, pse, st, kbar=25.5, gs_passes=2):
@@ -75,14 +75,10 @@ def algorithmic_bytes(cls, N, info, pse, st, kbar=25.5, gs_passes=2):
         # Z d (b_F, b_U in 48 B, Z 144 B, out 24 B), reorder (48 B), Z^T u and the combination
         # (Z 144 B, u 24 B, b_F and b_S 44 B in, x_F, x_S, x_U 68 B out) per particle
         return 2 * (144 * st["lower_blocks"] + 48 * N) + (48 + 144 + 24 + 48 + 144 + 24 + 44 + 68) * N
-    if cls == "ljit":        # one block Jacobi iteration of the learned factor: every pair block W (144 B) and
-        # inverse pivot (144 B) once, the fixed right-hand side (t or v_k) and the previous iterate in, the
-        # new iterate out (24 B each per particle)
-        return 144 * (st["lower_blocks"] + N) + 3 * 24 * N
-    if cls == "jacobi":      # one block Jacobi iteration on the IC(0) factor: every folded block Z_P L_PQ
-        # (144 B) and its column index (4 B) once, the fixed right-hand side and the previous iterate in,
-        # the new iterate out (24 B each per particle), the row offsets (4 B)
-        return 148 * st["lower_blocks"] + (3 * 24 + 4) * N
+    if cls in ("ljit", "jacobi"):   # one block Jacobi iteration on the folded factor: every block (144 B)
+        # once, the fixed right-hand side and the previous iterate in, the new iterate out (24 B each per
+        # particle), the first columns (16 B) and row offsets (4 B)
+        return 144 * st["lower_blocks"] + (3 * 24 + 20) * N
     if cls == "ichol":       # one factorisation: A blocks in, L blocks out (lower and diagonal)
         return 144 * 2 * (st["lower_blocks"] + N)
     if cls == "gmres_vec":   # Gram-Schmidt of a 17N-float vector on k basis vectors, per pass h = V^T w

@@ -306,8 +306,8 @@ struct fsd_ctx {
     int precond_mode = 0;                                // 0: exact sweeps, 1: IC(0) + Jacobi, 2: learned + Jacobi
     int jac_k = 0;                                       // Jacobi iterations per triangular solve
     int ic_jac_k = 0;                                    // the same for IC(0) (modes 1 and 2); 0: exact solves
-    float *d_Fblk = nullptr;                             // 36 per lower block: Z_P L_PQ
-    int *d_lrowidx = nullptr;                            // row P of every lower block
+    float *d_Fblk = nullptr, *d_Tblk = nullptr;          // 36 per lower / upper block: folded factor (k_jacobi.hip)
+    int4 *d_lell = nullptr, *d_uell = nullptr;           // first four columns of every lower / upper row
     float *d_jac = nullptr;                              // 4 x 6N iterates
     float *d_Lblk2 = nullptr, *d_Ldiag2 = nullptr;       // second factor buffer of the parallel IC(0) sweeps
     // learned factor (precond mode 2, learned.h) and its fallbacks to IC(0)
@@ -453,7 +453,12 @@ int k_scale_by_norm(fsd_ctx *ctx, int64_t n, float *v, const double *h, int K, d
 int k_saddle_precond(fsd_ctx *ctx, const float *b, float *x);
 // the factor's application by Jacobi iterations (k_jacobi.hip)
 int k_diag_inverse(fsd_ctx *ctx);
+int k_jacobi_init(fsd_ctx *ctx);
+int k_jacobi_ell(fsd_ctx *ctx);
 int k_jacobi_pack(fsd_ctx *ctx);
+int k_jacobi_pack_ldl(fsd_ctx *ctx, const float *W, const float *Dinv);
+int k_bj_apply(fsd_ctx *ctx, int k, int prof_slot, const float *R, const float *Zpost, const float *b0,
+               const float *b1, const float *bsaddle, float *x, int mode);
 int k_saddle_precond_jacobi(fsd_ctx *ctx, const float *b, float *x);
 int k_precond_apply_jacobi(fsd_ctx *ctx, const float *b, float *y);
 int k_saddle_multiply(fsd_ctx *ctx, const float4 *pos, const float *x, float *y);

@@ -461,6 +461,8 @@ __global__ void lp_node_D_kernel(int N, const int *lrow, const int *lcol, const 
 }
 
 // --------------------------------------------------- block Jacobi application
+// The iterations of the training loss, which keep every iterate for the reverse sweep (a solve's
+// applications run on the folded blocks, k_jacobi.hip).
 // v_0 = Dinv t with t = (b0 - b1)[perm P]; t is stored when tout != null
 __global__ void lj_pre_kernel(int N, const int *perm, const float *Dinv, const float *b0, const float *b1, float *tout,
                               float *vout)
@@ -512,30 +514,10 @@ __global__ void __launch_bounds__(256) lj_fwd_kernel(int N, const int *lrow, con
     vout[6 * (int64_t)P + a] = v;
 }
 
-// the preconditioner's output of a row's value g (unpermuted): mode 0: out = g (6N);
-// mode 1: the saddle preconditioner's combination x_F = b_F - g, x_S = b_S, x_U = g
-// (Saddle.cu:171-264 with g = G (b_F - b_U))
-__device__ __forceinline__ void lj_post_write(int N, int P, int a, const int *perm, float g, const float *b, float *out,
-                                              int mode)
-{
-    const int64_t i = perm[P], n6 = 6 * (int64_t)N, n11 = 11 * (int64_t)N;
-    if (mode == 0) {
-        out[6 * i + a] = g;
-        return;
-    }
-    out[6 * i + a] = b[6 * i + a] - g;
-    out[n11 + 6 * i + a] = g;
-    if (a < 5) out[n6 + 5 * i + a] = b[n6 + 5 * i + a];
-}
-
-// backward iteration: s = W^T x_in (stored when sout != null), x_out = v_k - Dinv s; the last
-// iteration of an application also writes the preconditioner's output (post_mode 0 or 1,
-// lj_post_write; -1: none)
+// backward iteration: s = W^T x_in (stored when sout != null), x_out = v_k - Dinv s
 __global__ void __launch_bounds__(256) lj_bwd_kernel(int N, const int *urow, const int *ucol, const int *upos,
                                                      const float *W, const float *Dinv, const float *vk,
-                                                     const float *xin, float *sout, float *xout,
-                                                     const int *perm = nullptr, const float *bpost = nullptr,
-                                                     float *outpost = nullptr, int post_mode = -1)
+                                                     const float *xin, float *sout, float *xout)
 {
     int P, a;
     const bool ok = row_lane(N, P, a);
@@ -556,18 +538,7 @@ __global__ void __launch_bounds__(256) lj_bwd_kernel(int N, const int *urow, con
 #pragma unroll
     for (int c = 0; c < 6; ++c) q += Dp[c] * s6[c];
     if (sout) sout[6 * (int64_t)P + a] = s;
-    const float x = vk[6 * (int64_t)P + a] - q;
-    xout[6 * (int64_t)P + a] = x;
-    if (post_mode >= 0) lj_post_write(N, P, a, perm, x, bpost, outpost, post_mode);
-}
-
-// g = x unpermuted; mode 0: out = g (6N); mode 1: the saddle preconditioner's
-// combination x_F = b_F - g, x_S = b_S, x_U = g (Saddle.cu:171-264 with g = G (b_F - b_U))
-__global__ void lj_post_kernel(int N, const int *perm, const float *x, const float *b, float *out, int mode)
-{
-    int P, a;
-    if (!row_lane(N, P, a)) return;
-    lj_post_write(N, P, a, perm, x[6 * (int64_t)P + a], b, out, mode);
+    xout[6 * (int64_t)P + a] = vk[6 * (int64_t)P + a] - q;
 }
 
 // ---------------------------------------------------- training loss, adjoint
@@ -1440,6 +1411,8 @@ int lp_forward(fsd_ctx *ctx, const float4 *pos, bool train, int inject, int *fai
     if (E)   // the pair blocks' one-step fill correction with the final pivots
         hipLaunchKernelGGL(lp_wfix_kernel, dim3(nblk(E, 128)), dim3(128), 0, ctx->stream, E, s.erow, ctx->d_lcol,
                            ctx->d_lrow, ctx->d_Ablk, s.Dinv, s.W);
+    // the blocks that lp_apply's iterations read
+    LRC(k_jacobi_pack_ldl(ctx, s.W, s.Dinv));
     FSD_HIP(hipGetLastError());
     prof_end(ctx, PROF_NET, pev);
     FSD_HIP(hipMemcpyAsync(s.h_fail, s.d_fail, sizeof(int) * 3, hipMemcpyDeviceToHost, ctx->stream));
@@ -1454,39 +1427,7 @@ int lp_forward(fsd_ctx *ctx, const float4 *pos, bool train, int inject, int *fai
 // the saddle preconditioner of b0 (17N) with G (b_F - b_U)
 int lp_apply(fsd_ctx *ctx, const float *b0, const float *b1, const float *bsaddle, float *x, int mode)
 {
-    LearnedState &s = *ctx->lp;
-    const int N = ctx->N, k = ctx->jac_k;
-    hipEvent_t ev;
-    prof_begin(ctx, PROF_TRSV, &ev);
-    const dim3 g(row_blocks(N)), b(256);
-    float *t = ctx->d_jac, *v[2] = {ctx->d_jac + 6 * (int64_t)N, ctx->d_jac + 12 * (int64_t)N};
-    float *xb[2] = {ctx->d_jac + 18 * (int64_t)N, ctx->d_jac + 12 * (int64_t)N};
-    hipLaunchKernelGGL(lj_pre_kernel, g, b, 0, ctx->stream, N, ctx->d_perm, s.Dinv, b0, b1, t, v[0]);
-    int cur = 0;
-    hipEvent_t e1;
-    prof_begin(ctx, PROF_LJIT, &e1);   // the k forward iterations, one event pair
-    for (int it = 0; it < k; ++it) {
-        hipLaunchKernelGGL(lj_fwd_kernel, g, b, 0, ctx->stream, N, ctx->d_lrow, ctx->d_lcol, s.W, s.Dinv, t, v[cur],
-                           (float *)nullptr, v[cur ^ 1]);
-        cur ^= 1;
-    }
-    prof_end_n(ctx, PROF_LJIT, e1, k);
-    const float *vk = v[cur];
-    // backward iterates alternate between the two buffers vk does not occupy
-    float *bo[2] = {xb[0], (vk == v[0]) ? v[1] : v[0]};
-    const float *xc = vk;
-    for (int it = 0; it < k; ++it) {   // the last iteration writes the preconditioner's output as well
-        float *out = bo[it & 1];
-        const bool last = it == k - 1;
-        hipLaunchKernelGGL(lj_bwd_kernel, g, b, 0, ctx->stream, N, ctx->d_urow, ctx->d_ucol, ctx->d_upos, s.W, s.Dinv,
-                           vk, xc, (float *)nullptr, out, last ? ctx->d_perm : (const int *)nullptr,
-                           last ? bsaddle : (const float *)nullptr, last ? x : (float *)nullptr, last ? mode : -1);
-        xc = out;
-    }
-    if (k == 0) hipLaunchKernelGGL(lj_post_kernel, g, b, 0, ctx->stream, N, ctx->d_perm, xc, bsaddle, x, mode);
-    FSD_HIP(hipGetLastError());
-    prof_end(ctx, PROF_TRSV, ev);
-    return 0;
+    return k_bj_apply(ctx, ctx->jac_k, PROF_LJIT, ctx->lp->Dinv, nullptr, b0, b1, bsaddle, x, mode);
 }
 
 // Backward of the factor assembly and the network: from gW (pair blocks) and gDinv

@@ -287,8 +287,9 @@ static int alloc_all(fsd_ctx *ctx)
     CK(hipMalloc(&ctx->d_Ablk, sizeof(float) * 36 * ctx->nlow_cap));
     CK(hipMalloc(&ctx->d_Lblk, sizeof(float) * 36 * ctx->nlow_cap));
     if (ctx->precond_mode != 0) {
-        CK(hipMalloc(&ctx->d_Fblk, sizeof(float) * 36 * ctx->nlow_cap));
-        CK(hipMalloc(&ctx->d_lrowidx, sizeof(int) * ctx->nlow_cap));
+        RC(k_jacobi_init(ctx));
+        for (float **pp : {&ctx->d_Fblk, &ctx->d_Tblk}) CK(hipMalloc(pp, sizeof(float) * 36 * ctx->nlow_cap));
+        for (int4 **pp : {&ctx->d_lell, &ctx->d_uell}) CK(hipMalloc(pp, sizeof(int4) * (size_t)N));
         CK(hipMalloc(&ctx->d_jac, sizeof(float) * 24 * (size_t)N));
     }
     if (ctx->p.factor_sweeps > 0) CK(hipMalloc(&ctx->d_Lblk2, sizeof(float) * 36 * ctx->nlow_cap));
@@ -362,7 +363,7 @@ static void free_all(fsd_ctx *ctx)
                     ctx->d_force, ctx->d_mask1, ctx->d_mask2, ctx->d_tp_finfo, ctx->d_tp_binfo,
                     ctx->d_tp_fbsrc, ctx->d_tp_bbsrc, ctx->d_tp_fblk, ctx->d_tp_bblk,
                     ctx->d_tp_finp, ctx->d_tp_binp, ctx->d_tp_fres, ctx->d_tp_bres, ctx->d_tp_fseq, ctx->d_tp_bseq, ctx->d_tp_fplace, ctx->d_tp_bplace,
-                    ctx->d_tp_Z, ctx->d_Fblk, ctx->d_lrowidx, ctx->d_jac, ctx->d_Lblk2, ctx->d_Ldiag2,
+                    ctx->d_tp_Z, ctx->d_Fblk, ctx->d_Tblk, ctx->d_lell, ctx->d_uell, ctx->d_jac, ctx->d_Lblk2, ctx->d_Ldiag2,
                     ctx->d_x64, ctx->d_r64, ctx->d_ybot64, ctx->d_norm64, ctx->d_refx32, ctx->d_refy32,
                     ctx->d_refr32, ctx->d_refd,
                     ctx->d_Z, ctx->d_lanV, ctx->d_lanw, ctx->d_lany0, ctx->d_lan_h, ctx->d_noise, ctx->d_posp,
@@ -393,10 +394,10 @@ static int grow_lower(fsd_ctx *ctx, int64_t need)
     for (int **pp : {&ctx->d_lcol, &ctx->d_ucol, &ctx->d_upos}) CK(hipMalloc(pp, sizeof(int) * cap));
     for (float **pp : {&ctx->d_Ablk, &ctx->d_Lblk}) CK(hipMalloc(pp, sizeof(float) * 36 * cap));
     if (ctx->d_Fblk) {
-        hipFree(ctx->d_Fblk);
-        hipFree(ctx->d_lrowidx);
-        CK(hipMalloc(&ctx->d_Fblk, sizeof(float) * 36 * cap));
-        CK(hipMalloc(&ctx->d_lrowidx, sizeof(int) * cap));
+        for (float **pp : {&ctx->d_Fblk, &ctx->d_Tblk}) {
+            hipFree(*pp);
+            CK(hipMalloc(pp, sizeof(float) * 36 * cap));
+        }
     }
     if (ctx->d_Lblk2) {
         hipFree(ctx->d_Lblk2);
@@ -496,6 +497,7 @@ static int precond_upload_blocks(fsd_ctx *ctx, const float4 *pos)
         CK(up(ctx->d_ucol, h.ucol.data(), sizeof(int) * ctx->pch.nlow));
         CK(up(ctx->d_upos, h.upos.data(), sizeof(int) * ctx->pch.nlow));
     }
+    if (ctx->precond_mode != 0) RC(k_jacobi_ell(ctx));
     RC(k_build_blocks(ctx, pos));
     return 0;
 }
