@@ -222,6 +222,8 @@ struct fsd_ctx {
     // neighbour list
     int maxn = 0;
     int *d_nneigh = nullptr, *d_nlist = nullptr;
+    // the same lists by slot, the particle's place in d_cell_list (with cells only): the neighbours' slots
+    int *d_snn = nullptr, *d_nslot = nullptr;
     int ncell[3] = {0, 0, 0}; int ncells = 0; bool use_cells = false;
     int *d_cell_of = nullptr, *d_cell_count = nullptr, *d_cell_start = nullptr, *d_cell_list = nullptr;
     int *d_flags = nullptr;     // [0] nlist overflow, [2] prune overflow, [4] nlist entries, [8] lub overflow,
@@ -255,16 +257,18 @@ struct fsd_ctx {
     rocfft_execution_info info_fwd = nullptr, info_inv = nullptr;
     void *d_fftwork = nullptr; size_t fftwork_size = 0;
     int tiles[3] = {0, 0, 0}; int ntiles = 0; int tile = 8;
-    int *d_porig = nullptr;       // 3 ints per particle: stencil origin (unwrapped)
-    int *d_ocell = nullptr;       // N: grid cell of each particle's (wrapped) stencil origin
-    int *d_olist = nullptr;       // N: particles sorted by origin cell, ascending id inside a cell
+    // set-up of the wave part, particles by slot (cell order of the neighbour list; identity without one)
+    float4 *d_spos = nullptr;     // N: position, w the particle's index (bits)
+    int *d_porig = nullptr;       // 3 ints per slot: stencil origin (unwrapped)
+    int *d_ocell = nullptr;       // N: grid cell of each slot's (wrapped) stencil origin
+    int *d_olist = nullptr;       // N: slots sorted by origin cell, ascending inside a cell
     int *d_ocount = nullptr;      // M: particles per origin cell (scratch)
     int *d_ostart = nullptr;      // M+1: first position of each origin cell in d_olist
     int *d_scan_tmp = nullptr;    // chunk totals of the multi-workgroup scan
     int contract_lds = 0;         // LDS bytes of the tile contraction (0: per-particle contraction)
     bool contract_split = false;  // the two-workgroup-per-tile contraction (P = 6, tile 8)
     float *d_wave = nullptr;      // 11 per particle: wave-space u (3) and gradient (8)
-    float4 *d_rec = nullptr;      // 3 per particle: force + couplet records of the current apply
+    float4 *d_rec = nullptr;      // 4 per slot: position, force and couplet records of the current apply
     bool spread_valid = false;
     const float *spread_pos = nullptr;
 
@@ -404,6 +408,7 @@ int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S);
 int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S);
 int k_setup_spread(fsd_ctx *ctx, const float4 *pos);
 int k_contract_lds(fsd_ctx *ctx);
+int k_real_init(fsd_ctx *ctx);       // LDS limits of the real-space kernels; nonzero on failure
 int scan_excl_chunks(int n);
 int k_gridk(fsd_ctx *ctx);
 float k_twopi(const fsd_ctx *ctx);

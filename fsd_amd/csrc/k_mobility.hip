@@ -7,6 +7,8 @@
 //                epilogue that adds the wave-space result, converts the velocity
 //                gradient to (W, E) and writes the generalised velocity.
 // Restates Mobility.cu:131-1542 and Helper_Mobility.cu:88-410.
+#include <algorithm>
+
 #include "fsd_internal.h"
 #include "green.h"
 
@@ -45,14 +47,19 @@ int k_gridk(fsd_ctx *ctx)
 // ------------------------------------------------- spreading set-up (per step)
 // Stencil origin exactly as Mobility.cu:203-225 (float fraction, truncation);
 // particles are then counting-sorted by the grid cell of their (wrapped)
-// origin, ascending particle id inside a cell, so spreading and contraction
+// origin, ascending inside a cell, so spreading and contraction
 // can find the particles of any block of origin cells as contiguous runs.
-__global__ void stencil_origin_kernel(const float4 *pos, int N, BoxF b, int Nx, int Ny, int Nz, int P, int *orig,
-                                      int *ocell, int *ocount)
+//
+// Particles stand by slot, their place in the neighbour list's cell order: what the wave part and
+// the real-space sum read of a particle's surroundings lies close together.
+__global__ void stencil_origin_kernel(const float4 *pos, const int *order, int N, BoxF b, int Nx, int Ny, int Nz,
+                                      int P, float4 *spos, int *orig, int *ocell, int *ocount)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
-    float4 p = pos[i];
+    const int id = order ? order[i] : i;
+    float4 p = pos[id];
+    spos[i] = make_float4(p.x, p.y, p.z, __int_as_float(id));
     float fx, fy, fz;
     box_make_fraction(b, p.x, p.y, p.z, fx, fy, fz);
     fx *= (float)Nx; fy *= (float)Ny; fz *= (float)Nz;
@@ -90,12 +97,18 @@ __global__ void ocell_sort_kernel(const int *start, int ncell, int *list)
 
 int scan_excl_large(fsd_ctx *ctx, const int *in, int *out, int n, int *tmp);
 
+// the order of the slots
+static const int *slot_order(const fsd_ctx *ctx)
+{
+    return (ctx->nlist_valid && ctx->use_cells) ? ctx->d_cell_list : nullptr;
+}
+
 int k_setup_spread(fsd_ctx *ctx, const float4 *pos)
 {
     const int N = ctx->N, M = ctx->M;
     FSD_HIP(hipMemsetAsync(ctx->d_ocount, 0, sizeof(int) * M, ctx->stream));
-    hipLaunchKernelGGL(stencil_origin_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, pos, N, ctx->box,
-                       ctx->pse.Nx, ctx->pse.Ny, ctx->pse.Nz, ctx->pse.P, ctx->d_porig, ctx->d_ocell, ctx->d_ocount);
+    hipLaunchKernelGGL(stencil_origin_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, pos,
+                       slot_order(ctx), N, ctx->box, ctx->pse.Nx, ctx->pse.Ny, ctx->pse.Nz, ctx->pse.P, ctx->d_spos, ctx->d_porig, ctx->d_ocell, ctx->d_ocount);
     if (scan_excl_large(ctx, ctx->d_ocount, ctx->d_ostart, M, ctx->d_scan_tmp)) return FSD_E_HIP;
     FSD_HIP(hipMemsetAsync(ctx->d_ocount, 0, sizeof(int) * M, ctx->stream));
     hipLaunchKernelGGL(ocell_scatter_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, ctx->d_ocell, N,
@@ -109,21 +122,30 @@ int k_setup_spread(fsd_ctx *ctx, const float4 *pos)
 }
 
 // ------------------------------------------------- force + couplet records
-// per particle: F (3) and the 8 stored couplet components (Mobility_TS2C_kernel,
-// Helper_Mobility.cu:294-336) packed as 3 float4
-__global__ void fc_records_kernel(const float *gF, int N, float4 *rec)
+// per slot one 64-byte record (half a cache line): position, F (3), the stresslet S (xx, xy, xz, yz, yy)
+// and w = -T/2, the couplet's antisymmetric part (Mobility_TS2C_kernel, Helper_Mobility.cu:294-336)
+__global__ void fc_records_kernel(const float *gF, const float4 *pos, const int *order, int N, float4 *rec)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
-    const float *f = gF + 6 * (int64_t)i;
-    const float *s = gF + 6 * (int64_t)N + 5 * (int64_t)i;
-    float Lx = -f[3], Ly = -f[4], Lz = -f[5];
-    float Sxx = s[0], Sxy = s[1], Sxz = s[2], Syz = s[3], Syy = s[4];
-    float C0 = Sxx, C1 = Sxy + 0.5f * Lz, C2 = Sxz - 0.5f * Ly, C3 = Syz + 0.5f * Lx;
-    float C4 = Syy, C5 = Sxy - 0.5f * Lz, C6 = Sxz + 0.5f * Ly, C7 = Syz - 0.5f * Lx;
-    rec[3 * (int64_t)i] = make_float4(f[0], f[1], f[2], C0);
-    rec[3 * (int64_t)i + 1] = make_float4(C1, C2, C3, C4);
-    rec[3 * (int64_t)i + 2] = make_float4(C5, C6, C7, 0.f);
+    const int id = order ? order[i] : i;
+    const float *f = gF + 6 * (int64_t)id;
+    const float *s = gF + 6 * (int64_t)N + 5 * (int64_t)id;
+    const float4 p = pos[id];
+    float4 *r = rec + 4 * (int64_t)i;
+    r[0] = make_float4(p.x, p.y, p.z, f[0]);
+    r[1] = make_float4(f[1], f[2], s[0], s[1]);
+    r[2] = make_float4(s[2], s[3], s[4], -0.5f * f[3]);
+    r[3] = make_float4(-0.5f * f[4], -0.5f * f[5], 0.f, 0.f);
+}
+
+// F and the couplet's stored components XX XY XZ YZ YY YX ZX ZY of a record: the 11 grid fields
+__device__ __forceinline__ void record_fields(const float4 q[4], float4 f[3])
+{
+    const float sxy = q[1].w, sxz = q[2].x, syz = q[2].y, wx = q[2].w, wy = q[3].x, wz = q[3].y;
+    f[0] = make_float4(q[0].w, q[1].x, q[1].y, q[1].z);
+    f[1] = make_float4(sxy + wz, sxz - wy, syz + wx, q[2].z);
+    f[2] = make_float4(sxy - wz, sxz + wy, syz - wx, 0.f);
 }
 
 // ------------------------------------------------------------ spreading
@@ -169,9 +191,8 @@ __device__ int halo_axis(int t0, int tile, int P, int n, int *list)
 // accumulates its 11 fields in registers and is written once (no atomics).
 #define SP_CH 256
 #define SP_MAXAX 32
-__global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const float4 *pos, const int *orig,
-                                                     const float4 *rec, const int *ostart, const int *olist,
-                                                     float *grid, int64_t M)
+__global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const int *orig, const float4 *rec, const int *ostart,
+                                                     const int *olist, float *grid, int64_t M)
 {
     __shared__ int s_ax[3][SP_MAXAX];
     __shared__ int s_nax[3];
@@ -243,9 +264,11 @@ __global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const float4 
             }
             const int i = olist[s_seg_beg[lo] + (q - s_seg_off[lo])];
             s_o[lt][0] = orig[3 * i]; s_o[lt][1] = orig[3 * i + 1]; s_o[lt][2] = orig[3 * i + 2];
-            const float4 p = pos[i];
-            s_p[lt][0] = p.x; s_p[lt][1] = p.y; s_p[lt][2] = p.z;
-            s_r[lt][0] = rec[3 * (int64_t)i]; s_r[lt][1] = rec[3 * (int64_t)i + 1]; s_r[lt][2] = rec[3 * (int64_t)i + 2];
+            float4 r[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) r[k] = rec[4 * (int64_t)i + k];
+            s_p[lt][0] = r[0].x; s_p[lt][1] = r[0].y; s_p[lt][2] = r[0].z;
+            record_fields(r, s_r[lt]);
         }
         __syncthreads();
         if (inside) {
@@ -296,9 +319,8 @@ __global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const float4 
 #define SP2_CAP 256
 typedef float mfma_f4 __attribute__((ext_vector_type(4)));
 template <int PP>
-__global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const float4 *pos, const int *orig,
-                                                             const float4 *rec, const int *ostart, const int *olist,
-                                                             float *grid, int64_t M)
+__global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const int *orig, const float4 *rec,
+                                                             const int *ostart, const int *olist, float *grid, int64_t M)
 {
     constexpr int T = 8, BL = 4, H = T + PP - 1, HB = BL + PP - 1, NT = 512, NW = NT / 64;
     constexpr int ZP[4] = {0, H - HB, HB, H};     // thirds of the halo's z cells: 4, 5 and 4 of them
@@ -310,7 +332,7 @@ __global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const
     __shared__ int s_wsum[NW];
     __shared__ float4 s_c[SP2_CAP];               // scaled offsets of the tile's first column (x, y), its columns
     __shared__ float4 s_z[SP2_CAP][2];            // factors along z
-    __shared__ float s_r[SP2_CAP * 12 + 4];       // records; rows 12 to 15 of a product read past a sphere's 12
+    __shared__ float s_r[SP2_CAP * 12 + 4];       // fields; rows 12 to 15 of a product read past a sphere's 12
     __shared__ unsigned short s_list[NW][SP2_CAP + 8];
 
     const int tile_id = xcd_remap(blockIdx.x, gridDim.x);
@@ -389,8 +411,10 @@ __global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const
             const bool second = o >= n1;
             const int i = olist[second ? s_beg[1][lo] + (o - n1) : s_beg[0][lo] + o];
             const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
-            const float4 q = pos[i];
-            const float4 r0 = rec[3 * (int64_t)i], r1 = rec[3 * (int64_t)i + 1], r2 = rec[3 * (int64_t)i + 2];
+            float4 r[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) r[k] = rec[4 * (int64_t)i + k];
+            const float4 q = r[0];
             // the sphere's origin is the halo cell (hc) up to the period, so a node at local (lx, ly, lz)
             // of its stencil is node o + (P - 1) - hc + l: with the node's position
             // h (o + P - 1 - hc) - L/2 + h l, its offset from the sphere is c + h l
@@ -415,10 +439,7 @@ __global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const
             s_c[lt] = make_float4(unit * cx, unit * (cy - q.y), __uint_as_float(mx | (my << T)), 0.f);
             s_z[lt][0] = make_float4(w[0], w[1], w[2], w[3]);
             s_z[lt][1] = make_float4(w[4], w[5], w[6], w[7]);
-            float4 *r = reinterpret_cast<float4 *>(s_r + 12 * lt);
-            r[0] = r0;
-            r[1] = r1;
-            r[2] = r2;
+            record_fields(r, reinterpret_cast<float4 *>(s_r + 12 * lt));
         }
         // this wave's spheres of the part: lane k < 18 lists run k
         unsigned short *list = s_list[wv];
@@ -499,7 +520,7 @@ __global__ void green_kernel(float2 *spec, const float4 *gk, int64_t Mh, GreenGe
 // Mobility_WaveSpace_ContractU/D (Mobility.cu:503-841): one wavefront per
 // particle, lanes over the (y, z) stencil pairs, loop over x.  Output per
 // particle: u (3) then the gradient in the reference's transposed slots.
-__global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float4 *pos, const int *orig,
+__global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float4 *spos, const int *orig,
                                                        const float *grid, int64_t M, int N, float quadw_prefac,
                                                        float *wave)
 {
@@ -508,7 +529,7 @@ __global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float
     if (wave_id >= N) return;
     const int i = wave_id;
     const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
-    const float4 p = pos[i];
+    const float4 p = spos[i];
     float acc[11];
 #pragma unroll
     for (int c = 0; c < 11; ++c) acc[c] = 0.f;
@@ -534,7 +555,7 @@ __global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float
     for (int c = 0; c < 11; ++c)
         for (int o = 32; o > 0; o >>= 1) acc[c] += __shfl_xor(acc[c], o, 64);
     if (lane == 0) {
-        float *w = wave + 11 * (int64_t)i;
+        float *w = wave + 11 * (int64_t)__float_as_int(p.w);
         w[0] = acc[0]; w[1] = acc[1]; w[2] = acc[2];
         // fields XX XY XZ YZ YY YX ZX ZY -> slots {XX, YX, ZX, ZY, YY, XY, XZ, YZ}
         w[3] = acc[3]; w[4] = acc[8]; w[5] = acc[9]; w[6] = acc[10];
@@ -548,7 +569,7 @@ __global__ void __launch_bounds__(256) contract_kernel(SpreadGeom g, const float
 // origin lies in the tile, one wavefront per particle, from LDS.  Requires
 // 11 (TILE + P - 1)^3 floats of LDS (TILE 8, P 6: 96.7 KB).
 #define CT_S 13
-__global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const float4 *pos, const int *orig,
+__global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const float4 *spos, const int *orig,
                                                             const int *ostart, const int *olist, const float *grid,
                                                             int64_t M, float quadw_prefac, float *wave)
 {
@@ -598,7 +619,7 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
         }
         const int i = olist[s_run_beg[lo] + (q - s_run_off[lo])];
         const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
-        const float4 p = pos[i];
+        const float4 p = spos[i];
         // local block coordinates of the stencil's first node (wrapped origin - tile start)
         const int bx = (((ox % g.Nx) + g.Nx) % g.Nx) - x0;
         const int by = (((oy % g.Ny) + g.Ny) % g.Ny) - y0;
@@ -623,7 +644,7 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
         for (int c = 0; c < 11; ++c)
             for (int o = 32; o > 0; o >>= 1) acc[c] += __shfl_xor(acc[c], o, 64);
         if (lane == 0) {
-            float *w = wave + 11 * (int64_t)i;
+            float *w = wave + 11 * (int64_t)__float_as_int(p.w);
             w[0] = acc[0]; w[1] = acc[1]; w[2] = acc[2];
             // fields XX XY XZ YZ YY YX ZX ZY -> slots {XX, YX, ZX, ZY, YY, XY, XZ, YZ}
             w[3] = acc[3]; w[4] = acc[8]; w[5] = acc[9]; w[6] = acc[10];
@@ -648,7 +669,7 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
 #define CT_NF 6
 #define CT_PCAP 128   // particles of a tile staged in LDS (about 45 in an 8^3 tile at volume fraction 0.45)
 template <int S, int PP>
-__global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, const float4 *pos, const int *orig,
+__global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, const float4 *spos, const int *orig,
                                                              const int *ostart, const int *olist, const float *grid,
                                                              int64_t M, float quadw_prefac, float *wave)
 {
@@ -696,9 +717,10 @@ __global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, co
     // CT_PCAP particles reads the rest from global memory): the index, the stencil origin in the
     // block's local frame (packed bytes) and the offsets (h o - L/2 - p) of the stencil's first node
     // from the particle, y also without p_y
-    auto stage = [&](int i, int &bpk, float4 &c) {
+    auto stage = [&](int i, int &id, int &bpk, float4 &c) {
         const int ox = orig[3 * i], oy = orig[3 * i + 1], oz = orig[3 * i + 2];
-        const float4 p = pos[i];
+        const float4 p = spos[i];
+        id = __float_as_int(p.w);
         const int bx = (((ox % g.Nx) + g.Nx) % g.Nx) - x0;
         const int by = (((oy % g.Ny) + g.Ny) % g.Ny) - y0;
         const int bz = (((oz % g.Nz) + g.Nz) % g.Nz) - z0;
@@ -718,11 +740,10 @@ __global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, co
         const int nst = min(__shfl(inc, 63, 64), CT_PCAP);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         for (int q = lt; q < nst; q += 64) {
-            const int i = olist[entry(q)];
-            int bpk;
+            int id, bpk;
             float4 c;
-            stage(i, bpk, c);
-            s_pi[q] = i;
+            stage(olist[entry(q)], id, bpk, c);
+            s_pi[q] = id;
             s_pb[q] = bpk;
             s_pc[q] = c;
         }
@@ -772,8 +793,7 @@ __global__ void __launch_bounds__(512, 4) contract_tile2_kernel(SpreadGeom g, co
             bpk = s_pb[q];
             c = s_pc[q];
         } else {
-            i = olist[entry(q)];
-            stage(i, bpk, c);
+            stage(olist[entry(q)], i, bpk, c);
         }
         const int bx = bpk & 0xff, by = (bpk >> 8) & 0xff, bz = bpk >> 16;
         const float *node = s_g + ((bx * S + by + ty0) * S + bz + tz) * CT_NF;
@@ -844,120 +864,240 @@ struct RealParams {
     float x_scale, inv_dr;   // ewald_n / (rcut - dr), 1 / dr
 };
 
-// Mobility_RealSpace_kernel (Mobility.cu:1046-1226) + LinearCombination/Add4
-// + Mobility_D2WE_kernel + Saddle_MakeGeneralizedU_kernel (+ the saddle's
-// x_U term), G lanes per particle (4, 8 or 16, the autotuner's choice; 16 by default).
-// Particles are taken in cell order (`order`, the neighbour list's cell-sorted
-// particles) with each XCD given one contiguous range of workgroups, so the
-// neighbours gathered by concurrent particles share that XCD's L2.
+// ------------------------------------------------------ real-space sum
+struct RealPair {
+    float dx, dy, dz, idist, fac;
+    int row;         // of the table
+    bool in;         // inside the cutoff
+};
+__device__ __forceinline__ RealPair real_pair(const RealParams &rp, float xi, float yi, float zi, float4 qj)
+{
+    RealPair p;
+    p.dx = xi - qj.x; p.dy = yi - qj.y; p.dz = zi - qj.z;
+    box_min_image(rp.b, p.dx, p.dy, p.dz);
+    const float d2 = dist2_nc(p.dx, p.dy, p.dz);
+    p.in = d2 < rp.rcut * rp.rcut && d2 >= rp.dr * rp.dr;
+    // distance and its inverse to their last bits, both from the unit's reciprocal square root by Newton steps
+    // (the root and the quotient apart take twice the instructions); d2 = 0 is not inside
+    const float y = __builtin_amdgcn_rsqf(d2);
+    float dist = d2 * y, h = 0.5f * y;
+    const float e = fmaf(-h, dist, 0.5f);
+    dist = fmaf(dist, e, dist);
+    h = fmaf(h, e, h);
+    dist = fmaf(fmaf(-dist, dist, d2), h, dist);
+    p.idist = h + h;
+    p.idist = fmaf(fmaf(-dist, p.idist, 1.0f), p.idist, p.idist);
+    // table position with the divisions by constants done once on the host (x_scale =
+    // ewald_n / (rcut - dr), inv_dr = 1 / dr)
+    const float xr = (dist - rp.dr) * rp.x_scale;
+    const int r = (int)floorf(xr);
+    p.row = r < 0 ? 0 : (r > rp.ewald_n - 1 ? rp.ewald_n - 1 : r);
+    p.fac = dist * rp.inv_dr - (float)p.row - 1.0f;
+    return p;
+}
+
+// A particle's sums: velocity, antisymmetric part of the velocity gradient, (yz - zy, zx - xz, xy - yx) / 2,
+// and its symmetric part (xx, 2 xy, 2 xz, 2 yz, yy)
+struct RealSum {
+    float u[3], t[3], e[5];
+};
+
+// Adds the pair's part (Mobility_RealSpace_kernel, Mobility.cu:1046-1226): q the neighbour's record, m and p the
+// table's rows row and row + 1.  With the unit separation R and the couplet C = S + A, A x = x cross w, the pair
+// sums are over s = S R and a = A R (C R = s + a, R C = s - a):
+//   u += f1 F + (f2 - f1)(R.F) R + g1 (C R - rCr R) + g2 (R C - 4 rCr R)
+//   D += X R + R Y + K2 1 + h1 C + (-4 h1 - h3) C^T
+//   X = K1 R - g2 F + h3 (C R + R C),  Y = -g1 F + h2 C R + h3 R C
+// of which the symmetric part takes only X + Y and the antisymmetric part (X - Y) cross R, a third fewer
+// operations than the nine components of D.
+__device__ __forceinline__ void real_add(const RealPair &w, const float4 q[4], float4 m1, float4 m2, float4 p1,
+                                         float4 p2, RealSum &o)
+{
+    const float fac = w.fac;
+    const float f1 = m1.x + (p1.x - m1.x) * fac;
+    const float f2 = m1.y + (p1.y - m1.y) * fac;
+    const float g1 = -(m1.z + (p1.z - m1.z) * fac);
+    const float g2 = -(m1.w + (p1.w - m1.w) * fac);
+    const float h1 = m2.x + (p2.x - m2.x) * fac;
+    const float h2 = m2.y + (p2.y - m2.y) * fac;
+    const float h3 = m2.z + (p2.z - m2.z) * fac;
+    const float R[3] = {w.dx * w.idist, w.dy * w.idist, w.dz * w.idist};
+    const float F[3] = {q[0].w, q[1].x, q[1].y};
+    const float sxx = q[1].z, sxy = q[1].w, sxz = q[2].x, syz = q[2].y, syy = q[2].z;
+    const float W[3] = {q[2].w, q[3].x, q[3].y};
+    const float s[3] = {sxx * R[0] + sxy * R[1] + sxz * R[2], sxy * R[0] + syy * R[1] + syz * R[2],
+                        sxz * R[0] + syz * R[1] - (sxx + syy) * R[2]};
+    const float a[3] = {R[1] * W[2] - R[2] * W[1], R[2] * W[0] - R[0] * W[2], R[0] * W[1] - R[1] * W[0]};
+    const float rF = R[0] * F[0] + R[1] * F[1] + R[2] * F[2];
+    const float rCr = R[0] * s[0] + R[1] * s[1] + R[2] * s[2];
+    const float gs = g1 + g2, gd = g1 - g2, gk = g1 + 4.f * g2, hd = h2 - h3, hs = h2 + 3.f * h3;
+    const float ku = (f2 - f1) * rF - gk * rCr;
+    const float K1 = gk * rF - (h2 + 6.f * h3) * rCr;
+    const float K2 = h3 * rCr - g2 * rF;
+    float Z[3], V[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        o.u[c] += f1 * F[c] + gs * s[c] + gd * a[c] + ku * R[c];
+        Z[c] = K1 * R[c] - gs * F[c] + hs * s[c] + hd * a[c];
+        V[c] = 0.5f * gd * F[c] - 0.5f * hd * (s[c] + a[c]);
+    }
+    const float ht = 5.f * h1 + h3, he = -3.f * h1 - h3;
+    o.t[0] += V[1] * R[2] - V[2] * R[1] + ht * W[0];
+    o.t[1] += V[2] * R[0] - V[0] * R[2] + ht * W[1];
+    o.t[2] += V[0] * R[1] - V[1] * R[0] + ht * W[2];
+    o.e[0] += Z[0] * R[0] + he * sxx + K2;
+    o.e[1] += Z[0] * R[1] + R[0] * Z[1] + 2.f * he * sxy;
+    o.e[2] += Z[0] * R[2] + R[0] * Z[2] + 2.f * he * sxz;
+    o.e[3] += Z[1] * R[2] + R[1] * Z[2] + 2.f * he * syz;
+    o.e[4] += Z[1] * R[1] + he * syy + K2;
+}
+
+// Sums over the G lanes of particle i, its own part, the wave-space result (wave, may be null),
+// Mobility_D2WE_kernel (Helper_Mobility.cu:235-283) and Saddle_MakeGeneralizedU_kernel with the
+// saddle's x_U term (addU, may be null).  Every lane forms the results; lane l writes number l.
 template <int G>
-__global__ void __launch_bounds__(256) realspace_kernel(RealParams rp, const float4 *pos, const float4 *rec,
-                                                        const float4 *tab, const int *nneigh, const int *nlist,
-                                                        int maxn, int N, const float *wave, const float *addU,
-                                                        int use_real, float *gU, const int *order)
+__device__ __forceinline__ void real_finish(const RealParams &rp, const float4 *rec, int N, const float *wave,
+                                            const float *addU, int use_real, float *gU, bool active, int slot, int i,
+                                            int lane, RealSum &o)
+{
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        o.u[c] = group_sum<G>(o.u[c]);
+        o.t[c] = group_sum<G>(o.t[c]);
+    }
+#pragma unroll
+    for (int c = 0; c < 5; ++c) o.e[c] = group_sum<G>(o.e[c]);
+    if (!active) return;
+    if (use_real) {
+        const float4 q0 = rec[4 * (int64_t)slot], q1 = rec[4 * (int64_t)slot + 1], q2 = rec[4 * (int64_t)slot + 2],
+                     q3 = rec[4 * (int64_t)slot + 3];
+        // self_y (C - 4 C^T)
+        const float x = rp.self_x, y = rp.self_y;
+        o.u[0] += x * q0.w; o.u[1] += x * q1.x; o.u[2] += x * q1.y;
+        o.t[0] += y * 5.f * q2.w; o.t[1] += y * 5.f * q3.x; o.t[2] += y * 5.f * q3.y;
+        o.e[0] -= y * 3.f * q1.z; o.e[4] -= y * 3.f * q2.z;
+        o.e[1] -= y * 6.f * q1.w; o.e[2] -= y * 6.f * q2.x; o.e[3] -= y * 6.f * q2.y;
+    }
+    if (wave) {
+        const float *w = wave + 11 * (int64_t)i, *D = w + 3;
+        o.u[0] += w[0]; o.u[1] += w[1]; o.u[2] += w[2];
+        o.t[0] += 0.5f * (D[3] - D[7]); o.t[1] += 0.5f * (D[6] - D[2]); o.t[2] += 0.5f * (D[1] - D[5]);
+        o.e[0] += D[0]; o.e[1] += D[1] + D[5]; o.e[2] += D[2] + D[6]; o.e[3] += D[3] + D[7]; o.e[4] += D[4];
+    }
+    const float out[11] = {o.u[0], o.u[1], o.u[2], o.t[0], o.t[1], o.t[2],
+                           2.f * o.e[0] + o.e[4], o.e[1], o.e[2], o.e[3], 2.f * o.e[4] + o.e[0]};
+    for (int l = lane; l < 11; l += G) {     // one round for 16 lanes
+        float v = out[0];
+#pragma unroll
+        for (int q = 1; q < 11; ++q) v = (l == q) ? out[q] : v;
+        if (addU && l < 6) v += addU[6 * (int64_t)i + l];
+        gU[l < 6 ? 6 * (int64_t)i + l : 6 * (int64_t)N + 5 * (int64_t)i + l - 6] = v;
+    }
+}
+
+// One particle by G lanes, its neighbours by slot (snn, nslot); table(row, m1, m2, p1, p2) gives the table's rows row and row + 1.
+template <int G, typename Tab>
+__device__ __forceinline__ void real_particle(const RealParams &rp, const float4 *rec, Tab table, const int *snn,
+                                              const int *nslot, int maxn, int N, const float *wave, const float *addU,
+                                              int use_real, float *gU, bool active, int slot, const int *order,
+                                              int lane)
+{
+    RealSum o = {};
+    const int i = (active && order) ? order[slot] : slot;
+    if (active && use_real) {
+        const float4 qi = rec[4 * (int64_t)slot];
+        const int nn = snn[slot];
+        for (int k = lane; k < nn; k += G) {
+            const int64_t j = nslot[(int64_t)slot * maxn + k];
+            float4 q[4];
+            q[0] = rec[4 * j];
+            const RealPair w = real_pair(rp, qi.x, qi.y, qi.z, q[0]);
+            if (!w.in) continue;
+#pragma unroll
+            for (int r = 1; r < 4; ++r) q[r] = rec[4 * j + r];
+            float4 m1, m2, p1, p2;
+            table(w.row, m1, m2, p1, p2);
+            real_add(w, q, m1, m2, p1, p2, o);
+        }
+    }
+    real_finish<G>(rp, rec, N, wave, addU, use_real, gU, active, slot, i, lane, o);
+}
+
+// Particles are taken by slot (cell order) with each XCD given one contiguous range of workgroups, so
+// the records gathered by concurrent particles lie close together in that XCD's L2; a particle's count,
+// list and record are found from its slot alone, in one round of loads.  Bound by its gathers at 16-byte
+// lanes (the texture units are busy all the time: four loads for a neighbour's record, four for the
+// table) with VALU work of two thirds of that: 31.5 us at N = 32768 and volume fraction 0.45, 8.1 us at
+// N = 4072 (by particle index, with the gradient's nine components: 36.6 and 9.0).
+template <int G>
+__global__ void __launch_bounds__(256) realspace_kernel(RealParams rp, const float4 *rec, const float4 *tab,
+                                                        const int *snn, const int *nslot, int maxn, int N,
+                                                        const float *wave, const float *addU, int use_real, float *gU,
+                                                        const int *order)
 {
     const int gid = xcd_remap(blockIdx.x, gridDim.x) * blockDim.x + threadIdx.x;
     const int slot = gid / G, lane = gid % G;
     const bool active = slot < N;
-    const int i = (active && order) ? order[slot] : slot;
-    float u[3] = {0.f, 0.f, 0.f};
-    float D[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (active && use_real) {
-        const float4 pi = pos[i];
-        const float mind2 = rp.dr * rp.dr, maxd2 = rp.rcut * rp.rcut;
-        const int nn = nneigh[i];
-        for (int k = lane; k < nn; k += G) {
-            const int j = nlist[(int64_t)i * maxn + k];
-            const float4 pj = pos[j];
-            float dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
-            box_min_image(rp.b, dx, dy, dz);
-            const float d2 = dist2_nc(dx, dy, dz);
-            if (!(d2 < maxd2 && d2 >= mind2)) continue;
-            const float dist = sqrtf(d2);
-            // table position with the divisions by constants done once on the host (x_scale =
-            // ewald_n / (rcut - dr), inv_dr = 1 / dr)
-            const float xr = (dist - rp.dr) * rp.x_scale;
-            int r_ind = (int)floorf(xr);
-            r_ind = r_ind < 0 ? 0 : (r_ind > rp.ewald_n - 1 ? rp.ewald_n - 1 : r_ind);
-            const float fac = dist * rp.inv_dr - (float)r_ind - 1.0f;
-            const float4 m1 = tab[2 * r_ind], p1 = tab[2 * r_ind + 2];
-            const float4 m2 = tab[2 * r_ind + 1], p2 = tab[2 * r_ind + 3];
-            const float f1 = m1.x + (p1.x - m1.x) * fac;
-            const float f2 = m1.y + (p1.y - m1.y) * fac;
-            const float g1 = -(m1.z + (p1.z - m1.z) * fac);
-            const float g2 = -(m1.w + (p1.w - m1.w) * fac);
-            const float h1 = m2.x + (p2.x - m2.x) * fac;
-            const float h2 = m2.y + (p2.y - m2.y) * fac;
-            const float h3 = m2.z + (p2.z - m2.z) * fac;
-            const float idist = 1.0f / dist;
-            const float R[3] = {dx * idist, dy * idist, dz * idist};
-            const float4 r0 = rec[3 * (int64_t)j], r1 = rec[3 * (int64_t)j + 1], r2 = rec[3 * (int64_t)j + 2];
-            const float Fj[3] = {r0.x, r0.y, r0.z};
-            const float C[8] = {r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, r2.y, r2.z};
-            const float rdotf = R[0] * Fj[0] + R[1] * Fj[1] + R[2] * Fj[2];
-            const float Cm[3][3] = {{C[0], C[1], C[2]}, {C[5], C[4], C[3]}, {C[6], C[7], -(C[0] + C[4])}};
-            float Cdr[3], rdC[3];
-            for (int a = 0; a < 3; ++a) {
-                Cdr[a] = Cm[a][0] * R[0] + Cm[a][1] * R[1] + Cm[a][2] * R[2];
-                rdC[a] = R[0] * Cm[0][a] + R[1] * Cm[1][a] + R[2] * Cm[2][a];
-            }
-            const float rCr = R[0] * Cdr[0] + R[1] * Cdr[1] + R[2] * Cdr[2];
-            // u_a += f1 F_a + (f2 - f1)(r.F) R_a + g1 (Cdr_a - rCr R_a) + g2 (rdC_a - 4 rCr R_a)
-            const float ku = (f2 - f1) * rdotf - (g1 + 4.f * g2) * rCr;
-            for (int a = 0; a < 3; ++a) u[a] += f1 * Fj[a] + g1 * Cdr[a] + g2 * rdC[a] + ku * R[a];
-            // D_ab += -g1 (R_a F_b - (r.F) R_a R_b) - g2 (d_ab (r.F) + F_a R_b - 4 (r.F) R_a R_b)
-            //       + h1 (C_ab - 4 C_ba) + h2 (R_a Cdr_b - rCr R_a R_b)
-            //       + h3 (d_ab rCr + Cdr_a R_b + R_a rdC_b + rdC_a R_b - 6 rCr R_a R_b - C_ba),
-            // gathered as X_a R_b + R_a Y_b + d_ab K2 + h1 C_ab + K3 C_ba
-            const float K1 = (g1 + 4.f * g2) * rdotf - (h2 + 6.f * h3) * rCr;
-            const float K2 = h3 * rCr - g2 * rdotf, K3 = -(4.f * h1 + h3);
-            float X[3], Y[3];
-            for (int a = 0; a < 3; ++a) {
-                X[a] = K1 * R[a] - g2 * Fj[a] + h3 * (Cdr[a] + rdC[a]);
-                Y[a] = -g1 * Fj[a] + h2 * Cdr[a] + h3 * rdC[a];
-            }
-            const int A[8] = {0, 0, 0, 1, 1, 1, 2, 2};
-            const int B[8] = {0, 1, 2, 2, 1, 0, 0, 1};
-            const int Cs[8] = {0, 5, 6, 7, 4, 1, 2, 3};
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int a = A[c], bb = B[c];
-                float d = X[a] * R[bb] + R[a] * Y[bb] + h1 * C[c] + K3 * C[Cs[c]];
-                if (a == bb) d += K2;
-                D[c] += d;
-            }
-        }
+    real_particle<G>(
+        rp, rec,
+        [&](int r, float4 &m1, float4 &m2, float4 &p1, float4 &p2) {
+            m1 = tab[2 * r]; p1 = tab[2 * r + 2];
+            m2 = tab[2 * r + 1]; p2 = tab[2 * r + 3];
+        },
+        snn, nslot, maxn, N, wave, addU, use_real, gU, active, slot, order, lane);
+}
+
+// The same with the table in LDS, one workgroup per CU with a contiguous range of the slots, which takes
+// half of the gathers off the texture units: 27.4 us at N = 32768, 180 us at N = 262144 (volume fraction
+// 0.4; 200 from global memory).  Held are the rows from r = RS_RMIN on (spheres that do not overlap read
+// no others; those come from global memory), as two arrays of 16-byte rows, which spreads random rows
+// over all banks.
+//
+// Every workgroup loads the table (107 KB at xi = 0.5), so the list has to be long enough.  Table in LDS
+// and from global memory, by list entries: 0.33 M 12.0 and 11.3 us, 0.50 M 12.3 and 12.8, 0.75 M 14.4 and
+// 16.0, 1.0 M 18.9 and 18.1 (its workgroups end with a short pass), 1.1 M 16.5 and 19.2, 2.7 M 30 and 33,
+// 5.2 M 52 and 61.
+#define RS_RMIN 1.9f
+#define RS_ROWS 5000       // 156 KB of LDS; a longer table (xi below 0.38) stays in global memory
+#define RS_LDS_MIN 700000
+template <int G>
+__global__ void __launch_bounds__(1024) realspace_lds_kernel(RealParams rp, const float4 *rec, const float4 *tab,
+                                                             int row0, int nrows, const int *snn, const int *nslot,
+                                                             int maxn, int N, const float *wave, const float *addU,
+                                                             float *gU, const int *order)
+{
+    extern __shared__ float4 s_tab[];        // [2][nrows]
+    float4 *s_a = s_tab, *s_b = s_tab + nrows;
+    for (int q = threadIdx.x; q < 2 * nrows; q += 1024) (q & 1 ? s_b : s_a)[q >> 1] = tab[2 * row0 + q];
+    __syncthreads();
+    const int per = (N + gridDim.x - 1) / gridDim.x, first = xcd_remap(blockIdx.x, gridDim.x) * per;
+    const int last = min(first + per, N), lane = threadIdx.x % G;
+    for (int s0 = first; s0 < last; s0 += 1024 / G) {
+        const int slot = s0 + threadIdx.x / G;
+        const bool active = slot < last;
+        real_particle<G>(
+            rp, rec,
+            [&](int r, float4 &m1, float4 &m2, float4 &p1, float4 &p2) {
+                const int q = r - row0;
+                if (q >= 0) {
+                    m1 = s_a[q]; p1 = s_a[q + 1];
+                    m2 = s_b[q]; p2 = s_b[q + 1];
+                } else {
+                    m1 = tab[2 * r]; p1 = tab[2 * r + 2];
+                    m2 = tab[2 * r + 1]; p2 = tab[2 * r + 3];
+                }
+            },
+            snn, nslot, maxn, N, wave, addU, 1, gU, active, slot, order, lane);
     }
-#pragma unroll
-    for (int a = 0; a < 3; ++a) u[a] = group_sum<G>(u[a]);
-#pragma unroll
-    for (int c = 0; c < 8; ++c) D[c] = group_sum<G>(D[c]);
-    if (!active || lane != 0) return;
-    const float4 r0 = rec[3 * (int64_t)i], r1 = rec[3 * (int64_t)i + 1], r2 = rec[3 * (int64_t)i + 2];
-    if (use_real) {
-        const float C[8] = {r0.w, r1.x, r1.y, r1.z, r1.w, r2.x, r2.y, r2.z};
-        u[0] += rp.self_x * r0.x; u[1] += rp.self_x * r0.y; u[2] += rp.self_x * r0.z;
-        D[0] += rp.self_y * (C[0] - 4.f * C[0]); D[1] += rp.self_y * (C[1] - 4.f * C[5]);
-        D[2] += rp.self_y * (C[2] - 4.f * C[6]); D[3] += rp.self_y * (C[3] - 4.f * C[7]);
-        D[4] += rp.self_y * (C[4] - 4.f * C[4]); D[5] += rp.self_y * (C[5] - 4.f * C[1]);
-        D[6] += rp.self_y * (C[6] - 4.f * C[2]); D[7] += rp.self_y * (C[7] - 4.f * C[3]);
-    }
-    if (wave) {
-        const float *w = wave + 11 * (int64_t)i;
-        u[0] += w[0]; u[1] += w[1]; u[2] += w[2];
-        for (int c = 0; c < 8; ++c) D[c] += w[3 + c];
-    }
-    // D2WE (Helper_Mobility.cu:235-283)
-    const float W0 = 0.5f * (D[3] - D[7]), W1 = 0.5f * (D[6] - D[2]), W2 = 0.5f * (D[1] - D[5]);
-    const float e0 = D[0], e1 = 0.5f * (D[1] + D[5]), e2 = 0.5f * (D[2] + D[6]), e3 = 0.5f * (D[3] + D[7]), e4 = D[4];
-    float *o6 = gU + 6 * (int64_t)i;
-    float add[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (addU)
-        for (int a = 0; a < 6; ++a) add[a] = addU[6 * (int64_t)i + a];
-    o6[0] = u[0] + add[0]; o6[1] = u[1] + add[1]; o6[2] = u[2] + add[2];
-    o6[3] = W0 + add[3]; o6[4] = W1 + add[4]; o6[5] = W2 + add[5];
-    float *o5 = gU + 6 * (int64_t)N + 5 * (int64_t)i;
-    o5[0] = 2.f * e0 + e4; o5[1] = 2.f * e1; o5[2] = 2.f * e2; o5[3] = 2.f * e3; o5[4] = 2.f * e4 + e0;
+}
+
+int k_real_init(fsd_ctx *ctx)
+{
+    for (auto k : {realspace_lds_kernel<4>, realspace_lds_kernel<8>, realspace_lds_kernel<16>})
+        if (hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                2 * sizeof(float4) * RS_ROWS) != hipSuccess)
+            return -1;
+    return 0;
 }
 
 // inverse transform of the 11 half spectra in d_spec and contraction of the
@@ -994,14 +1134,14 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
     const bool tiled = ctx->tune.contract == 0 && ctx->contract_lds;
     if (tiled && ctx->contract_split)
         hipLaunchKernelGGL((contract_tile2_kernel<13, 6>), dim3(2 * ctx->ntiles), dim3(512), ctx->contract_lds,
-                           ctx->stream, g, pos, ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp,
+                           ctx->stream, g, ctx->d_spos, ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp,
                            ps.quadW * ps.prefac, ctx->d_wave);
     else if (tiled)
-        hipLaunchKernelGGL(contract_tile_kernel, dim3(ctx->ntiles), dim3(512), ctx->contract_lds, ctx->stream, g, pos,
+        hipLaunchKernelGGL(contract_tile_kernel, dim3(ctx->ntiles), dim3(512), ctx->contract_lds, ctx->stream, g, ctx->d_spos,
                            ctx->d_porig, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp,
                            ps.quadW * ps.prefac, ctx->d_wave);
     else
-        hipLaunchKernelGGL(contract_kernel, dim3(nblk((int64_t)N * 64, 256)), dim3(256), 0, ctx->stream, g, pos,
+        hipLaunchKernelGGL(contract_kernel, dim3(nblk((int64_t)N * 64, 256)), dim3(256), 0, ctx->stream, g, ctx->d_spos,
                            ctx->d_porig, ctx->d_grid, Mp, N, ps.quadW * ps.prefac, ctx->d_wave);
     FSD_HIP(hipGetLastError());
     prof_end(ctx, PROF_CONTRACT, ev);
@@ -1015,7 +1155,9 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
     const int N = ctx->N;
     const fsd_pse_info &ps = ctx->pse;
     float4 *rec = ctx->d_rec;
-    hipLaunchKernelGGL(fc_records_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, gF, N, rec);
+    const int *order = slot_order(ctx);
+    hipLaunchKernelGGL(fc_records_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, gF, pos, order, N,
+                       rec);
     FSD_HIP(hipGetLastError());
     const SpreadGeom g = spread_geom(ctx);
     const int64_t Mp = (int64_t)ps.Nx * ps.Ny * g.pz;   // grid field stride
@@ -1028,11 +1170,11 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
         hipEvent_t ev;
         prof_begin(ctx, PROF_SPREAD, &ev);
         if (ctx->tile == 8 && ctx->pse.P == 6 && ctx->tune.spread == 0)
-            hipLaunchKernelGGL(spread_mfma_kernel<6>, dim3(ctx->ntiles), dim3(512), 0, ctx->stream, g, pos,
+            hipLaunchKernelGGL(spread_mfma_kernel<6>, dim3(ctx->ntiles), dim3(512), 0, ctx->stream, g,
                                ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid, Mp);
         else
             hipLaunchKernelGGL(spread_kernel, dim3(ctx->ntiles), dim3(ctx->tile * ctx->tile * ctx->tile), 0,
-                               ctx->stream, g, pos, ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid,
+                               ctx->stream, g, ctx->d_porig, rec, ctx->d_ostart, ctx->d_olist, ctx->d_grid,
                                Mp);
         FSD_HIP(hipGetLastError());
         prof_end(ctx, PROF_SPREAD, ev);
@@ -1075,22 +1217,26 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
     // the processing order is the neighbour list's cell list (identity without a list, wave part
     // only, or for a box of fewer than three cells per side, whose list is built over all pairs)
     if (!ctx->nlist_valid && (parts & 1)) { ctx->err = "neighbour list not built"; return FSD_E_STATE; }
-    const int *order = (ctx->nlist_valid && ctx->use_cells) ? ctx->d_cell_list : nullptr;
+    const int *snn = ctx->use_cells ? ctx->d_snn : ctx->d_nneigh, *nslot = ctx->use_cells ? ctx->d_nslot : ctx->d_nlist;
     hipEvent_t ev;
     prof_begin(ctx, PROF_REAL, &ev);
     const int G = ctx->tune.real_g, blk = ctx->tune.real_blk;
     const dim3 rg(nblk((int64_t)N * G, blk)), rb(blk);
     const float4 *tab = reinterpret_cast<const float4 *>(ctx->d_ewald);
     const int ur = (parts & 1) ? 1 : 0;
-    if (G == 4)
-        hipLaunchKernelGGL(realspace_kernel<4>, rg, rb, 0, ctx->stream, rp, pos, rec, tab, ctx->d_nneigh, ctx->d_nlist,
-                           ctx->maxn, N, wave, addU, ur, gU, order);
-    else if (G == 8)
-        hipLaunchKernelGGL(realspace_kernel<8>, rg, rb, 0, ctx->stream, rp, pos, rec, tab, ctx->d_nneigh, ctx->d_nlist,
-                           ctx->maxn, N, wave, addU, ur, gU, order);
-    else
-        hipLaunchKernelGGL(realspace_kernel<16>, rg, rb, 0, ctx->stream, rp, pos, rec, tab, ctx->d_nneigh,
-                           ctx->d_nlist, ctx->maxn, N, wave, addU, ur, gU, order);
+    const int row0 = std::max(0, std::min((int)(RS_RMIN / rp.dr) - 1, ctx->ewald_nR - 2)), nrows = ctx->ewald_nR - row0;
+    const bool lds = ur && ctx->nlist_total >= RS_LDS_MIN && nrows <= RS_ROWS;
+    auto go = [&](auto plain, auto in_lds) {
+        if (lds)
+            hipLaunchKernelGGL(in_lds, dim3(256), dim3(1024), 2 * sizeof(float4) * nrows, ctx->stream, rp, rec, tab,
+                               row0, nrows, snn, nslot, ctx->maxn, N, wave, addU, gU, order);
+        else
+            hipLaunchKernelGGL(plain, rg, rb, 0, ctx->stream, rp, rec, tab, snn, nslot, ctx->maxn, N,
+                               wave, addU, ur, gU, order);
+    };
+    if (G == 4) go(realspace_kernel<4>, realspace_lds_kernel<4>);
+    else if (G == 8) go(realspace_kernel<8>, realspace_lds_kernel<8>);
+    else go(realspace_kernel<16>, realspace_lds_kernel<16>);
     FSD_HIP(hipGetLastError());
     prof_end(ctx, PROF_REAL, ev);
     return 0;

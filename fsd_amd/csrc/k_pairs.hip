@@ -168,9 +168,10 @@ __global__ void __launch_bounds__(64) cell_sort_kernel(const int *start, int nce
 
 // One entry run [q0, q1) of the cell-sorted particles (list null: the particles q0 .. q1 - 1
 // themselves) tested against particle i by its 16 lanes; the neighbours are appended to its row in
-// the run's order.  Returns the new count (which may exceed maxn; entries beyond it are dropped).
+// the run's order, and their slots (positions in the sorted list) to its slot row.  Returns the new count
+// (which may exceed maxn; entries beyond it are dropped).
 __device__ __forceinline__ int nlist_run(const float4 *pos, const BoxF &b, float4 pi, int i, const int *list, int q0,
-                                         int q1, int lane, float rl2, int maxn, int *row, int cnt)
+                                         int q1, int lane, float rl2, int maxn, int *row, int *srow, int cnt)
 {
     const int first = (threadIdx.x & 63) & ~(PG - 1);
     for (int k = q0; k < q1; k += PG) {
@@ -183,7 +184,10 @@ __device__ __forceinline__ int nlist_run(const float4 *pos, const BoxF &b, float
         const bool ok = in && j != i && dist2_nc(dx, dy, dz) < rl2;
         const unsigned m = (unsigned)(__ballot(ok) >> first) & 0xffffu;
         const int o = cnt + __popc(m & ((1u << lane) - 1u));
-        if (ok && o < maxn) row[o] = j;
+        if (ok && o < maxn) {
+            row[o] = j;
+            if (list) srow[o] = q;
+        }
         cnt += __popc(m);
     }
     return cnt;
@@ -194,8 +198,8 @@ __device__ __forceinline__ int nlist_run(const float4 *pos, const BoxF &b, float
 // two where the column wraps.
 __global__ void __launch_bounds__(PGB) nlist_cells_kernel(const float4 *pos, int N, BoxF b, int cx, int cy, int cz,
                                                           const int *cell_of, const int *start, const int *list,
-                                                          float rl2, int maxn, int *nneigh, int *nlist, int *overflow,
-                                                          int *total)
+                                                          float rl2, int maxn, int *nneigh, int *nlist, int *nslot,
+                                                          int *snn, int *overflow, int *total)
 {
     __shared__ int s_cnt[PGB / PG];
     int lane;
@@ -205,7 +209,8 @@ __global__ void __launch_bounds__(PGB) nlist_cells_kernel(const float4 *pos, int
         const float4 pi = pos[i];
         const int c = cell_of[i];
         const int ix = c / (cy * cz), iy = (c / cz) % cy, iz = c % cz;
-        int *row = nlist + (int64_t)i * maxn;
+        const int slot = (xcd_remap(blockIdx.x, gridDim.x) * PGB + threadIdx.x) / PG;
+        int *row = nlist + (int64_t)i * maxn, *srow = nslot + (int64_t)slot * maxn;
         cnt = 0;
         for (int o = 0; o < 9; ++o) {
             int jx = ix + o / 3 - 1, jy = iy + o % 3 - 1;
@@ -213,16 +218,16 @@ __global__ void __launch_bounds__(PGB) nlist_cells_kernel(const float4 *pos, int
             jy = jy < 0 ? jy + cy : (jy >= cy ? jy - cy : jy);
             const int *st = start + (jx * cy + jy) * cz;
             if (iz == 0) {
-                cnt = nlist_run(pos, b, pi, i, list, st[cz - 1], st[cz], lane, rl2, maxn, row, cnt);
-                cnt = nlist_run(pos, b, pi, i, list, st[0], st[2], lane, rl2, maxn, row, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[cz - 1], st[cz], lane, rl2, maxn, row, srow, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[0], st[2], lane, rl2, maxn, row, srow, cnt);
             } else if (iz == cz - 1) {
-                cnt = nlist_run(pos, b, pi, i, list, st[cz - 2], st[cz], lane, rl2, maxn, row, cnt);
-                cnt = nlist_run(pos, b, pi, i, list, st[0], st[1], lane, rl2, maxn, row, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[cz - 2], st[cz], lane, rl2, maxn, row, srow, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[0], st[1], lane, rl2, maxn, row, srow, cnt);
             } else {
-                cnt = nlist_run(pos, b, pi, i, list, st[iz - 1], st[iz + 2], lane, rl2, maxn, row, cnt);
+                cnt = nlist_run(pos, b, pi, i, list, st[iz - 1], st[iz + 2], lane, rl2, maxn, row, srow, cnt);
             }
         }
-        if (lane == 0) nneigh[i] = cnt < maxn ? cnt : maxn;
+        if (lane == 0) nneigh[i] = snn[slot] = cnt < maxn ? cnt : maxn;
     }
     if (lane == 0) s_cnt[threadIdx.x / PG] = cnt;
     pg_block_counts(s_cnt, maxn, overflow, total);
@@ -237,7 +242,8 @@ __global__ void __launch_bounds__(PGB) nlist_allpairs_kernel(const float4 *pos, 
     const int i = pg_particle(N, nullptr, lane);
     int cnt = -1;
     if (i >= 0) {
-        cnt = nlist_run(pos, b, pos[i], i, nullptr, 0, N, lane, rl2, maxn, nlist + (int64_t)i * maxn, 0);
+        cnt = nlist_run(pos, b, pos[i], i, nullptr, 0, N, lane, rl2, maxn, nlist + (int64_t)i * maxn, nullptr,
+                        0);
         if (lane == 0) nneigh[i] = cnt < maxn ? cnt : maxn;
     }
     if (lane == 0) s_cnt[threadIdx.x / PG] = cnt;
@@ -284,6 +290,7 @@ int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
     const float rl = ctx->pse.rcut + ctx->p.r_buff;
     const float rl2 = rl * rl;
     hipEvent_t ev;
+    ctx->spread_valid = false;      // its arrays are in the order of the list before
     prof_begin(ctx, PROF_NLIST, &ev);
     for (int attempt = 0; attempt < 2; ++attempt) {
         FSD_HIP(hipMemsetAsync(ctx->d_flags, 0, 8 * sizeof(int), ctx->stream));
@@ -299,7 +306,8 @@ int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
                                ctx->d_cell_start, ctx->ncells, ctx->d_cell_list);
             hipLaunchKernelGGL(nlist_cells_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
                                ctx->ncell[0], ctx->ncell[1], ctx->ncell[2], ctx->d_cell_of, ctx->d_cell_start,
-                               ctx->d_cell_list, rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags, ctx->d_flags + 4);
+                               ctx->d_cell_list, rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_nslot, ctx->d_snn,
+                               ctx->d_flags, ctx->d_flags + 4);
         } else {
             hipLaunchKernelGGL(nlist_allpairs_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
                                rl2, ctx->maxn, ctx->d_nneigh, ctx->d_nlist, ctx->d_flags, ctx->d_flags + 4);
@@ -315,6 +323,10 @@ int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
         int newmax = ((need + 32) / 32) * 32 + 32;
         FSD_HIP(hipFree(ctx->d_nlist));
         FSD_HIP(hipMalloc(&ctx->d_nlist, sizeof(int) * (size_t)N * newmax));
+        if (ctx->use_cells) {
+            FSD_HIP(hipFree(ctx->d_nslot));
+            FSD_HIP(hipMalloc(&ctx->d_nslot, sizeof(int) * (size_t)N * newmax));
+        }
         ctx->maxn = newmax;
     }
     // positions the list was built at, for the rebuild check

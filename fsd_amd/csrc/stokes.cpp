@@ -216,6 +216,8 @@ static int alloc_all(fsd_ctx *ctx)
         CK(hipMalloc(&ctx->d_cell_count, sizeof(int) * ctx->ncells));
         CK(hipMalloc(&ctx->d_cell_start, sizeof(int) * (ctx->ncells + 1)));
         CK(hipMalloc(&ctx->d_cell_list, sizeof(int) * N));
+        CK(hipMalloc(&ctx->d_snn, sizeof(int) * N));
+        CK(hipMalloc(&ctx->d_nslot, sizeof(int) * (size_t)N * ctx->maxn));
     }
     CK(hipMalloc(&ctx->d_flags, sizeof(int) * 16));
     CK(hipMalloc(&ctx->d_pos_last, sizeof(float4) * (size_t)N));
@@ -237,6 +239,7 @@ static int alloc_all(fsd_ctx *ctx)
     ctx->tile = 8;
     ctx->tiles[0] = (ps.Nx + 7) / 8; ctx->tiles[1] = (ps.Ny + 7) / 8; ctx->tiles[2] = (ps.Nz + 7) / 8;
     ctx->ntiles = ctx->tiles[0] * ctx->tiles[1] * ctx->tiles[2];
+    CK(hipMalloc(&ctx->d_spos, sizeof(float4) * (size_t)N));
     CK(hipMalloc(&ctx->d_porig, sizeof(int) * 3 * N));
     CK(hipMalloc(&ctx->d_ocell, sizeof(int) * N));
     CK(hipMalloc(&ctx->d_olist, sizeof(int) * N));
@@ -245,6 +248,7 @@ static int alloc_all(fsd_ctx *ctx)
     CK(hipMalloc(&ctx->d_scan_tmp, sizeof(int) * 2 * (scan_excl_chunks(ctx->M) + 1)));
     if (ctx->tile + ps.P - 1 > 32) { ctx->err = "spreading support P too large for the tile halo"; return FSD_E_PARAM; }
     ctx->contract_lds = k_contract_lds(ctx);
+    if (k_real_init(ctx)) { ctx->err = "the real-space sum's LDS request was refused"; return FSD_E_HIP; }
     // FSD_TRSV_LEVELS=1 runs the triangular sweeps one launch per level; IC(0) applied by Jacobi
     // iterations needs no sweep plans (the learned mode keeps them for an exact IC(0) fallback)
     {
@@ -256,7 +260,7 @@ static int alloc_all(fsd_ctx *ctx)
         ctx->tp_joint = jt && jt[0] == '1';
     }
     CK(hipMalloc(&ctx->d_wave, sizeof(float) * 11 * (size_t)N));
-    CK(hipMalloc(&ctx->d_rec, sizeof(float4) * 3 * (size_t)N));
+    CK(hipMalloc(&ctx->d_rec, sizeof(float4) * 4 * (size_t)N));
     {
         // transforms: this library's kernels when the grid fits (k_fft.hip); FSD_FFT_3D=1 keeps the
         // 3-D library plans and the separate Green's function
@@ -352,7 +356,7 @@ static int alloc_all(fsd_ctx *ctx)
 static void free_all(fsd_ctx *ctx)
 {
     lp_free(ctx);
-    void *ptrs[] = {ctx->d_nneigh, ctx->d_nlist, ctx->d_cell_of, ctx->d_cell_count, ctx->d_cell_start,
+    void *ptrs[] = {ctx->d_nneigh, ctx->d_nlist, ctx->d_snn, ctx->d_nslot, ctx->d_spos, ctx->d_cell_of, ctx->d_cell_count, ctx->d_cell_start,
                     ctx->d_cell_list, ctx->d_flags, ctx->d_pos_last, ctx->d_lub_n, ctx->d_lub_j, ctx->d_lub_a, ctx->d_lub_b,
                     ctx->d_lub_self, ctx->d_grid, ctx->d_spec, ctx->d_gridk, ctx->d_fftwork, ctx->d_porig,
                     ctx->d_ocell, ctx->d_olist, ctx->d_ocount, ctx->d_ostart, ctx->d_scan_tmp, ctx->d_wave, ctx->d_rec,
