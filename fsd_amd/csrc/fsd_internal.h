@@ -333,9 +333,11 @@ struct fsd_ctx {
     // saddle / GMRES
     float *d_V = nullptr, *d_w = nullptr, *d_t = nullptr, *d_t2 = nullptr;
     float *d_Z = nullptr;         // M^-1 V of the right-preconditioned solve (allocated on first use)
-    double *d_part = nullptr; int part_blocks = 0; double *h_part = nullptr;
+    double *d_part[2] = {nullptr, nullptr};     // partial sums of the Gram-Schmidt kernels (in turn)
+    double *h_part = nullptr;     // pinned: Hessenberg columns
+    double *h_nrm = nullptr;      // pinned: partial sums of norms the host finishes
     hipEvent_t gm_ev[2] = {nullptr, nullptr};   // readbacks of the Hessenberg columns (two slots)
-    int kmax = 64;                // most vectors of one multidot (restart + 1, at least 64)
+    int kmax = 64;                // restart + 1, at least 64
     float *d_rhs = nullptr, *d_sol = nullptr;
     // FP64-residual iterative refinement (allocated on first use)
     double *d_x64 = nullptr, *d_r64 = nullptr, *d_ybot64 = nullptr, *d_norm64 = nullptr;
@@ -352,8 +354,8 @@ struct fsd_ctx {
     bool bro_alloc = false;
     int m_lanczos_ff = 2, m_lanczos_nf = 2;   // Krylov sizes carried between steps (Stokes.cc:122-123)
     float *d_lanV = nullptr;      // (BRO_MMAX + 1) x 11N Lanczos basis
-    float *d_lanw = nullptr, *d_lany0 = nullptr;           // 11N each
-    double *d_lan_h = nullptr, *h_lan = nullptr;           // 256 doubles (device, pinned host)
+    float *d_lany0 = nullptr;     // 11N
+    double *h_lan = nullptr;      // pinned: 3 doubles per Lanczos step, then partial sums
     float *d_noise = nullptr;     // generated noise: 11N far real | 6M far grid | 6N near | 6N RFD
     const float *inj_ff_real = nullptr, *inj_ff_grid = nullptr, *inj_nf = nullptr, *inj_rfd = nullptr;
     float4 *d_posp = nullptr;     // shifted positions of the random finite difference
@@ -451,10 +453,18 @@ int k_axpby(fsd_ctx *ctx, int64_t n, float a, const float *x, float b, const flo
 int k_copy(fsd_ctx *ctx, int64_t n, const float *x, float *y);
 int k_fill(fsd_ctx *ctx, int64_t n, float v, float *y);
 int autotune_run(fsd_ctx *ctx, const float4 *pos);
-int k_multidot(fsd_ctx *ctx, int64_t n, int k, const float *V, int64_t ldv, const float *w, double *out);
-int k_multi_axpy(fsd_ctx *ctx, int64_t n, int k, const float *V, int64_t ldv, const double *h, float *w);
-int k_nrm2(fsd_ctx *ctx, int64_t n, const float *x, double *out);
-int k_scale_by_norm(fsd_ctx *ctx, int64_t n, float *v, const double *h, int K, double *hn_out);
+// Gram-Schmidt pieces.  w <- w - V V^T w (K columns of length n, once or twice: passes), w / |w|; the
+// coefficients from kfirst on of the passes and the norm go to pinned memory (h1, h2, norm).
+// Partial sums of |w|^2 (their count in *nch).  v = w / |w| with |w|^2 the sum of such partials (|w| to *hn).
+// out = x0 - sum c_k V_k with, if part, partial pairs of |prev - out|^2 and |out|^2.
+// gs_part_doubles(n, K): room for the partials of K sums
+int64_t gs_part_doubles(int64_t n, int K);
+int k_gs_orthonormalise(fsd_ctx *ctx, int64_t n, int K, const float *V, float *w, int passes, int kfirst, double *h1,
+                        double *h2, double *norm);
+int k_gs_norm(fsd_ctx *ctx, int64_t n, const float *w, double *out, int *nch);
+int k_gs_scale(fsd_ctx *ctx, int64_t n, const float *w, float *v, const double *part, double *hn);
+int k_gs_combine(fsd_ctx *ctx, int64_t n, int K, const float *V, const double *c, const float *x0, float *out,
+                 const float *prev, double *part, int *nch);
 int k_saddle_precond(fsd_ctx *ctx, const float *b, float *x);
 // the factor's application by Jacobi iterations (k_jacobi.hip)
 int k_diag_inverse(fsd_ctx *ctx);

@@ -44,55 +44,34 @@ int k_fill(fsd_ctx *ctx, int64_t n, float v, float *y)
     return 0;
 }
 
-// partial dot products: block (chunk, k) reduces sum_q V_k[q] w[q] over its chunk
-#define DOT_CHUNK 4096
-__global__ void __launch_bounds__(256) multidot_partial_kernel(int64_t n, const float *V, int64_t ldv, const float *w,
-                                                               double *part, int nchunks)
-{
-    __shared__ double red[4];
-    const int k = blockIdx.y, ch = blockIdx.x;
-    const float *v = V + (int64_t)k * ldv;
-    const int64_t beg = (int64_t)ch * DOT_CHUNK;
-    const int64_t end = min(n, beg + DOT_CHUNK);
-    double s = 0.0;
-    for (int64_t q = beg + threadIdx.x; q < end; q += 256) s += (double)v[q] * (double)w[q];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) part[(int64_t)k * nchunks + ch] = red[0] + red[1] + red[2] + red[3];
-}
+// ---------------------------------------------- Gram-Schmidt, norms, combinations
+// The orthogonalisation of GMRES and Lanczos: two classical passes of h = V^T w, w -= V h, then
+// v = w / |w|; FP64 sums of FP32 vectors.  The host never waits inside; what it needs (h, |w|) block 0
+// writes to pinned memory.
+//
+// Short vectors (n up to GS_FUSED) are bound by launches and by the latency of a block's loads: four
+// launches, in each of which every block first sums the partials of the launch before (in the same
+// order in every block), and where a chunk of w stays in registers between w -= V h1 and its part of
+// h2 = V^T w.  Long vectors are bound by reading V, and the partials that every block would read are
+// no longer small against that: the sums get a launch of their own, and the products a block per vector
+// and four chunks (17 us for a mean of 40 vectors at n = 557056; 25 us with eight vectors to a block, at
+// one, two or four chunks).
+//   short: dots | sum, axpy, dots | sum, axpy, norm | sum, scale
+//   long:  dots | sum | axpy | dots | sum | axpy, norm | sum, scale
+// The short products and the updates read the vectors eight at a time, and the eight sums over a wave's
+// lanes share one butterfly (10 exchanges, 48 one by one).
+#define GS_NT 256
+#define GS_CH (4 * GS_NT)     // numbers of a block, four to a thread
+#define GS_KMAX 256
+#define GS_FUSED (1 << 17)
+#define GS_LONG 4             // chunks of a block of the long products
 
-__global__ void __launch_bounds__(256) reduce_parts_kernel(const double *part, int nchunks, double *out)
+static int gs_chunks(int64_t n) { return (int)((n + GS_CH - 1) / GS_CH); }
+static int gs_dot_blocks(int64_t n) { return n > GS_FUSED ? (gs_chunks(n) + GS_LONG - 1) / GS_LONG : gs_chunks(n); }
+int64_t gs_part_doubles(int64_t n, int K)      // for every length up to n
 {
-    __shared__ double red[4];
-    const int k = blockIdx.x;
-    double s = 0.0;
-    for (int c = threadIdx.x; c < nchunks; c += 256) s += part[(int64_t)k * nchunks + c];
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) out[k] = red[0] + red[1] + red[2] + red[3];
-}
-
-// the same on float4 (n, ldv multiples of 4, 16-byte aligned vectors): a quarter of the load instructions
-__global__ void __launch_bounds__(256) multidot_partial4_kernel(int64_t n4, const float4 *V, int64_t ldv4,
-                                                                const float4 *w, double *part, int nchunks)
-{
-    __shared__ double red[4];
-    const int k = blockIdx.y, ch = blockIdx.x;
-    const float4 *v = V + (int64_t)k * ldv4;
-    const int64_t beg = (int64_t)ch * (DOT_CHUNK / 4);
-    const int64_t end = min(n4, beg + DOT_CHUNK / 4);
-    double s = 0.0;
-    for (int64_t q = beg + threadIdx.x; q < end; q += 256) {
-        const float4 a = v[q], b = w[q];
-        s += (double)a.x * (double)b.x + (double)a.y * (double)b.y + (double)a.z * (double)b.z +
-             (double)a.w * (double)b.w;
-    }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) part[(int64_t)k * nchunks + ch] = red[0] + red[1] + red[2] + red[3];
+    const int64_t blocks = n > GS_FUSED ? std::max(gs_dot_blocks(n), GS_FUSED / GS_CH) : gs_chunks(n);
+    return std::max(std::min(K, GS_KMAX) * blocks, (int64_t)gs_chunks(n));
 }
 
 static bool vec4_ok(int64_t n, int64_t ldv, const void *a, const void *b)
@@ -100,97 +79,345 @@ static bool vec4_ok(int64_t n, int64_t ldv, const void *a, const void *b)
     return n % 4 == 0 && ldv % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b)) & 15) == 0;
 }
 
-// out[k] = <V_k, w> for k < K (out is a device array of K doubles)
-int k_multidot(fsd_ctx *ctx, int64_t n, int K, const float *V, int64_t ldv, const float *w, double *out)
+// this thread's four numbers of chunk c (VEC: 16-byte accesses), zero past the end
+template <bool VEC>
+__device__ __forceinline__ void gs_load(const float *p, int64_t n, int c, float (&x)[4])
 {
-    const int nchunks = (int)((n + DOT_CHUNK - 1) / DOT_CHUNK);
-    if (vec4_ok(n, ldv, V, w))
-        hipLaunchKernelGGL(multidot_partial4_kernel, dim3(nchunks, K), dim3(256), 0, ctx->stream, n / 4,
-                           reinterpret_cast<const float4 *>(V), ldv / 4, reinterpret_cast<const float4 *>(w),
-                           ctx->d_part, nchunks);
-    else
-        hipLaunchKernelGGL(multidot_partial_kernel, dim3(nchunks, K), dim3(256), 0, ctx->stream, n, V, ldv, w,
-                           ctx->d_part, nchunks);
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3(K), dim3(256), 0, ctx->stream, ctx->d_part, nchunks, out);
-    FSD_HIP(hipGetLastError());
-    return 0;
-}
-
-// w -= sum_k h[k] V_k
-__global__ void multi_axpy_kernel(int64_t n, int K, const float *V, int64_t ldv, const double *h, float *w)
-{
-    __shared__ float hs[256];
-    for (int k = threadIdx.x; k < K; k += blockDim.x) hs[k] = (float)h[k];
-    __syncthreads();
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    float s = w[q];
-    for (int k = 0; k < K; ++k) s -= hs[k] * V[(int64_t)k * ldv + q];
-    w[q] = s;
-}
-
-// the same on float4 (same order of operations per element)
-__global__ void multi_axpy4_kernel(int64_t n4, int K, const float4 *V, int64_t ldv4, const double *h, float4 *w)
-{
-    __shared__ float hs[256];
-    for (int k = threadIdx.x; k < K; k += blockDim.x) hs[k] = (float)h[k];
-    __syncthreads();
-    int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n4) return;
-    float4 s = w[q];
-    for (int k = 0; k < K; ++k) {
-        const float4 v = V[(int64_t)k * ldv4 + q];
-        s.x -= hs[k] * v.x; s.y -= hs[k] * v.y; s.z -= hs[k] * v.z; s.w -= hs[k] * v.w;
+    if (VEC) {
+        const int64_t q = (int64_t)c * GS_NT + threadIdx.x;
+        const float4 v = q < n / 4 ? reinterpret_cast<const float4 *>(p)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
+        x[0] = v.x; x[1] = v.y; x[2] = v.z; x[3] = v.w;
+    } else {
+        const int64_t q = (int64_t)c * GS_CH + threadIdx.x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = q + GS_NT * e < n ? p[q + GS_NT * e] : 0.f;
     }
-    w[q] = s;
 }
 
-int k_multi_axpy(fsd_ctx *ctx, int64_t n, int K, const float *V, int64_t ldv, const double *h, float *w)
+template <bool VEC>
+__device__ __forceinline__ void gs_store(float *p, int64_t n, int c, const float (&x)[4])
 {
-    if (K > 256) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
-    if (vec4_ok(n, ldv, V, w))
-        hipLaunchKernelGGL(multi_axpy4_kernel, dim3(nblk(n / 4, 256)), dim3(256), 0, ctx->stream, n / 4, K,
-                           reinterpret_cast<const float4 *>(V), ldv / 4, h, reinterpret_cast<float4 *>(w));
-    else
-        hipLaunchKernelGGL(multi_axpy_kernel, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, n, K, V, ldv, h, w);
-    FSD_HIP(hipGetLastError());
-    return 0;
+    if (VEC) {
+        const int64_t q = (int64_t)c * GS_NT + threadIdx.x;
+        if (q < n / 4) reinterpret_cast<float4 *>(p)[q] = make_float4(x[0], x[1], x[2], x[3]);
+    } else {
+        const int64_t q = (int64_t)c * GS_CH + threadIdx.x;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (q + GS_NT * e < n) p[q + GS_NT * e] = x[e];
+    }
 }
 
-// v *= 1 / hn, hn = sqrt(max(h[K] - sum_{k<K} h[k]^2, 0)): the norm of the second
-// Gram-Schmidt pass's result from its dot products (h[0..K)) and |w'|^2 (h[K]).
-// Every block forms hn the same way; block 0 stores it in *hn_out.
-__global__ void __launch_bounds__(256) scale_by_norm_kernel(int64_t n, float *v, const double *h, int K,
-                                                            double *hn_out)
+// x -= sum_k h[k] V_k on chunk c
+template <bool VEC>
+__device__ __forceinline__ void gs_update(const float *V, int64_t n, int c, int K, const float *h, float (&x)[4])
 {
-    __shared__ float s_inv;
-    if (threadIdx.x < 64) {
-        double acc = 0.0;
-        for (int k = threadIdx.x; k < K; k += 64) acc += h[k] * h[k];
-        for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
-        if (threadIdx.x == 0) {
-            const double hn = sqrt(fmax(h[K] - acc, 0.0));
-            s_inv = hn > 0.0 ? (float)(1.0 / hn) : 0.f;
-            if (blockIdx.x == 0) *hn_out = hn;
+    for (int k0 = 0; k0 < K; k0 += 8) {
+        float v[8][4];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) gs_load<VEC>(V + (int64_t)min(k0 + k, K - 1) * n, n, c, v[k]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            if (k0 + k < K) {
+                const float a = h[k0 + k];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[e] -= a * v[k][e];
+            }
+    }
+}
+
+// p[k] += <V_{k0 + k}, x> on chunk c, k < 8
+template <bool VEC>
+__device__ __forceinline__ void gs_dots8(const float *V, int64_t n, int c, int K, int k0, const float (&x)[4],
+                                         double (&p)[8])
+{
+    float v[8][4];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) gs_load<VEC>(V + (int64_t)min(k0 + k, K - 1) * n, n, c, v[k]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+        p[k] += (double)v[k][0] * (double)x[0] + (double)v[k][1] * (double)x[1] + (double)v[k][2] * (double)x[2] +
+                (double)v[k][3] * (double)x[3];
+}
+
+// the eight sums over the wave: returns sum gs_mine(lane)
+__device__ __forceinline__ int gs_mine(int lane) { return (lane >> 5 & 1) * 4 + (lane >> 4 & 1) * 2 + (lane >> 3 & 1); }
+__device__ __forceinline__ double gs_butterfly(double (&p)[8], int lane)
+{
+    // halves of the eight go to either half of the lanes, three times
+#pragma unroll
+    for (int m = 4, o = 32; m >= 1; m >>= 1, o >>= 1) {
+        const bool up = lane & o;
+#pragma unroll
+        for (int k = 0; k < m; ++k) {
+            const double keep = up ? p[k + m] : p[k], give = up ? p[k] : p[k + m];
+            p[k] = keep + __shfl_xor(give, o, 64);
         }
     }
-    __syncthreads();
-    const float inv = s_inv;
-    for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (int64_t)gridDim.x * blockDim.x)
-        v[q] *= inv;
+    double s = p[0];
+    for (int o = 4; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    return s;
 }
 
-int k_scale_by_norm(fsd_ctx *ctx, int64_t n, float *v, const double *h, int K, double *hn_out)
+// sum over the block (one value for every thread)
+__device__ __forceinline__ double block_sum(double s, double (&red)[GS_NT / 64])
 {
-    hipLaunchKernelGGL(scale_by_norm_kernel, dim3(std::min<int64_t>(nblk(n, 256), 1024)), dim3(256), 0, ctx->stream,
-                       n, v, h, K, hn_out);
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+}
+
+// partials of V^T w, short vectors: block (c, g) takes the vectors 8 g .. 8 g + 7 on chunk c
+template <bool VEC>
+__global__ void __launch_bounds__(GS_NT) gs_dots_kernel(int64_t n, int K, const float *V, const float *w, double *out)
+{
+    __shared__ double s_d[GS_NT / 64][8];
+    const int lane = threadIdx.x & 63, k0 = 8 * blockIdx.y;
+    double p[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) p[k] = 0.0;
+    float x[4];
+    gs_load<VEC>(w, n, blockIdx.x, x);
+    gs_dots8<VEC>(V, n, blockIdx.x, K, k0, x, p);
+    const double s = gs_butterfly(p, lane);
+    if ((lane & 7) == 0) s_d[threadIdx.x >> 6][gs_mine(lane)] = s;
+    __syncthreads();
+    const int k = threadIdx.x;
+    if (k < 8 && k0 + k < K)
+        out[(int64_t)(k0 + k) * gridDim.x + blockIdx.x] = s_d[0][k] + s_d[1][k] + s_d[2][k] + s_d[3][k];
+}
+
+// the same for long vectors: block (b, k) takes vector k on chunks GS_LONG b and on
+template <bool VEC>
+__global__ void __launch_bounds__(GS_NT) gs_dots_long_kernel(int64_t n, const float *V, const float *w, double *out)
+{
+    __shared__ double s_red[GS_NT / 64];
+    const float *v = V + (int64_t)blockIdx.y * n;
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < GS_LONG; ++c) {
+        float a[4], x[4];
+        gs_load<VEC>(v, n, GS_LONG * blockIdx.x + c, a);
+        gs_load<VEC>(w, n, GS_LONG * blockIdx.x + c, x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += (double)a[e] * (double)x[e];
+    }
+    s = block_sum(s, s_red);
+    if (threadIdx.x == 0) out[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] = s;
+}
+
+// sums of np partials each; sum k (k >= kfirst) also to hout
+__global__ void __launch_bounds__(GS_NT) gs_sum_kernel(const double *part, int np, double *out, double *hout, int kfirst)
+{
+    __shared__ double s_red[GS_NT / 64];
+    const int k = blockIdx.x;
+    double s = 0.0;
+    for (int c = threadIdx.x; c < np; c += GS_NT) s += part[(int64_t)k * np + c];
+    s = block_sum(s, s_red);
+    if (threadIdx.x == 0) {
+        out[k] = s;
+        if (hout && k >= kfirst) hout[k - kfirst] = s;
+    }
+}
+
+// AXPY: w -= V h, h the sums of part (K x np; np = 1: the sums themselves), which block 0 puts into
+// hout (may be null) from kfirst on.  out: K x gridDim.x partial dots (DOT) or partial squares (NORM)
+template <bool VEC, bool AXPY, bool DOT, bool NORM>
+__global__ void __launch_bounds__(GS_NT) gs_kernel(int64_t n, int K, const float *V, float *w, const double *part,
+                                                   int np, double *hout, int kfirst, double *out)
+{
+    __shared__ float s_h[GS_KMAX];
+    __shared__ double s_d[GS_NT / 64][GS_KMAX], s_red[GS_NT / 64];
+    const int c = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float x[4];
+    gs_load<VEC>(w, n, c, x);
+    if (AXPY) {
+        // as many lanes per sum as the block has (at most a wave, at least eight), or one where there is nothing
+        // to sum
+        const int L = np == 1 ? 1 : K <= 4 ? 64 : K <= 8 ? 32 : K <= 16 ? 16 : 8, l = threadIdx.x & (L - 1);
+        for (int kb = 0; kb < K; kb += GS_NT / L) {
+            const int k = kb + threadIdx.x / L;
+            double s = 0.0;
+            if (k < K) {
+                const double *p = part + (int64_t)k * np;
+#pragma unroll 8
+                for (int q = l; q < np; q += L) s += p[q];
+            }
+            for (int o = L >> 1; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (l == 0 && k < K) {
+                s_h[k] = (float)s;
+                if (hout && c == 0 && k >= kfirst) hout[k - kfirst] = s;
+            }
+        }
+        __syncthreads();
+        gs_update<VEC>(V, n, c, K, s_h, x);
+        gs_store<VEC>(w, n, c, x);
+    }
+    if (DOT) {
+        for (int k0 = 0; k0 < K; k0 += 8) {
+            double p[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) p[k] = 0.0;
+            gs_dots8<VEC>(V, n, c, K, k0, x, p);
+            const double s = gs_butterfly(p, lane);
+            const int k = k0 + gs_mine(lane);
+            if ((lane & 7) == 0 && k < K) s_d[wv][k] = s;
+        }
+        __syncthreads();
+        for (int k = threadIdx.x; k < K; k += GS_NT)
+            out[(int64_t)k * gridDim.x + c] = s_d[0][k] + s_d[1][k] + s_d[2][k] + s_d[3][k];
+    }
+    if (NORM) {
+        double s = 0.0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s += (double)x[e] * (double)x[e];
+        s = block_sum(s, s_red);
+        if (threadIdx.x == 0) out[c] = s;
+    }
+}
+
+// v = w / |w| with |w|^2 the sum of nch partials; block 0 puts |w| into hn
+template <bool VEC>
+__global__ void __launch_bounds__(GS_NT) gs_scale_kernel(int64_t n, const float *w, float *v, const double *part,
+                                                         double *hn)
+{
+    __shared__ double s_red[GS_NT / 64];
+    float x[4];
+    gs_load<VEC>(w, n, blockIdx.x, x);
+    double s = 0.0;
+#pragma unroll 4
+    for (int c = threadIdx.x; c < (int)gridDim.x; c += GS_NT) s += part[c];
+    const double h = sqrt(block_sum(s, s_red));
+    if (hn && blockIdx.x == 0 && threadIdx.x == 0) *hn = h;
+    const float inv = h > 0.0 ? (float)(1.0 / h) : 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) x[e] *= inv;
+    gs_store<VEC>(v, n, blockIdx.x, x);
+}
+
+// out = x0 - sum_k c[k] V_k (x0 may be null); with part also the partials of |prev - out|^2 and |out|^2
+struct GsCoef { float c[GS_KMAX]; };
+template <bool VEC>
+__global__ void __launch_bounds__(GS_NT) gs_combine_kernel(int64_t n, int K, const float *V, GsCoef coef,
+                                                           const float *x0, float *out, const float *prev,
+                                                           double *part)
+{
+    __shared__ float s_h[GS_KMAX];
+    __shared__ double s_red[GS_NT / 64];
+    for (int k = threadIdx.x; k < K; k += GS_NT) s_h[k] = coef.c[k];
+    float x[4];
+    if (x0) {
+        gs_load<VEC>(x0, n, blockIdx.x, x);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = 0.f;
+    }
+    __syncthreads();
+    gs_update<VEC>(V, n, blockIdx.x, K, s_h, x);
+    gs_store<VEC>(out, n, blockIdx.x, x);
+    if (part) {
+        float y[4];
+        gs_load<VEC>(prev, n, blockIdx.x, y);
+        double d = 0.0, s = 0.0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const double t = (double)(y[e] - x[e]);
+            d += t * t;
+            s += (double)x[e] * (double)x[e];
+        }
+        d = block_sum(d, s_red);
+        s = block_sum(s, s_red);
+        if (threadIdx.x == 0) { part[2 * blockIdx.x] = d; part[2 * blockIdx.x + 1] = s; }
+    }
+}
+
+template <bool AXPY, bool DOT, bool NORM>
+static int gs_launch(fsd_ctx *ctx, int64_t n, int K, const float *V, const float *w, const double *part, int np,
+                     double *hout, int kfirst, double *out)
+{
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gs_chunks(n)), dim3(GS_NT), 0, ctx->stream, n, K, V, const_cast<float *>(w),
+                           part, np, hout, kfirst, out);
+    };
+    if (vec4_ok(n, n, V ? V : w, w)) go(gs_kernel<true, AXPY, DOT, NORM>);
+    else go(gs_kernel<false, AXPY, DOT, NORM>);
     FSD_HIP(hipGetLastError());
     return 0;
 }
 
-int k_nrm2(fsd_ctx *ctx, int64_t n, const float *x, double *out)
+static int gs_dots(fsd_ctx *ctx, int64_t n, int K, const float *V, const float *w, double *out)
 {
-    return k_multidot(ctx, n, 1, x, 0, x, out);  // returns the squared norm
+    const bool vec = vec4_ok(n, n, V, w), lng = n > GS_FUSED;
+    const dim3 grid(gs_dot_blocks(n), lng ? K : (K + 7) / 8);
+    if (lng) {
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GS_NT), 0, ctx->stream, n, V, w, out); };
+        vec ? go(gs_dots_long_kernel<true>) : go(gs_dots_long_kernel<false>);
+    } else {
+        auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GS_NT), 0, ctx->stream, n, K, V, w, out); };
+        vec ? go(gs_dots_kernel<true>) : go(gs_dots_kernel<false>);
+    }
+    FSD_HIP(hipGetLastError());
+    return 0;
+}
+
+int k_gs_orthonormalise(fsd_ctx *ctx, int64_t n, int K, const float *V, float *w, int passes, int kfirst, double *h1,
+                        double *h2, double *norm)
+{
+    if (K > GS_KMAX) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
+    double *a = ctx->d_part[0], *b = ctx->d_part[1];
+    int rc = gs_dots(ctx, n, K, V, w, a);
+    for (int pass = 1; pass <= passes && !rc; ++pass) {
+        double *h = pass == 1 ? h1 : h2;
+        const bool last = pass == passes;
+        int np = gs_dot_blocks(n);
+        if (n > GS_FUSED) {
+            hipLaunchKernelGGL(gs_sum_kernel, dim3(K), dim3(GS_NT), 0, ctx->stream, a, np, b, h, kfirst);
+            std::swap(a, b);
+            np = 1;
+            h = nullptr;
+        }
+        if (last) rc = gs_launch<true, false, true>(ctx, n, K, V, w, a, np, h, kfirst, b);
+        else if (n > GS_FUSED) rc = gs_launch<true, false, false>(ctx, n, K, V, w, a, np, h, kfirst, nullptr);
+        else rc = gs_launch<true, true, false>(ctx, n, K, V, w, a, np, h, kfirst, b);
+        if (!last && n > GS_FUSED && !rc) rc = gs_dots(ctx, n, K, V, w, b);
+        std::swap(a, b);
+    }
+    return rc ? rc : k_gs_scale(ctx, n, w, w, a, norm);
+}
+
+int k_gs_norm(fsd_ctx *ctx, int64_t n, const float *w, double *out, int *nch)
+{
+    if (nch) *nch = gs_chunks(n);
+    return gs_launch<false, false, true>(ctx, n, 0, nullptr, w, nullptr, 0, nullptr, 0, out);
+}
+
+int k_gs_scale(fsd_ctx *ctx, int64_t n, const float *w, float *v, const double *part, double *hn)
+{
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gs_chunks(n)), dim3(GS_NT), 0, ctx->stream, n, w, v, part, hn);
+    };
+    const bool vec = vec4_ok(n, n, w, v);
+    vec ? go(gs_scale_kernel<true>) : go(gs_scale_kernel<false>);
+    FSD_HIP(hipGetLastError());
+    return 0;
+}
+
+int k_gs_combine(fsd_ctx *ctx, int64_t n, int K, const float *V, const double *c, const float *x0, float *out,
+                 const float *prev, double *part, int *nch)
+{
+    if (K > GS_KMAX) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
+    GsCoef coef;
+    for (int k = 0; k < GS_KMAX; ++k) coef.c[k] = k < K ? (float)c[k] : 0.f;
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(gs_chunks(n)), dim3(GS_NT), 0, ctx->stream, n, K, V, coef, x0, out, prev, part);
+    };
+    const bool vec = vec4_ok(n, n, V, out) && vec4_ok(n, n, x0, prev);
+    vec ? go(gs_combine_kernel<true>) : go(gs_combine_kernel<false>);
+    if (nch) *nch = gs_chunks(n);
+    FSD_HIP(hipGetLastError());
+    return 0;
 }
 
 // ------------------------------------------------------------ saddle

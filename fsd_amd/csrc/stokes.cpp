@@ -318,14 +318,13 @@ static int alloc_all(fsd_ctx *ctx)
     CK(hipMalloc(&ctx->d_w, sizeof(float) * n17));
     CK(hipMalloc(&ctx->d_t, sizeof(float) * n17));
     CK(hipMalloc(&ctx->d_t2, sizeof(float) * n17));
-    // dot partials of up to kmax vectors, then 2 kmax + 2 doubles of results (two projection passes, a norm)
-    ctx->part_blocks = (int)((n17 + 4095) / 4096);
     ctx->kmax = std::max(64, ctx->p.gmres_restart + 1);
-    CK(hipMalloc(&ctx->d_part, sizeof(double) * ((size_t)ctx->part_blocks * ctx->kmax + 2 * ctx->kmax + 2)));
-    // pinned: two slots of 2 kmax + 2 doubles (Hessenberg columns read back while the next
-    // iteration runs), then kmax solution coefficients
-    CK(hipHostMalloc((void **)&ctx->h_part, sizeof(double) * (2 * (2 * ctx->kmax + 2) + ctx->kmax),
-                     hipHostMallocDefault));
+    for (double *&p : ctx->d_part)
+        CK(hipMalloc(&p, sizeof(double) * gs_part_doubles(n17, std::max(ctx->kmax, BRO_MMAX))));
+    // pinned: two slots of 2 kmax + 1 doubles (a Hessenberg column's two passes and norm, written by the
+    // kernels while the host takes the one before); two norms' partial sums
+    CK(hipHostMalloc((void **)&ctx->h_part, sizeof(double) * 2 * (2 * ctx->kmax + 1), hipHostMallocDefault));
+    CK(hipHostMalloc((void **)&ctx->h_nrm, sizeof(double) * 2 * gs_part_doubles(n17, 1), hipHostMallocDefault));
     for (hipEvent_t *e : {&ctx->gm_ev[0], &ctx->gm_ev[1]}) CK(hipEventCreateWithFlags(e, hipEventDisableTiming));
     CK(hipMalloc(&ctx->d_rhs, sizeof(float) * n17));
     CK(hipMalloc(&ctx->d_sol, sizeof(float) * n17));
@@ -363,19 +362,20 @@ static void free_all(fsd_ctx *ctx)
                     ctx->d_ewald, ctx->d_res_dist, ctx->d_res_vals, ctx->d_pn, ctx->d_plist, ctx->d_pless,
                     ctx->d_perm, ctx->d_iperm, ctx->d_lrow, ctx->d_urow, ctx->d_lcol, ctx->d_ucol, ctx->d_upos,
                     ctx->d_Ablk, ctx->d_Lblk, ctx->d_Adiag, ctx->d_Ldiag, ctx->d_lev_f, ctx->d_lev_b, ctx->d_tmp6a,
-                    ctx->d_tmp6b, ctx->d_g12, ctx->d_V, ctx->d_w, ctx->d_t, ctx->d_t2, ctx->d_part, ctx->d_rhs, ctx->d_sol, ctx->d_sol_prev, ctx->d_sol_prev2,
+                    ctx->d_tmp6b, ctx->d_g12, ctx->d_V, ctx->d_w, ctx->d_t, ctx->d_t2, ctx->d_part[0], ctx->d_part[1], ctx->d_rhs, ctx->d_sol, ctx->d_sol_prev, ctx->d_sol_prev2,
                     ctx->d_force, ctx->d_mask1, ctx->d_mask2, ctx->d_tp_finfo, ctx->d_tp_binfo,
                     ctx->d_tp_fbsrc, ctx->d_tp_bbsrc, ctx->d_tp_fblk, ctx->d_tp_bblk,
                     ctx->d_tp_finp, ctx->d_tp_binp, ctx->d_tp_fres, ctx->d_tp_bres, ctx->d_tp_fseq, ctx->d_tp_bseq, ctx->d_tp_fplace, ctx->d_tp_bplace,
                     ctx->d_tp_Z, ctx->d_Fblk, ctx->d_Tblk, ctx->d_lell, ctx->d_uell, ctx->d_jac, ctx->d_Lblk2, ctx->d_Ldiag2,
                     ctx->d_x64, ctx->d_r64, ctx->d_ybot64, ctx->d_norm64, ctx->d_refx32, ctx->d_refy32,
                     ctx->d_refr32, ctx->d_refd,
-                    ctx->d_Z, ctx->d_lanV, ctx->d_lanw, ctx->d_lany0, ctx->d_lan_h, ctx->d_noise, ctx->d_posp,
+                    ctx->d_Z, ctx->d_lanV, ctx->d_lany0, ctx->d_noise, ctx->d_posp,
                     ctx->d_rfd_rhs, ctx->d_rfd_sol, ctx->d_fft_tw, ctx->d_fft_loc};
     for (void *p : ptrs)
         if (p) hipFree(p);
     if (ctx->h_flags) hipHostFree(ctx->h_flags);
     if (ctx->h_part) hipHostFree(ctx->h_part);
+    if (ctx->h_nrm) hipHostFree(ctx->h_nrm);
     for (hipEvent_t e : ctx->gm_ev)
         if (e) hipEventDestroy(e);
     if (ctx->h_lan) hipHostFree(ctx->h_lan);
@@ -710,18 +710,17 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
     float *V = ctx->d_V, *w = ctx->d_w, *t = ctx->d_t;
     if (right && !ctx->d_Z) CK(hipMalloc(&ctx->d_Z, sizeof(float) * n * R));
     float *Z = ctx->d_Z;
-    const int KM = ctx->kmax, HS = 2 * KM + 2;
-    double *d_h = ctx->d_part + (int64_t)ctx->part_blocks * KM;   // 2 kmax + 2 doubles after the partials
-    std::vector<double> H((size_t)(R + 1) * R, 0.0), cs(R), sn(R), g(R + 1), yv(R + 1);
-    auto hostsync = [&](int count) -> int {
-        CK(hipMemcpyAsync(ctx->h_part, d_h, sizeof(double) * count, hipMemcpyDeviceToHost, ctx->stream));
-        CK(hipStreamSynchronize(ctx->stream));
-        return 0;
+    const int KM = ctx->kmax, HS = 2 * KM + 1;
+    std::vector<double> H((size_t)(R + 1) * R, 0.0), cs(R), sn(R), g(R + 1), yv(R + 1), coef(R);
+    int nch = 0;
+    double *hn[2] = {ctx->h_nrm, ctx->h_nrm + gs_part_doubles(n, 1)};     // partials of |r|^2 and |b|^2
+    auto norm = [&](const double *p) {
+        double s = 0.0;
+        for (int c = 0; c < nch; ++c) s += p[c];
+        return std::sqrt(s);
     };
-    RC(k_nrm2(ctx, n, b, d_h));
-    RC(hostsync(1));
-    const double bn = std::sqrt(ctx->h_part[0]);
-    const double target = (double)tol * bn;
+    RC(k_gs_norm(ctx, n, b, hn[1], &nch));
+    double bn = 0.0, target = 0.0;
     int iters = 0, restarts = 0;
     double resid = 0.0;
     for (;;) {
@@ -737,9 +736,13 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
             RC(k_saddle_precond(ctx, t, w));
             r = w;
         }
-        RC(k_nrm2(ctx, n, r, d_h));
-        RC(hostsync(1));
-        const double beta = std::sqrt(ctx->h_part[0]);
+        RC(k_gs_norm(ctx, n, r, hn[0], &nch));
+        CK(hipStreamSynchronize(ctx->stream));
+        const double beta = norm(hn[0]);
+        if (restarts == 0) {
+            bn = norm(hn[1]);
+            target = (double)tol * bn;
+        }
         resid = beta;
         if (st && iters == 0 && restarts == 0) st->initial_residual = (float)(beta / bn);
         if (resid <= target || iters >= maxit || beta == 0.0) break;
@@ -747,7 +750,7 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
         std::fill(g.begin(), g.end(), 0.0);
         g[0] = beta;
         // Arnoldi step j runs entirely on the device (its new basis vector is normalised there), and
-        // its Hessenberg column is read back into slot j & 1 of the pinned buffer; so step j + 1 can
+        // its Hessenberg column is written into slot j & 1 of the pinned buffer; so step j + 1 can
         // be enqueued before the host has that column, and the host waits only for it.  Near
         // convergence (estimate within 1.5 x the target) the next step is enqueued after the check.
         auto enqueue = [&](int j) -> int {
@@ -763,22 +766,10 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
             }
             hipEvent_t ev;
             prof_begin(ctx, PROF_GMRES_VEC, &ev);
-            // CGS2: two passes of h = V^T w, w -= V h.  The second pass also forms |w'|^2 (w' is
-            // the next basis slot itself); after it |w''|^2 = |w'|^2 - |h2|^2, with h2 tiny, so
-            // the norm needs no pass of its own
-            RC(k_multidot(ctx, n, j + 1, V, n, vn, d_h));
-            RC(k_multi_axpy(ctx, n, j + 1, V, n, d_h, vn));
-            if (ctx->p.gs_passes == 1) {   // one classical pass: no second projection, direct norm
-                RC(k_nrm2(ctx, n, vn, d_h + KM + j + 1));
-                RC(k_scale_by_norm(ctx, n, vn, d_h + KM + j + 1, 0, d_h + 2 * KM + 1));
-            } else {
-                RC(k_multidot(ctx, n, j + 2, V, n, vn, d_h + KM));
-                RC(k_multi_axpy(ctx, n, j + 1, V, n, d_h + KM, vn));
-                RC(k_scale_by_norm(ctx, n, vn, d_h + KM, j + 1, d_h + 2 * KM + 1));
-            }
+            // CGS2: two passes of h = V^T w, w -= V h (one with gs_passes 1), then the norm
+            double *hs = ctx->h_part + (size_t)(j & 1) * HS;
+            RC(k_gs_orthonormalise(ctx, n, j + 1, V, vn, ctx->p.gs_passes == 1 ? 1 : 2, 0, hs, hs + KM, hs + 2 * KM));
             prof_end(ctx, PROF_GMRES_VEC, ev);
-            CK(hipMemcpyAsync(ctx->h_part + (size_t)(j & 1) * HS, d_h, sizeof(double) * HS, hipMemcpyDeviceToHost,
-                              ctx->stream));
             CK(hipEventRecord(ctx->gm_ev[j & 1], ctx->stream));
             return 0;
         };
@@ -795,7 +786,7 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
             const double *hs = ctx->h_part + (size_t)(i & 1) * HS;
             const bool two_pass = ctx->p.gs_passes != 1;
             for (int k = 0; k <= i; ++k) H[(size_t)k * R + i] = two_pass ? hs[k] + hs[KM + k] : hs[k];
-            H[(size_t)(i + 1) * R + i] = hs[2 * KM + 1];
+            H[(size_t)(i + 1) * R + i] = hs[2 * KM];
             for (int k = 0; k < i; ++k) {
                 const double a = H[(size_t)k * R + i], c = H[(size_t)(k + 1) * R + i];
                 H[(size_t)k * R + i] = cs[k] * a + sn[k] * c;
@@ -821,10 +812,8 @@ static int gmres_core(fsd_ctx *ctx, const float4 *pos, const float *b, float *x,
             for (int k = j + 1; k <= i; ++k) s -= H[(size_t)j * R + k] * yv[k];
             yv[j] = s / H[(size_t)j * R + j];
         }
-        double *coef = ctx->h_part + 2 * (size_t)HS;
         for (int j = 0; j <= i; ++j) coef[j] = -yv[j];
-        CK(hipMemcpyAsync(d_h, coef, sizeof(double) * (i + 1), hipMemcpyHostToDevice, ctx->stream));
-        RC(k_multi_axpy(ctx, n, i + 1, right ? Z : V, n, d_h, x));
+        RC(k_gs_combine(ctx, n, i + 1, right ? Z : V, coef.data(), x, x, nullptr, nullptr, nullptr));
         CK(hipStreamSynchronize(ctx->stream));
         ++restarts;
         if (resid <= target || iters >= maxit) break;
@@ -883,10 +872,9 @@ static int alloc_brownian(fsd_ctx *ctx)
     if (ctx->bro_alloc) return 0;
     const int64_t N = ctx->N, n11 = 11 * N;
     CK(hipMalloc(&ctx->d_lanV, sizeof(float) * (BRO_MMAX + 1) * n11));
-    CK(hipMalloc(&ctx->d_lanw, sizeof(float) * n11));
     CK(hipMalloc(&ctx->d_lany0, sizeof(float) * n11));
-    CK(hipMalloc(&ctx->d_lan_h, sizeof(double) * 256));
-    CK(hipHostMalloc((void **)&ctx->h_lan, sizeof(double) * 256, hipHostMallocDefault));
+    CK(hipHostMalloc((void **)&ctx->h_lan, sizeof(double) * (3 * BRO_MMAX + 2 * gs_part_doubles(n11, 1)),
+                     hipHostMallocDefault));
     CK(hipMalloc(&ctx->d_noise, sizeof(float) * (n11 + 6 * (int64_t)ctx->M + 12 * N)));
     CK(hipMalloc(&ctx->d_posp, sizeof(float4) * N));
     CK(hipMalloc(&ctx->d_rfd_rhs, sizeof(float) * 17 * N));
@@ -917,92 +905,71 @@ static int bro_noise(fsd_ctx *ctx, int stream, uint32_t timestep, const float **
 // one vector at a time until the relative change of y drops below tol or the
 // basis holds BRO_MMAX - 1 vectors.  Each new vector is reorthogonalised
 // against the whole basis (two classical Gram-Schmidt passes with FP64 dot
-// products); T_m^(1/2) e_1 is formed in FP64 on the host.
+// products); T_m^(1/2) e_1 is formed in FP64 on the host.  The device runs the
+// first m steps through: a step needs nothing from the host, which takes their
+// coefficients after the last (and drops the steps past an exhausted space).
 // op: 0 = real-space far-field mobility (11N), 1 = lubrication R_FU (6N).
 static int lanczos_sqrt(fsd_ctx *ctx, const float4 *pos, int op, const float *psi, float *y, int *m_io, float tol)
 {
     const int64_t n = (op == 0 ? 11 : 6) * (int64_t)ctx->N;
-    float *V = ctx->d_lanV, *w = ctx->d_lanw, *y0 = ctx->d_lany0;
-    double *dh = ctx->d_lan_h, *hh = ctx->h_lan;
+    float *V = ctx->d_lanV, *y0 = ctx->d_lany0;
+    // pinned: per step |w| and the two passes' h_jj; |psi| in the last step's place; partial sums
+    double *hh = ctx->h_lan, *hx = hh + 3 * (BRO_MMAX - 1), *hs = hh + 3 * BRO_MMAX;
     const double tol_beta = 1e-8;
-    auto fetch = [&](int cnt) -> int {
-        CK(hipMemcpyAsync(hh, dh, sizeof(double) * cnt, hipMemcpyDeviceToHost, ctx->stream));
-        CK(hipStreamSynchronize(ctx->stream));
-        return 0;
+    auto enqueue = [&](int j) -> int {
+        float *vj = V + (int64_t)j * n, *w = vj + n;
+        if (op == 0) RC(k_mobility(ctx, pos, vj, w, 1, nullptr));
+        else RC(k_rfu_apply(ctx, vj, w, nullptr, 1.0f));
+        return k_gs_orthonormalise(ctx, n, j + 1, V, w, 2, j, hh + 3 * j + 1, hh + 3 * j + 2, hh + 3 * j);
     };
-    auto apply = [&](const float *x, float *out) -> int {
-        if (op == 0) return k_mobility(ctx, pos, x, out, 1, nullptr);
-        return k_rfu_apply(ctx, x, out, nullptr, 1.0f);
+    std::vector<double> alpha, off;
+    bool breakdown = false;
+    // alpha_j and (unless the Krylov space is exhausted) off_j of a finished step
+    auto take = [&](int j) {
+        alpha.push_back(hh[3 * j + 1] + hh[3 * j + 2]);
+        if (hh[3 * j] < tol_beta) breakdown = true;
+        else off.push_back(hh[3 * j]);
     };
-    RC(k_nrm2(ctx, n, psi, dh));
-    RC(fetch(1));
-    const double xnorm = std::sqrt(hh[0]);
+    double xnorm = 0.0;
+    int nch = 0;
+    // out = xnorm V_m T_m^(1/2) e_1; with prev also the partials of |prev - out|^2 and |out|^2
+    auto combine = [&](int m, float *out, const float *prev) -> int {
+        std::vector<double> t(m);
+        tridiag_sqrt_e1(m, alpha.data(), off.data(), t.data());
+        for (double &c : t) c *= -xnorm;
+        return k_gs_combine(ctx, n, m, V, t.data(), nullptr, out, prev, prev ? hs : nullptr, &nch);
+    };
+    RC(k_gs_norm(ctx, n, psi, ctx->d_part[0], nullptr));
+    RC(k_gs_scale(ctx, n, psi, V, ctx->d_part[0], hx));
+    int m = std::max(1, std::min(*m_io, BRO_MMAX - 2));
+    for (int j = 0; j < m; ++j) RC(enqueue(j));
+    CK(hipStreamSynchronize(ctx->stream));
+    xnorm = *hx;
     if (xnorm == 0.0) {
         RC(k_fill(ctx, n, 0.f, y));
         return 0;
     }
-    RC(k_axpby(ctx, n, (float)(1.0 / xnorm), psi, 0.0f, nullptr, V));
-    std::vector<double> alpha, off;
-    bool breakdown = false;
-    // appends alpha_j and (unless the Krylov space is exhausted) off_j and v_{j+1}
-    auto step = [&](int j) -> int {
-        float *vj = V + (int64_t)j * n;
-        RC(apply(vj, w));
-        double a = 0.0;
-        for (int pass = 0; pass < 2; ++pass)
-            for (int c0 = 0; c0 <= j; c0 += 64) {
-                const int K = std::min(64, j + 1 - c0);
-                RC(k_multidot(ctx, n, K, V + (int64_t)c0 * n, n, w, dh));
-                RC(k_multi_axpy(ctx, n, K, V + (int64_t)c0 * n, n, dh, w));
-                if (j >= c0 && j < c0 + K) {
-                    RC(fetch(K));
-                    a += hh[j - c0];
-                }
-            }
-        RC(k_nrm2(ctx, n, w, dh));
-        RC(fetch(1));
-        const double b = std::sqrt(hh[0]);
-        alpha.push_back(a);
-        if (b < tol_beta) { breakdown = true; return 0; }
-        off.push_back(b);
-        RC(k_axpby(ctx, n, (float)(1.0 / b), w, 0.0f, nullptr, V + (int64_t)(j + 1) * n));
-        return 0;
-    };
-    // out = xnorm V_m T_m^(1/2) e_1
-    auto combine = [&](int m, float *out) -> int {
-        std::vector<double> t(m);
-        tridiag_sqrt_e1(m, alpha.data(), off.data(), t.data());
-        RC(k_fill(ctx, n, 0.f, out));
-        for (int c0 = 0; c0 < m; c0 += 64) {
-            const int K = std::min(64, m - c0);
-            for (int k = 0; k < K; ++k) hh[k] = -xnorm * t[c0 + k];
-            CK(hipMemcpyAsync(dh, hh, sizeof(double) * K, hipMemcpyHostToDevice, ctx->stream));
-            RC(k_multi_axpy(ctx, n, K, V + (int64_t)c0 * n, n, dh, out));
-            CK(hipStreamSynchronize(ctx->stream));
-        }
-        return 0;
-    };
-    int m = std::max(1, std::min(*m_io, BRO_MMAX - 2));
     for (int j = 0; j < m; ++j) {
-        RC(step(j));
+        take(j);
         if (breakdown) { m = j + 1; break; }
     }
-    RC(combine(m, y0));
+    // the results of successive m alternate between the two buffers
+    float *cur = y0, *next = y;
+    RC(combine(m, cur, nullptr));
     double err = 1.0;
-    bool wrote = false;
     while (!breakdown && err > tol && m < BRO_MMAX - 1) {
-        RC(step(m));
-        RC(combine(m + 1, y));
-        wrote = true;
-        RC(k_axpby(ctx, n, 1.0f, y0, -1.0f, y, y0));      // y0 <- y0 - y
-        RC(k_nrm2(ctx, n, y0, dh));
-        RC(k_nrm2(ctx, n, y, dh + 1));
-        RC(fetch(2));
-        err = std::sqrt(hh[0]) / std::max(std::sqrt(hh[1]), 1e-300);
-        RC(k_copy(ctx, n, y, y0));
+        RC(enqueue(m));
+        CK(hipStreamSynchronize(ctx->stream));
+        take(m);
+        RC(combine(m + 1, next, cur));
+        CK(hipStreamSynchronize(ctx->stream));
+        double d = 0.0, s = 0.0;
+        for (int c = 0; c < nch; ++c) { d += hs[2 * c]; s += hs[2 * c + 1]; }
+        err = std::sqrt(d) / std::max(std::sqrt(s), 1e-300);
+        std::swap(cur, next);
         ++m;
     }
-    if (!wrote) RC(k_copy(ctx, n, y0, y));
+    if (cur != y) RC(k_copy(ctx, n, cur, y));
     *m_io = m - 1;
     return 0;
 }
@@ -1077,14 +1044,15 @@ static int bro_rfd(fsd_ctx *ctx, const float4 *pos, uint32_t timestep, float *dr
 static int true_residual(fsd_ctx *ctx, const float4 *pos, const float *b, const float *x, float *out)
 {
     const int64_t n = 17 * (int64_t)ctx->N;
-    double *d_h = ctx->d_part + (int64_t)ctx->part_blocks * ctx->kmax;
+    double *hr = ctx->h_nrm, *hb = hr + gs_part_doubles(n, 1), nr = 0.0, nb = 0.0;
+    int nch = 0;
     RC(k_saddle_multiply(ctx, pos, x, ctx->d_t));
     RC(k_axpby(ctx, n, 1.0f, b, -1.0f, ctx->d_t, ctx->d_t));
-    RC(k_nrm2(ctx, n, ctx->d_t, d_h));
-    RC(k_nrm2(ctx, n, b, d_h + 1));
-    CK(hipMemcpyAsync(ctx->h_part, d_h, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    RC(k_gs_norm(ctx, n, ctx->d_t, hr, &nch));
+    RC(k_gs_norm(ctx, n, b, hb, nullptr));
     CK(hipStreamSynchronize(ctx->stream));
-    *out = (float)(std::sqrt(ctx->h_part[0]) / std::max(std::sqrt(ctx->h_part[1]), 1e-300));
+    for (int c = 0; c < nch; ++c) { nr += hr[c]; nb += hb[c]; }
+    *out = (float)(std::sqrt(nr) / std::max(std::sqrt(nb), 1e-300));
     return 0;
 }
 
