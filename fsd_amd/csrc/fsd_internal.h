@@ -12,6 +12,7 @@
 //               per permuted particle a dense 6x6 diagonal block and one 6x6
 //               block per lower neighbour (36 floats, row-major).
 #pragma once
+#include <functional>
 #include <hip/hip_runtime.h>
 #include <rocfft/rocfft.h>
 #include <stdint.h>
@@ -262,7 +263,9 @@ struct fsd_ctx {
     int *d_porig = nullptr;       // 3 ints per slot: stencil origin (unwrapped)
     int *d_ocell = nullptr;       // N: grid cell of each slot's (wrapped) stencil origin
     int *d_olist = nullptr;       // N: slots sorted by origin cell, ascending inside a cell
-    int *d_ocount = nullptr;      // M: particles per origin cell (scratch)
+    int *d_ocount = nullptr;      // M: particles per origin cell (scratch, zero between set-ups)
+    int *d_orank = nullptr;       // N: place among the slots of the same origin cell, in arrival order
+    bool ocount_zero = false;     // the counts are zero (or will be, in stream order)
     int *d_ostart = nullptr;      // M+1: first position of each origin cell in d_olist
     int *d_scan_tmp = nullptr;    // chunk totals of the multi-workgroup scan
     int contract_lds = 0;         // LDS bytes of the tile contraction (0: per-particle contraction)
@@ -336,6 +339,7 @@ struct fsd_ctx {
     double *d_part[2] = {nullptr, nullptr};     // partial sums of the Gram-Schmidt kernels (in turn)
     double *h_part = nullptr;     // pinned: Hessenberg columns
     double *h_nrm = nullptr;      // pinned: partial sums of norms the host finishes
+    hipEvent_t chk_ev = nullptr;  // the list's check or the lubrication pairs' counts
     hipEvent_t gm_ev[2] = {nullptr, nullptr};   // readbacks of the Hessenberg columns (two slots)
     int kmax = 64;                // restart + 1, at least 64
     float *d_rhs = nullptr, *d_sol = nullptr;
@@ -398,7 +402,11 @@ void prof_host(fsd_ctx *ctx, int slot, double ms);
 // kernel groups (launchers live with their kernels)
 int k_build_nlist(fsd_ctx *ctx, const float4 *pos);
 int k_update_nlist(fsd_ctx *ctx, const float4 *pos, bool *rebuilt);
+int k_nlist_check(fsd_ctx *ctx, const float4 *pos);                     // k_update_nlist in two parts
+int k_nlist_settle(fsd_ctx *ctx, const float4 *pos, bool *rebuilt);
 int k_build_lub_pairs(fsd_ctx *ctx, const float4 *pos);
+int k_lub_pairs_launch(fsd_ctx *ctx, const float4 *pos);                // k_build_lub_pairs in two parts
+int k_lub_pairs_settle(fsd_ctx *ctx, const float4 *pos);
 int k_lub_pairs_into(fsd_ctx *ctx, const float4 *pos, int maxlub, int *lub_n, int *lub_j, float4 *lub_a,
                      float4 *lub_b, float *lub_self, int *overflow);
 int k_rfu_apply_with(fsd_ctx *ctx, const float *U, float *F, const int *lub_n, const int *lub_j, const float4 *lub_a,
@@ -408,13 +416,18 @@ int k_rfu_apply(fsd_ctx *ctx, const float *U, float *F, const float *xF, float s
 int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F);
 int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S);
 int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S);
-int k_setup_spread(fsd_ctx *ctx, const float4 *pos);
+int k_setup_spread(fsd_ctx *ctx, const float4 *pos, const float *gF = nullptr);   // gF: also its records
 int k_contract_lds(fsd_ctx *ctx);
 int k_real_init(fsd_ctx *ctx);       // LDS limits of the real-space kernels; nonzero on failure
+#define SCAN_CHUNK 4096
+#define SCAN_SELF 1024         // chunks whose offsets a workgroup sums for itself
 int scan_excl_chunks(int n);
+int scan_chunked(fsd_ctx *ctx, const int *in, int *out, int n, int *tmp, bool *totals);
 int k_gridk(fsd_ctx *ctx);
 float k_twopi(const fsd_ctx *ctx);
-int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int parts, const float *addU);
+// before_real (may be null): called once, between the wave part and the real-space sum; it may rebuild the list
+int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int parts, const float *addU,
+               const std::function<int(bool *rebuilt)> *before_real = nullptr);
 int k_prune(fsd_ctx *ctx, const float4 *pos);
 int k_build_blocks(fsd_ctx *ctx, const float4 *pos);
 int k_ichol(fsd_ctx *ctx, float lambda, int *failed);

@@ -44,6 +44,27 @@ int k_gridk(fsd_ctx *ctx)
     return 0;
 }
 
+// ------------------------------------------------- force + couplet records
+// per slot one 64-byte record (half a cache line): position, F (3), the stresslet S (xx, xy, xz, yz, yy)
+// and w = -T/2, the couplet's antisymmetric part (Mobility_TS2C_kernel, Helper_Mobility.cu:294-336)
+__device__ __forceinline__ void write_record(const float *gF, int N, int id, float4 p, float4 *r)
+{
+    const float *f = gF + 6 * (int64_t)id;
+    const float *s = gF + 6 * (int64_t)N + 5 * (int64_t)id;
+    r[0] = make_float4(p.x, p.y, p.z, f[0]);
+    r[1] = make_float4(f[1], f[2], s[0], s[1]);
+    r[2] = make_float4(s[2], s[3], s[4], -0.5f * f[3]);
+    r[3] = make_float4(-0.5f * f[4], -0.5f * f[5], 0.f, 0.f);
+}
+
+__global__ void fc_records_kernel(const float *gF, const float4 *pos, const int *order, int N, float4 *rec)
+{
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= N) return;
+    const int id = order ? order[i] : i;
+    write_record(gF, N, id, pos[id], rec + 4 * (int64_t)i);
+}
+
 // ------------------------------------------------- spreading set-up (per step)
 // Stencil origin exactly as Mobility.cu:203-225 (float fraction, truncation);
 // particles are then counting-sorted by the grid cell of their (wrapped)
@@ -52,8 +73,14 @@ int k_gridk(fsd_ctx *ctx)
 //
 // Particles stand by slot, their place in the neighbour list's cell order: what the wave part and
 // the real-space sum read of a particle's surroundings lies close together.
+//
+// Four launches (origins, counts and the product's records; scan within chunks; scatter; order and
+// starts), each a few dependent loads long, so their number is what they cost (eight took 27 us at
+// N = 4072): the counting atomics give each particle its place in its cell, the last launch leaves
+// the counts zero, and the chunks' offsets are summed where they are used.
 __global__ void stencil_origin_kernel(const float4 *pos, const int *order, int N, BoxF b, int Nx, int Ny, int Nz,
-                                      int P, float4 *spos, int *orig, int *ocell, int *ocount)
+                                      int P, const float *gF, float4 *rec, float4 *spos, int *orig, int *ocell,
+                                      int *orank, int *ocount)
 {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -72,22 +99,69 @@ __global__ void stencil_origin_kernel(const float4 *pos, const int *order, int N
     int wx = ((ox % Nx) + Nx) % Nx, wy = ((oy % Ny) + Ny) % Ny, wz = ((oz % Nz) + Nz) % Nz;
     const int c = (wx * Ny + wy) * Nz + wz;
     ocell[i] = c;
-    atomicAdd(&ocount[c], 1);
+    orank[i] = atomicAdd(&ocount[c], 1);
+    if (gF) write_record(gF, N, id, p, rec + 4 * (int64_t)i);
 }
 
-__global__ void ocell_scatter_kernel(const int *ocell, int N, const int *start, int *fill, int *list)
+// offset of the chunks before chunk c (part: totals, or the offsets themselves), for the whole block
+__device__ __forceinline__ int chunk_offset(const int *part, bool totals, int c)
 {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int c = ocell[i];
-    list[start[c] + atomicAdd(&fill[c], 1)] = i;
+    if (!totals) return part[c];
+    __shared__ int s_w[4];
+    int s = 0;
+    for (int q = threadIdx.x; q < c; q += 256) s += part[q];
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = s;
+    __syncthreads();
+    return s_w[0] + s_w[1] + s_w[2] + s_w[3];
 }
 
-__global__ void ocell_sort_kernel(const int *start, int ncell, int *list)
+__global__ void __launch_bounds__(256) ocell_scatter_kernel(const int *ocell, const int *orank, int N, const int *start,
+                                                            const int *part, int nc, bool totals, int *list)
 {
-    int c = blockIdx.x * blockDim.x + threadIdx.x;
+    // offsets of all chunks (at most SCAN_SELF when they are not given): four to a thread
+    __shared__ int s_off[SCAN_SELF], s_w[4];
+    const int lt = threadIdx.x, i = blockIdx.x * blockDim.x + lt;
+    const int c = i < N ? ocell[i] : 0, r = i < N ? orank[i] : 0;
+    const int st = start[c];
+    if (totals) {
+        int v[4], s = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = 4 * lt + k < nc ? part[4 * lt + k] : 0;
+            s += v[k];
+        }
+        int inc = s;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(inc, o, 64);
+            if ((lt & 63) >= o) inc += y;
+        }
+        if ((lt & 63) == 63) s_w[lt >> 6] = inc;
+        __syncthreads();
+        int pre = inc - s;
+        for (int w = 0; w < (lt >> 6); ++w) pre += s_w[w];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            s_off[4 * lt + k] = pre;
+            pre += v[k];
+        }
+        __syncthreads();
+    }
+    if (i < N) list[st + (totals ? s_off[c / SCAN_CHUNK] : part[c / SCAN_CHUNK]) + r] = i;
+}
+
+// orders the cells' slots, completes their starts and clears the counts
+__global__ void __launch_bounds__(256) ocell_sort_kernel(int *start, int *count, const int *part, bool totals,
+                                                         int ncell, int N, int *list)
+{
+    static_assert(SCAN_CHUNK % 256 == 0, "a block's cells lie in one chunk");
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    const int n = c < ncell ? count[c] : 0, s0 = c < ncell ? start[c] : 0;
+    const int s = s0 + chunk_offset(part, totals, blockIdx.x * 256 / SCAN_CHUNK), e = s + n;
     if (c >= ncell) return;
-    const int s = start[c], e = start[c + 1];
+    start[c] = s;
+    count[c] = 0;
+    if (c == ncell - 1) start[ncell] = N;
     for (int a = s + 1; a < e; ++a) {
         int key = list[a], q = a - 1;
         while (q >= s && list[q] > key) { list[q + 1] = list[q]; --q; }
@@ -95,48 +169,32 @@ __global__ void ocell_sort_kernel(const int *start, int ncell, int *list)
     }
 }
 
-int scan_excl_large(fsd_ctx *ctx, const int *in, int *out, int n, int *tmp);
-
 // the order of the slots
 static const int *slot_order(const fsd_ctx *ctx)
 {
     return (ctx->nlist_valid && ctx->use_cells) ? ctx->d_cell_list : nullptr;
 }
 
-int k_setup_spread(fsd_ctx *ctx, const float4 *pos)
+int k_setup_spread(fsd_ctx *ctx, const float4 *pos, const float *gF)
 {
     const int N = ctx->N, M = ctx->M;
-    FSD_HIP(hipMemsetAsync(ctx->d_ocount, 0, sizeof(int) * M, ctx->stream));
-    hipLaunchKernelGGL(stencil_origin_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, pos,
-                       slot_order(ctx), N, ctx->box, ctx->pse.Nx, ctx->pse.Ny, ctx->pse.Nz, ctx->pse.P, ctx->d_spos, ctx->d_porig, ctx->d_ocell, ctx->d_ocount);
-    if (scan_excl_large(ctx, ctx->d_ocount, ctx->d_ostart, M, ctx->d_scan_tmp)) return FSD_E_HIP;
-    FSD_HIP(hipMemsetAsync(ctx->d_ocount, 0, sizeof(int) * M, ctx->stream));
-    hipLaunchKernelGGL(ocell_scatter_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, ctx->d_ocell, N,
-                       ctx->d_ostart, ctx->d_ocount, ctx->d_olist);
-    hipLaunchKernelGGL(ocell_sort_kernel, dim3(nblk(M, 256)), dim3(256), 0, ctx->stream, ctx->d_ostart, M,
-                       ctx->d_olist);
+    if (!ctx->ocount_zero) FSD_HIP(hipMemsetAsync(ctx->d_ocount, 0, sizeof(int) * M, ctx->stream));
+    ctx->ocount_zero = false;
+    hipLaunchKernelGGL(stencil_origin_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, pos, slot_order(ctx), N,
+                       ctx->box, ctx->pse.Nx, ctx->pse.Ny, ctx->pse.Nz, ctx->pse.P, gF, ctx->d_rec, ctx->d_spos,
+                       ctx->d_porig, ctx->d_ocell, ctx->d_orank, ctx->d_ocount);
+    bool totals;
+    const int *part = ctx->d_scan_tmp, nc = scan_excl_chunks(M);
+    if (scan_chunked(ctx, ctx->d_ocount, ctx->d_ostart, M, ctx->d_scan_tmp, &totals)) return FSD_E_HIP;
+    hipLaunchKernelGGL(ocell_scatter_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, ctx->d_ocell, ctx->d_orank,
+                       N, ctx->d_ostart, part, nc, totals, ctx->d_olist);
+    hipLaunchKernelGGL(ocell_sort_kernel, dim3(nblk(M, 256)), dim3(256), 0, ctx->stream, ctx->d_ostart, ctx->d_ocount,
+                       part, totals, M, N, ctx->d_olist);
     FSD_HIP(hipGetLastError());
+    ctx->ocount_zero = true;
     ctx->spread_valid = true;
     ctx->spread_pos = (const float *)pos;
     return 0;
-}
-
-// ------------------------------------------------- force + couplet records
-// per slot one 64-byte record (half a cache line): position, F (3), the stresslet S (xx, xy, xz, yz, yy)
-// and w = -T/2, the couplet's antisymmetric part (Mobility_TS2C_kernel, Helper_Mobility.cu:294-336)
-__global__ void fc_records_kernel(const float *gF, const float4 *pos, const int *order, int N, float4 *rec)
-{
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= N) return;
-    const int id = order ? order[i] : i;
-    const float *f = gF + 6 * (int64_t)id;
-    const float *s = gF + 6 * (int64_t)N + 5 * (int64_t)id;
-    const float4 p = pos[id];
-    float4 *r = rec + 4 * (int64_t)i;
-    r[0] = make_float4(p.x, p.y, p.z, f[0]);
-    r[1] = make_float4(f[1], f[2], s[0], s[1]);
-    r[2] = make_float4(s[2], s[3], s[4], -0.5f * f[3]);
-    r[3] = make_float4(-0.5f * f[4], -0.5f * f[5], 0.f, 0.f);
 }
 
 // F and the couplet's stored components XX XY XZ YZ YY YX ZX ZY of a record: the 11 grid fields
@@ -1150,23 +1208,27 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
 
 // ------------------------------------------------------------ driver
 // gU = M gF (+ addU on the first 6N rows); parts: 1 real, 2 wave, 3 both
-int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int parts, const float *addU)
+int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int parts, const float *addU,
+               const std::function<int(bool *)> *before_real)
 {
     const int N = ctx->N;
     const fsd_pse_info &ps = ctx->pse;
     float4 *rec = ctx->d_rec;
     const int *order = slot_order(ctx);
-    hipLaunchKernelGGL(fc_records_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, gF, pos, order, N,
-                       rec);
+    auto records = [&]() {
+        hipLaunchKernelGGL(fc_records_kernel, dim3(nblk(N, 256)), dim3(256), 0, ctx->stream, gF, pos, order, N, rec);
+    };
+    if ((parts & 2) && (!ctx->spread_valid || ctx->spread_pos != (const float *)pos)) {
+        const int rc = k_setup_spread(ctx, pos, gF);
+        if (rc) return rc;
+    } else {
+        records();
+    }
     FSD_HIP(hipGetLastError());
     const SpreadGeom g = spread_geom(ctx);
     const int64_t Mp = (int64_t)ps.Nx * ps.Ny * g.pz;   // grid field stride
     const float *wave = nullptr;
     if (parts & 2) {
-        if (!ctx->spread_valid || ctx->spread_pos != (const float *)pos) {
-            int rc = k_setup_spread(ctx, pos);
-            if (rc) return rc;
-        }
         hipEvent_t ev;
         prof_begin(ctx, PROF_SPREAD, &ev);
         if (ctx->tile == 8 && ctx->pse.P == 6 && ctx->tune.spread == 0)
@@ -1208,6 +1270,15 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
         const int rcw = k_wave_contract(ctx, pos, fx);
         if (rcw) return rcw;
         wave = ctx->d_wave;
+    }
+    if (before_real) {
+        bool rebuilt = false;
+        const int rc = (*before_real)(&rebuilt);
+        if (rc) return rc;
+        if (rebuilt) {
+            order = slot_order(ctx);
+            records();
+        }
     }
     RealParams rp;
     rp.b = ctx->box; rp.rcut = ps.rcut; rp.dr = 0.001f; rp.self_x = ps.self_x; rp.self_y = ps.self_y;

@@ -51,9 +51,7 @@ int scan_excl(fsd_ctx *ctx, const int *in, int *out, int n)
 }
 
 // multi-workgroup exclusive scan for long arrays: each workgroup scans
-// SCAN_CHUNK elements (4 per thread) and records its total; the totals are
-// scanned by one workgroup; a third pass adds each chunk's offset.
-#define SCAN_CHUNK 4096
+// SCAN_CHUNK elements (4 per thread) and records its total
 __global__ void __launch_bounds__(1024) scan_chunks_kernel(const int *in, int *out, int n, int *part)
 {
     __shared__ int wsum[16];
@@ -92,24 +90,18 @@ __global__ void __launch_bounds__(1024) scan_chunks_kernel(const int *in, int *o
     if (tid == 0) part[blockIdx.x] = wsum[15];
 }
 
-__global__ void scan_add_kernel(int *out, int n, const int *part_scan, int nchunks)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] += part_scan[i / SCAN_CHUNK];
-    if (i == 0) out[n] = part_scan[nchunks];
-}
-
 int scan_excl_chunks(int n) { return (n + SCAN_CHUNK - 1) / SCAN_CHUNK; }
 
-// out[0..n] = exclusive scan of in[0..n); tmp holds 2 (chunks + 1) ints
-int scan_excl_large(fsd_ctx *ctx, const int *in, int *out, int n, int *tmp)
+// The first two passes for a caller whose next kernels add the chunks' offsets themselves: out[i] = scan of
+// in within i's chunk of SCAN_CHUNK, tmp[c] the offset of chunk c from chunk block to chunk block.  Up to
+// SCAN_SELF chunks tmp holds their totals instead (*totals), which a workgroup sums as it needs them.
+int scan_chunked(fsd_ctx *ctx, const int *in, int *out, int n, int *tmp, bool *totals)
 {
     const int nc = scan_excl_chunks(n);
-    if (nc <= 1) return scan_excl(ctx, in, out, n);
-    int *part = tmp, *part_scan = tmp + nc + 1;
+    *totals = nc <= SCAN_SELF;
+    int *part = *totals ? tmp : tmp + nc + 1;
     hipLaunchKernelGGL(scan_chunks_kernel, dim3(nc), dim3(1024), 0, ctx->stream, in, out, n, part);
-    hipLaunchKernelGGL(scan_excl_kernel, dim3(1), dim3(1024), 0, ctx->stream, part, part_scan, nc);
-    hipLaunchKernelGGL(scan_add_kernel, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, out, n, part_scan, nc);
+    if (!*totals) hipLaunchKernelGGL(scan_excl_kernel, dim3(1), dim3(1024), 0, ctx->stream, part, tmp, nc);
     FSD_HIP(hipGetLastError());
     return 0;
 }
@@ -264,24 +256,39 @@ __global__ void max_disp_kernel(const float4 *pos, const float4 *last, int N, Bo
 
 // the list is kept while no particle has moved r_buff / 2 since it was built (the buffer then
 // still holds every pair within rcut), rebuilt otherwise or when the box changed
-int k_update_nlist(fsd_ctx *ctx, const float4 *pos, bool *rebuilt)
+//
+// In two parts, so that a caller can queue what does not need the list between them: the check's
+// launch, and the wait for its answer (with the rebuild).  At most one check is in flight.
+int k_nlist_check(fsd_ctx *ctx, const float4 *pos)
+{
+    if (!ctx->nlist_valid) return 0;
+    const float half = 0.5f * ctx->p.r_buff;
+    // the kernel stores into the pinned host flag itself (a store per moved particle, none in the
+    // usual call): one launch where clearing, copying and reading a device flag were three.
+    // Nothing of this context is in flight on the flag: every call drains the stream.
+    *(volatile int *)(ctx->h_flags + 6) = 0;
+    hipLaunchKernelGGL(max_disp_kernel, dim3(nblk(ctx->N, 256)), dim3(256), 0, ctx->stream, pos, ctx->d_pos_last,
+                       ctx->N, ctx->box, half * half, ctx->h_flags + 6);
+    FSD_HIP(hipGetLastError());
+    FSD_HIP(hipEventRecord(ctx->chk_ev, ctx->stream));
+    return 0;
+}
+
+int k_nlist_settle(fsd_ctx *ctx, const float4 *pos, bool *rebuilt)
 {
     *rebuilt = false;
     if (ctx->nlist_valid) {
-        const float half = 0.5f * ctx->p.r_buff;
-        // the kernel stores into the pinned host flag itself (a store per moved particle, none in the
-        // usual call): one launch where clearing, copying and reading a device flag were three.
-        // Nothing of this context is in flight on the flag: every call drains the stream.
-        volatile int *moved = ctx->h_flags + 6;
-        *moved = 0;
-        hipLaunchKernelGGL(max_disp_kernel, dim3(nblk(ctx->N, 256)), dim3(256), 0, ctx->stream, pos, ctx->d_pos_last,
-                           ctx->N, ctx->box, half * half, ctx->h_flags + 6);
-        FSD_HIP(hipGetLastError());
-        FSD_HIP(hipStreamSynchronize(ctx->stream));
-        if (!*moved) return 0;
+        FSD_HIP(hipEventSynchronize(ctx->chk_ev));
+        if (!*(volatile int *)(ctx->h_flags + 6)) return 0;
     }
     *rebuilt = true;
     return k_build_nlist(ctx, pos);
+}
+
+int k_update_nlist(fsd_ctx *ctx, const float4 *pos, bool *rebuilt)
+{
+    const int rc = k_nlist_check(ctx, pos);
+    return rc ? rc : k_nlist_settle(ctx, pos, rebuilt);
 }
 
 int k_build_nlist(fsd_ctx *ctx, const float4 *pos)
@@ -410,35 +417,53 @@ __global__ void __launch_bounds__(PGB) lub_pairs_kernel(const float4 *pos, int N
     pg_block_counts(s_cnt, maxlub, overflow, total);
 }
 
-int k_build_lub_pairs(fsd_ctx *ctx, const float4 *pos)
+// in two parts like the list's check: the launch, and the wait for the counts (with a second attempt at a
+// larger capacity)
+int k_lub_pairs_launch(fsd_ctx *ctx, const float4 *pos)
 {
     const int N = ctx->N;
     if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     const float rl2 = ctx->p.rlub * ctx->p.rlub;
-    for (int attempt = 0; attempt < 2; ++attempt) {
-        // flags 8 (most pairs of a particle, when more than maxlub) and 9 (pairs in all)
-        FSD_HIP(hipMemsetAsync(ctx->d_flags + 8, 0, 2 * sizeof(int), ctx->stream));
-        hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
-                           ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, rl2, ctx->maxlub, ctx->d_lub_n, ctx->d_lub_j,
-                           ctx->d_lub_a, ctx->d_lub_b, ctx->d_lub_self, ctx->d_flags + 8, ctx->d_flags + 9,
-                           cell_order(ctx));
-        FSD_HIP(hipGetLastError());
-        FSD_HIP(hipMemcpyAsync(ctx->h_flags + 8, ctx->d_flags + 8, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        FSD_HIP(hipStreamSynchronize(ctx->stream));
+    // flags 8 (most pairs of a particle, when more than maxlub) and 9 (pairs in all)
+    FSD_HIP(hipMemsetAsync(ctx->d_flags + 8, 0, 2 * sizeof(int), ctx->stream));
+    hipLaunchKernelGGL(lub_pairs_kernel, dim3(nblk(N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, N, ctx->box,
+                       ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, rl2, ctx->maxlub, ctx->d_lub_n, ctx->d_lub_j,
+                       ctx->d_lub_a, ctx->d_lub_b, ctx->d_lub_self, ctx->d_flags + 8, ctx->d_flags + 9,
+                       cell_order(ctx));
+    FSD_HIP(hipGetLastError());
+    FSD_HIP(hipMemcpyAsync(ctx->h_flags + 8, ctx->d_flags + 8, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    FSD_HIP(hipEventRecord(ctx->chk_ev, ctx->stream));
+    return 0;
+}
+
+int k_lub_pairs_settle(fsd_ctx *ctx, const float4 *pos)
+{
+    const int N = ctx->N;
+    for (int attempt = 0;; ++attempt) {
+        FSD_HIP(hipEventSynchronize(ctx->chk_ev));
         ctx->lub_total = ctx->h_flags[9];
         int need = ctx->h_flags[8];
         if (need == 0) break;
         if (attempt == 1) { ctx->err = "lubrication pair capacity exceeded"; return FSD_E_CAPACITY; }
+        FSD_HIP(hipStreamSynchronize(ctx->stream));
         int nm = ((need + 16) / 16) * 16 + 16;
         FSD_HIP(hipFree(ctx->d_lub_j)); FSD_HIP(hipFree(ctx->d_lub_a)); FSD_HIP(hipFree(ctx->d_lub_b));
         FSD_HIP(hipMalloc(&ctx->d_lub_j, sizeof(int) * (size_t)N * nm));
         FSD_HIP(hipMalloc(&ctx->d_lub_a, sizeof(float4) * (size_t)N * nm));
         FSD_HIP(hipMalloc(&ctx->d_lub_b, sizeof(float4) * (size_t)N * nm));
         ctx->maxlub = nm;
+        const int rc = k_lub_pairs_launch(ctx, pos);
+        if (rc) return rc;
     }
     ctx->lub_valid = true;
     return 0;
+}
+
+int k_build_lub_pairs(fsd_ctx *ctx, const float4 *pos)
+{
+    const int rc = k_lub_pairs_launch(ctx, pos);
+    return rc ? rc : k_lub_pairs_settle(ctx, pos);
 }
 
 // Pair records into caller-provided buffers (capacity maxlub per particle); the

@@ -244,6 +244,7 @@ static int alloc_all(fsd_ctx *ctx)
     CK(hipMalloc(&ctx->d_ocell, sizeof(int) * N));
     CK(hipMalloc(&ctx->d_olist, sizeof(int) * N));
     CK(hipMalloc(&ctx->d_ocount, sizeof(int) * (size_t)ctx->M));
+    CK(hipMalloc(&ctx->d_orank, sizeof(int) * N));
     CK(hipMalloc(&ctx->d_ostart, sizeof(int) * ((size_t)ctx->M + 1)));
     CK(hipMalloc(&ctx->d_scan_tmp, sizeof(int) * 2 * (scan_excl_chunks(ctx->M) + 1)));
     if (ctx->tile + ps.P - 1 > 32) { ctx->err = "spreading support P too large for the tile halo"; return FSD_E_PARAM; }
@@ -325,7 +326,7 @@ static int alloc_all(fsd_ctx *ctx)
     // kernels while the host takes the one before); two norms' partial sums
     CK(hipHostMalloc((void **)&ctx->h_part, sizeof(double) * 2 * (2 * ctx->kmax + 1), hipHostMallocDefault));
     CK(hipHostMalloc((void **)&ctx->h_nrm, sizeof(double) * 2 * gs_part_doubles(n17, 1), hipHostMallocDefault));
-    for (hipEvent_t *e : {&ctx->gm_ev[0], &ctx->gm_ev[1]}) CK(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    for (hipEvent_t *e : {&ctx->gm_ev[0], &ctx->gm_ev[1], &ctx->chk_ev}) CK(hipEventCreateWithFlags(e, hipEventDisableTiming));
     CK(hipMalloc(&ctx->d_rhs, sizeof(float) * n17));
     CK(hipMalloc(&ctx->d_sol, sizeof(float) * n17));
     CK(hipMemset(ctx->d_sol, 0, sizeof(float) * n17));
@@ -358,7 +359,7 @@ static void free_all(fsd_ctx *ctx)
     void *ptrs[] = {ctx->d_nneigh, ctx->d_nlist, ctx->d_snn, ctx->d_nslot, ctx->d_spos, ctx->d_cell_of, ctx->d_cell_count, ctx->d_cell_start,
                     ctx->d_cell_list, ctx->d_flags, ctx->d_pos_last, ctx->d_lub_n, ctx->d_lub_j, ctx->d_lub_a, ctx->d_lub_b,
                     ctx->d_lub_self, ctx->d_grid, ctx->d_spec, ctx->d_gridk, ctx->d_fftwork, ctx->d_porig,
-                    ctx->d_ocell, ctx->d_olist, ctx->d_ocount, ctx->d_ostart, ctx->d_scan_tmp, ctx->d_wave, ctx->d_rec,
+                    ctx->d_ocell, ctx->d_olist, ctx->d_ocount, ctx->d_orank, ctx->d_ostart, ctx->d_scan_tmp, ctx->d_wave, ctx->d_rec,
                     ctx->d_ewald, ctx->d_res_dist, ctx->d_res_vals, ctx->d_pn, ctx->d_plist, ctx->d_pless,
                     ctx->d_perm, ctx->d_iperm, ctx->d_lrow, ctx->d_urow, ctx->d_lcol, ctx->d_ucol, ctx->d_upos,
                     ctx->d_Ablk, ctx->d_Lblk, ctx->d_Adiag, ctx->d_Ldiag, ctx->d_lev_f, ctx->d_lev_b, ctx->d_tmp6a,
@@ -376,7 +377,7 @@ static void free_all(fsd_ctx *ctx)
     if (ctx->h_flags) hipHostFree(ctx->h_flags);
     if (ctx->h_part) hipHostFree(ctx->h_part);
     if (ctx->h_nrm) hipHostFree(ctx->h_nrm);
-    for (hipEvent_t e : ctx->gm_ev)
+    for (hipEvent_t e : {ctx->gm_ev[0], ctx->gm_ev[1], ctx->chk_ev})
         if (e) hipEventDestroy(e);
     if (ctx->h_lan) hipHostFree(ctx->h_lan);
     if (ctx->plan_fwd) rocfft_plan_destroy(ctx->plan_fwd);
@@ -1360,9 +1361,17 @@ int fsd_rse(fsd_ctx *ctx, const float *d_pos4, float shear_rate, const float *d_
 
 int fsd_mobility(fsd_ctx *ctx, const float *d_pos4, const float *d_gF11, float *d_gU11, int32_t parts)
 {
-    RC(current_nlist(ctx, reinterpret_cast<const float4 *>(d_pos4)));
+    const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
+    if (!ctx->nlist_valid) { ctx->err = "neighbour list not built"; return FSD_E_STATE; }
     ctx->spread_valid = false;
-    RC(k_mobility(ctx, reinterpret_cast<const float4 *>(d_pos4), d_gF11, d_gU11, parts, nullptr));
+    // the host waits for the list's check with the wave part in the queue, which does not need the list
+    RC(k_nlist_check(ctx, pos));
+    const std::function<int(bool *)> settle = [&](bool *rebuilt) {
+        RC(k_nlist_settle(ctx, pos, rebuilt));
+        ctx->nlist_builds += *rebuilt;
+        return 0;
+    };
+    RC(k_mobility(ctx, pos, d_gF11, d_gU11, parts, nullptr, &settle));
     CK(hipStreamSynchronize(ctx->stream));
     return 0;
 }
@@ -1540,9 +1549,20 @@ int fsd_get_precond(fsd_ctx *ctx, int32_t *h_pn, int32_t *h_plist, int64_t plist
 int fsd_saddle_multiply(fsd_ctx *ctx, const float *d_pos4, const float *d_x17, float *d_y17)
 {
     const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
-    RC(ensure_lub(ctx, pos));
+    if (!ctx->nlist_valid) { ctx->err = "neighbour list not built"; return FSD_E_STATE; }
+    if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
     ctx->spread_valid = false;
-    RC(k_saddle_multiply(ctx, pos, d_x17, d_y17));
+    // like fsd_mobility; the lubrication pairs' counts come in under the real-space sum
+    RC(k_nlist_check(ctx, pos));
+    const std::function<int(bool *)> settle = [&](bool *rebuilt) {
+        RC(k_nlist_settle(ctx, pos, rebuilt));
+        ctx->nlist_builds += *rebuilt;
+        return k_lub_pairs_launch(ctx, pos);
+    };
+    const int64_t n11 = 11 * (int64_t)ctx->N;
+    RC(k_mobility(ctx, pos, d_x17, d_y17, 3, d_x17 + n11, &settle));
+    RC(k_lub_pairs_settle(ctx, pos));
+    RC(k_rfu_apply(ctx, d_x17 + n11, d_y17 + n11, d_x17, -1.0f));
     CK(hipStreamSynchronize(ctx->stream));
     return 0;
 }
