@@ -339,6 +339,7 @@ struct fsd_ctx {
     double *d_part[2] = {nullptr, nullptr};     // partial sums of the Gram-Schmidt kernels (in turn)
     double *h_part = nullptr;     // pinned: Hessenberg columns
     double *h_nrm = nullptr;      // pinned: partial sums of norms the host finishes
+    int chk_seq = 0;              // number of the last check (d_flags[10]: of the last that found a move)
     hipEvent_t chk_ev = nullptr;  // the list's check or the lubrication pairs' counts
     hipEvent_t gm_ev[2] = {nullptr, nullptr};   // readbacks of the Hessenberg columns (two slots)
     int kmax = 64;                // restart + 1, at least 64
@@ -413,9 +414,10 @@ int k_rfu_apply_with(fsd_ctx *ctx, const float *U, float *F, const int *lub_n, c
                      const float4 *lub_b, const float *lub_self, int maxlub);
 int noalloc_init_device();   // k_noalloc.hip: device address of the static scratch, once per device
 int k_rfu_apply(fsd_ctx *ctx, const float *U, float *F, const float *xF, float sign_out);
-int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F);
-int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S);
-int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S);
+// guarded: queued behind a k_nlist_check that is not settled; nothing is added if it finds the list too old
+int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F, bool guarded = false);
+int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S, bool guarded = false);
+int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S, bool guarded = false);
 int k_setup_spread(fsd_ctx *ctx, const float4 *pos, const float *gF = nullptr);   // gF: also its records
 int k_contract_lds(fsd_ctx *ctx);
 int k_real_init(fsd_ctx *ctx);       // LDS limits of the real-space kernels; nonzero on failure

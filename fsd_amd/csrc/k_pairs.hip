@@ -244,21 +244,26 @@ __global__ void __launch_bounds__(PGB) nlist_allpairs_kernel(const float4 *pos, 
 
 // NeighborList::distanceCheck of HOOMD: some particle has moved at least r_buff / 2 (minimum
 // image) since the list was built
-__global__ void max_disp_kernel(const float4 *pos, const float4 *last, int N, BoxF b, float lim2, int *flag)
+__global__ void max_disp_kernel(const float4 *pos, const float4 *last, int N, BoxF b, float lim2, int *flag, int *dflag,
+                                int seq)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const float4 p = pos[i], q = last[i];
     float dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
     box_min_image(b, dx, dy, dz);
-    if (dist2_nc(dx, dy, dz) >= lim2) *flag = 1;
+    if (dist2_nc(dx, dy, dz) >= lim2) {
+        *flag = 1;
+        *dflag = seq;
+    }
 }
 
 // the list is kept while no particle has moved r_buff / 2 since it was built (the buffer then
 // still holds every pair within rcut), rebuilt otherwise or when the box changed
 //
 // In two parts, so that a caller can queue what does not need the list between them: the check's
-// launch, and the wait for its answer (with the rebuild).  At most one check is in flight.
+// launch, and the wait for its answer (with the rebuild).  At most one check is in flight; its number in a
+// device flag tells the kernels queued behind it the answer.
 int k_nlist_check(fsd_ctx *ctx, const float4 *pos)
 {
     if (!ctx->nlist_valid) return 0;
@@ -268,7 +273,7 @@ int k_nlist_check(fsd_ctx *ctx, const float4 *pos)
     // Nothing of this context is in flight on the flag: every call drains the stream.
     *(volatile int *)(ctx->h_flags + 6) = 0;
     hipLaunchKernelGGL(max_disp_kernel, dim3(nblk(ctx->N, 256)), dim3(256), 0, ctx->stream, pos, ctx->d_pos_last,
-                       ctx->N, ctx->box, half * half, ctx->h_flags + 6);
+                       ctx->N, ctx->box, half * half, ctx->h_flags + 6, ctx->d_flags + 10, ++ctx->chk_seq);
     FSD_HIP(hipGetLastError());
     FSD_HIP(hipEventRecord(ctx->chk_ev, ctx->stream));
     return 0;
@@ -600,15 +605,28 @@ __device__ __forceinline__ void pg_add(float *o, int lane, const float *v, float
     if (lane < M) o[lane] += sign * f;
 }
 
+// The operators that add to their result leave it as it is when the check they were queued behind (guard)
+// found the list too old, so that the host waits once per call, after the operator, and runs it again
+// in that case.
+struct MovedGuard {
+    const int *flag;      // device flag of the check, null without one
+    int seq;              // the check's number
+};
+static MovedGuard moved_guard(const fsd_ctx *ctx, bool guarded)
+{
+    return MovedGuard{guarded ? ctx->d_flags + 10 : nullptr, ctx->chk_seq};
+}
+
 // Lubrication_RFE_kernel (Lubrication.cu:350-608): F += R_FE : E
 __global__ void __launch_bounds__(PGB) rfe_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
                                                   const int *nlist, int maxn, LubTable t, float rl2, EParams ep,
-                                                  float *F, const int *order)
+                                                  float *F, const int *order, MovedGuard guard)
 {
     __shared__ PairRing ring;
     int lane;
     const int i = pg_particle(N, order, lane);
     if (i < 0) return;
+    const int moved = guard.flag ? *guard.flag : 0;
     float Ei[3][3];
     strain_block(ep, i, Ei);
     float acc[6] = {0, 0, 0, 0, 0, 0};
@@ -639,18 +657,20 @@ __global__ void __launch_bounds__(PGB) rfe_kernel(const float4 *pos, int N, BoxF
     });
 #pragma unroll
     for (int a = 0; a < 6; ++a) acc[a] = group_sum<PG>(acc[a]);
+    if (moved && moved == guard.seq) return;
     pg_add<6>(F + 6 * (int64_t)i, lane, acc, 1.f);
 }
 
 // Lubrication_RSU_kernel (Lubrication.cu:650-911): S -= R_SU U
 __global__ void __launch_bounds__(PGB) rsu_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
                                                   const int *nlist, int maxn, LubTable t, float rl2, const float *U,
-                                                  float *S, const int *order)
+                                                  float *S, const int *order, MovedGuard guard)
 {
     __shared__ PairRing ring;
     int lane;
     const int i = pg_particle(N, order, lane);
     if (i < 0) return;
+    const int moved = guard.flag ? *guard.flag : 0;
     float ui[3], wi[3];
     for (int a = 0; a < 3; ++a) { ui[a] = U[6 * (int64_t)i + a]; wi[a] = U[6 * (int64_t)i + 3 + a]; }
     float si[5] = {0, 0, 0, 0, 0};
@@ -680,18 +700,20 @@ __global__ void __launch_bounds__(PGB) rsu_kernel(const float4 *pos, int N, BoxF
     });
 #pragma unroll
     for (int c = 0; c < 5; ++c) si[c] = group_sum<PG>(si[c]);
+    if (moved && moved == guard.seq) return;
     pg_add<5>(S + 5 * (int64_t)i, lane, si, -1.f);
 }
 
 // Lubrication_RSE_kernel (Lubrication.cu:953-1211): S += R_SE : E, cutoff r^2 < 16
 __global__ void __launch_bounds__(PGB) rse_kernel(const float4 *pos, int N, BoxF b, const int *nneigh,
                                                   const int *nlist, int maxn, LubTable t, EParams ep, float *S,
-                                                  const int *order)
+                                                  const int *order, MovedGuard guard)
 {
     __shared__ PairRing ring;
     int lane;
     const int i = pg_particle(N, order, lane);
     if (i < 0) return;
+    const int moved = guard.flag ? *guard.flag : 0;
     float Ei[3][3];
     strain_block(ep, i, Ei);
     float Si[5] = {0, 0, 0, 0, 0};
@@ -726,6 +748,7 @@ __global__ void __launch_bounds__(PGB) rse_kernel(const float4 *pos, int N, BoxF
     });
 #pragma unroll
     for (int c = 0; c < 5; ++c) Si[c] = group_sum<PG>(Si[c]);
+    if (moved && moved == guard.seq) return;
     pg_add<5>(S + 5 * (int64_t)i, lane, Si, 1.f);
 }
 
@@ -739,32 +762,32 @@ static EParams make_ep(fsd_ctx *ctx, float shear_rate, const float *ori)
     return ep;
 }
 
-int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F)
+int k_rfe(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *F, bool guarded)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     hipLaunchKernelGGL(rfe_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
                        ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, ctx->p.rlub * ctx->p.rlub,
-                       make_ep(ctx, shear_rate, ori), F, cell_order(ctx));
+                       make_ep(ctx, shear_rate, ori), F, cell_order(ctx), moved_guard(ctx, guarded));
     FSD_HIP(hipGetLastError());
     return 0;
 }
 
-int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S)
+int k_rsu(fsd_ctx *ctx, const float4 *pos, const float *U, float *S, bool guarded)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     hipLaunchKernelGGL(rsu_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
                        ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, ctx->p.rlub * ctx->p.rlub, U, S,
-                       cell_order(ctx));
+                       cell_order(ctx), moved_guard(ctx, guarded));
     FSD_HIP(hipGetLastError());
     return 0;
 }
 
-int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S)
+int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, float *S, bool guarded)
 {
     LubTable t{ctx->d_res_dist, ctx->d_res_vals, ctx->table_min, ctx->table_dr};
     hipLaunchKernelGGL(rse_kernel, dim3(nblk(ctx->N, PGB / PG)), dim3(PGB), 0, ctx->stream, pos, ctx->N, ctx->box,
                        ctx->d_nneigh, ctx->d_nlist, ctx->maxn, t, make_ep(ctx, shear_rate, ori), S,
-                       cell_order(ctx));
+                       cell_order(ctx), moved_guard(ctx, guarded));
     FSD_HIP(hipGetLastError());
     return 0;
 }

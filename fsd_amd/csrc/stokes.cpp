@@ -220,6 +220,7 @@ static int alloc_all(fsd_ctx *ctx)
         CK(hipMalloc(&ctx->d_nslot, sizeof(int) * (size_t)N * ctx->maxn));
     }
     CK(hipMalloc(&ctx->d_flags, sizeof(int) * 16));
+    CK(hipMemset(ctx->d_flags, 0, sizeof(int) * 16));
     CK(hipMalloc(&ctx->d_pos_last, sizeof(float4) * (size_t)N));
     CK(hipHostMalloc((void **)&ctx->h_flags, sizeof(int) * 16, hipHostMallocDefault));
     // lubrication records
@@ -1323,40 +1324,63 @@ int fsd_rfd_drift(fsd_ctx *ctx, const float *d_pos4, uint32_t timestep, float *d
     return 0;
 }
 
+// The lubrication operators run behind the list's check without waiting for it; the host looks once,
+// at the end, and runs them again over a new list (or pair records of a larger capacity) if it must.
 int fsd_rfu(fsd_ctx *ctx, const float *d_pos4, const float *d_U6, float *d_F6)
 {
     const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
-    RC(ensure_lub(ctx, pos));
+    if (!ctx->nlist_valid) { ctx->err = "neighbour list not built"; return FSD_E_STATE; }
+    RC(k_nlist_check(ctx, pos));
+    RC(k_lub_pairs_launch(ctx, pos));
     RC(k_rfu_apply(ctx, d_U6, d_F6, nullptr, 1.0f));
     CK(hipStreamSynchronize(ctx->stream));
+    bool again = false;
+    RC(k_nlist_settle(ctx, pos, &again));
+    ctx->nlist_builds += again;
+    if (again) RC(k_lub_pairs_launch(ctx, pos));
+    const int capacity = ctx->maxlub;
+    RC(k_lub_pairs_settle(ctx, pos));
+    if (again || ctx->maxlub != capacity) {
+        RC(k_rfu_apply(ctx, d_U6, d_F6, nullptr, 1.0f));
+        CK(hipStreamSynchronize(ctx->stream));
+    }
+    return 0;
+}
+
+extern "C++" template <class Run>
+static int behind_check(fsd_ctx *ctx, const float4 *pos, Run run)
+{
+    if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
+    if (!ctx->nlist_valid) { ctx->err = "neighbour list not built"; return FSD_E_STATE; }
+    RC(k_nlist_check(ctx, pos));
+    RC(run(true));
+    CK(hipStreamSynchronize(ctx->stream));
+    bool rebuilt = false;
+    RC(k_nlist_settle(ctx, pos, &rebuilt));
+    ctx->nlist_builds += rebuilt;
+    if (rebuilt) {
+        RC(run(false));
+        CK(hipStreamSynchronize(ctx->stream));
+    }
     return 0;
 }
 
 int fsd_rfe(fsd_ctx *ctx, const float *d_pos4, float shear_rate, const float *d_ori3, float *d_F6)
 {
-    if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
-    RC(current_nlist(ctx, reinterpret_cast<const float4 *>(d_pos4)));
-    RC(k_rfe(ctx, reinterpret_cast<const float4 *>(d_pos4), shear_rate, d_ori3, d_F6));
-    CK(hipStreamSynchronize(ctx->stream));
-    return 0;
+    const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
+    return behind_check(ctx, pos, [&](bool guarded) { return k_rfe(ctx, pos, shear_rate, d_ori3, d_F6, guarded); });
 }
 
 int fsd_rsu(fsd_ctx *ctx, const float *d_pos4, const float *d_U6, float *d_S5)
 {
-    if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
-    RC(current_nlist(ctx, reinterpret_cast<const float4 *>(d_pos4)));
-    RC(k_rsu(ctx, reinterpret_cast<const float4 *>(d_pos4), d_U6, d_S5));
-    CK(hipStreamSynchronize(ctx->stream));
-    return 0;
+    const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
+    return behind_check(ctx, pos, [&](bool guarded) { return k_rsu(ctx, pos, d_U6, d_S5, guarded); });
 }
 
 int fsd_rse(fsd_ctx *ctx, const float *d_pos4, float shear_rate, const float *d_ori3, float *d_S5)
 {
-    if (!ctx->have_table) { ctx->err = "resistance table not set"; return FSD_E_STATE; }
-    RC(current_nlist(ctx, reinterpret_cast<const float4 *>(d_pos4)));
-    RC(k_rse(ctx, reinterpret_cast<const float4 *>(d_pos4), shear_rate, d_ori3, d_S5));
-    CK(hipStreamSynchronize(ctx->stream));
-    return 0;
+    const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
+    return behind_check(ctx, pos, [&](bool guarded) { return k_rse(ctx, pos, shear_rate, d_ori3, d_S5, guarded); });
 }
 
 int fsd_mobility(fsd_ctx *ctx, const float *d_pos4, const float *d_gF11, float *d_gU11, int32_t parts)

@@ -9,7 +9,7 @@ allowed.  A second product of a context starts from what the first left and has 
 
 A product whose positions have moved finds that after its wave part is queued, rebuilds the list and sums
 real space over the new one: it differs from a fresh context's in the order of the sums only (1e-6;
-1e-5 allowed).
+1e-5 allowed).  So do the lubrication operators.
 """
 import numpy as np
 import pytest
@@ -62,6 +62,9 @@ def test_list_rebuilt_in_product(N, L):
     b = _pos(q)
     for got, want in ((st.mobility(b, x), fresh.mobility(b, x)), (st.mobility(b, x), fresh.mobility(b, x))):
         assert (got - want).abs().max() <= 1e-5 * want.abs().max()
-    st.build_nlist(_pos(p))
-    got, want = st.saddle_multiply(b, y), fresh.saddle_multiply(b, y)
-    assert (got - want).abs().max() <= 1e-5 * want.abs().max()
+    ops = (lambda s: s.saddle_multiply(b, y), lambda s: s.rfu(b, y[:6 * N]), lambda s: s.rsu(b, y[:6 * N]),
+           lambda s: s.rfe(b, 1.0), lambda s: s.rse(b, 1.0))
+    for op in ops:                           # the last four run again if the check they are queued behind says so
+        st.build_nlist(_pos(p))
+        got, want = op(st), op(fresh)
+        assert (got - want).abs().max() <= 1e-5 * want.abs().max()
