@@ -45,10 +45,12 @@ METRIC = "steps/s at N=32k phi=0.45: learned vs IChol precond at equal residual 
 HBM_PEAK_GBS = 8000.0
 GUESS_TEXT = {"previous": "previous solution", "extrapolate": "linear extrapolation of the last two solutions",
               "quadratic": "quadratic extrapolation of the last three solutions"}
+# one iteration's Gram-Schmidt (one pass, long vectors): four kernels timed together
+GMRES_VEC = "gs_dots_long_kernel<true> + gs_sum_kernel + gs_kernel<true, true, false, true> + gs_scale_kernel<true>"
 # kernel-class name -> kernel name in rocprofv3 traces
 KERNEL_NAMES = {"spread": "spread_mfma_kernel<6>", "green": "x_green_kernel<4, 256, true>", "contract": "contract_tile2_kernel<13, 6>",
-                "realspace": "realspace_kernel<16>", "rfu": "rfu_apply_kernel<8>", "sweep": "tp_sweep1_kernel",
-                "ichol": "ichol_level_kernel", "gmres_vec": "multidot_partial4_kernel", "ljit": "bj_iter_kernel<false>",
+                "realspace": "realspace_lds_kernel<16>", "rfu": "rfu_apply_kernel<8>", "sweep": "tp_sweep1_kernel",
+                "ichol": "ichol_level_kernel", "gmres_vec": GMRES_VEC, "ljit": "bj_iter_kernel<false>",
                 "jacobi": "bj_iter_kernel<false>"}
 
 
@@ -254,16 +256,16 @@ def main():
     traffic, kname = None, KERNEL_NAMES.get(head_dom)
     shapes = arms[head]["launch_shapes"]
     if head_dom == "realspace":      # the autotuner's lanes per particle
-        kname = "realspace_kernel<%d>" % shapes["real_lanes"]
+        kname = "realspace_lds_kernel<%d>" % shapes["real_lanes"]
     elif head_dom == "rfu":
         kname = "rfu_apply_kernel<%d>" % shapes["rfu_lanes"]
     tfile = os.path.join(ROOT, "profiles", "traffic_N32768.json")
     if os.path.exists(tfile):
         with open(tfile) as f:
             tr = json.load(f)
-        k = tr.get("kernels", {}).get(kname)
-        if k:
-            traffic = 1024.0 * (k["fetch_kib"] * tr["fetch_factor"] + k["write_kib"] * tr["write_factor"])
+        ks = [tr.get("kernels", {}).get(k) for k in (kname or "").split(" + ")]
+        if all(ks):
+            traffic = sum(1024.0 * (k["fetch_kib"] * tr["fetch_factor"] + k["write_kib"] * tr["write_factor"]) for k in ks)
     log("# %s: %.2f ms/step, dominant kernel class %s (%d launches, %.3f ms avg)"
         % (head, arms[head]["ms_per_step"], head_dom, launches, avg_ms))
     cpu = None
