@@ -7,7 +7,7 @@
 //               functions) + one symmetric 6x6 self block per particle,
 //               built once per step and reused by every R_FU apply;
 //   PSE grids   11 real fields [11][Nx][Ny][pitch] (z fastest; grid_pitch) and their
-//               half spectra [11][Nx*Ny*(Nz/2+1)] (rocFFT R2C/C2R);
+//               half spectra [11][Nx*Ny*(Nz/2+1)];
 //   IC(0)       block-sparse lower factor on the RCM-permuted particle graph:
 //               per permuted particle a dense 6x6 diagonal block and one 6x6
 //               block per lower neighbour (36 floats, row-major).

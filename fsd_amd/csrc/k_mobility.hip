@@ -368,7 +368,9 @@ __global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const int *or
 // share it and the records.  Per node this takes 64 spheres (those that reach any of the 4 x 4
 // x 4 nodes), of which 19 count, at twice the VALU's rate.  The same sums on the VALU were bound
 // by lanes that waited for the longest of 36 short runs of spheres (34.6 us per product at N =
-// 32768) or, with those runs merged, by LDS bank conflicts (each lane its own sphere: 34.6 us).
+// 32768) or, with those runs merged, by LDS bank conflicts (each lane its own sphere: 34.6 us); this form takes
+// 23 us (13 us at N = 4072), of which half are the dependent loads before the products and the
+// stores after them.
 // The tile's halo of 13^3 origin cells is staged in LDS.  Its spheres are in the order of buckets
 // (x, third of z, y): a wave of the lower nodes needs the first two thirds, one of the upper
 // nodes the last two, so its spheres are 18 runs of nine buckets each, which it lists.  A halo of
@@ -722,8 +724,9 @@ __global__ void __launch_bounds__(512) contract_tile_kernel(SpreadGeom g, const 
 // four particles at once (a wave per particle kept 36 lanes busy and spent more on the
 // sums than on the nodes).  The LDS block is node-major, six fields to a node, so a node
 // is three 8-byte reads; lanes of consecutive z are six words apart, which conflicts
-// nowhere inside a particle.  The block is loaded by 16 lanes per row of 13 nodes: the
-// wrapped row offsets come from a table and z is fixed per lane.
+// nowhere inside a particle.  The block is loaded by the seven waves that
+// do not stage particles, 30 values of a thread in flight.  Per product at N = 32768: 43 us with a
+// wave per particle, 23 us so.
 #define CT_NF 6
 #define CT_PCAP 128   // particles of a tile staged in LDS (about 45 in an 8^3 tile at volume fraction 0.45)
 template <int S, int PP>

@@ -10,7 +10,9 @@
 // per particle leaves 145 waves on 256 CUs at N = 9261 and waits for ~150 of them in
 // turn.  The lanes read 16 list entries at a time and append the pairs that pass the
 // cutoff, in list order, to a small LDS ring; the pair work (about a third of the list
-// at r < 4) then runs on 16 pairs at a time with every lane busy.
+// at r < 4) then runs on 16 pairs at a time with every lane busy.  At N = 32768 and volume
+// fraction 0.45 the lubrication pairs take 42 us (119 with a thread per particle); at N =
+// 9261 the pairs, R_FU, R_FE, R_SU and R_SE together 110 us (491).
 constexpr int PG = 16;                  // lanes per particle
 constexpr int PGB = 256;                // threads per workgroup
 struct PairRing {

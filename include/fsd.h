@@ -205,7 +205,7 @@ int fsd_build_precond(fsd_ctx *ctx, const float *d_pos4, fsd_solve_stats *stats)
  * (spreading, contraction and x-transform kernels of the wave-space part; lanes per
  * particle and workgroup size of the real-space sum and of R_FU) and keeps the fastest.
  * h_choice8 (may be null): spread (0 tiled, 1 per-tile), contract (0 tiled, 1 per
- * particle), xpass (0 fused x transforms, 1 3-D rocFFT), real-space lanes, real-space
+ * particle), xpass (0 transforms in LDS, 1 3-D rocFFT), real-space lanes, real-space
  * workgroup, R_FU lanes, R_FU workgroup, tuned; h_us3 (may be null): the best time per
  * apply in microseconds of the wave part, the real part and R_FU.  Allocates scratch. */
 int fsd_autotune(fsd_ctx *ctx, const float *d_pos4, int32_t *h_choice8, float *h_us3);
