@@ -14,12 +14,12 @@
 #pragma once
 #include <functional>
 #include <hip/hip_runtime.h>
-#include <rocfft/rocfft.h>
 #include <stdint.h>
 #include <string>
 #include <vector>
 #include "fsd.h"
 #include "precond_plan.h"
+#include "fft_library.h"
 #include "fft_small.h"
 
 #define FSD_MAXP 14        // pruned neighbours incl. self (kissing number 12 + self + 1)
@@ -249,14 +249,12 @@ struct fsd_ctx {
     float *d_grid = nullptr;      // 11 real grids, rows of grid_pitch floats
     float2 *d_spec = nullptr;     // 11*Mh complex
     float4 *d_gridk = nullptr;    // Mh
-    rocfft_plan plan_fwd = nullptr, plan_inv = nullptr;
     // this library's transforms (k_fft.hip), used unless the grid does not fit them
     bool fft_lds = false;
     FftAxis fft_axis[3];
     float2 *d_fft_tw = nullptr;
     unsigned short *d_fft_loc = nullptr;
-    rocfft_execution_info info_fwd = nullptr, info_inv = nullptr;
-    void *d_fftwork = nullptr; size_t fftwork_size = 0;
+    FftLibrary fft3;              // 3-D library plans, made on first use (fft_plans_3d)
     int tiles[3] = {0, 0, 0}; int ntiles = 0; int tile = 8;
     // set-up of the wave part, particles by slot (cell order of the neighbour list; identity without one)
     float4 *d_spos = nullptr;     // N: position, w the particle's index (bits)

@@ -1181,12 +1181,10 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
         if (!rc) rc = k_fft_yz_inverse(ctx);
         if (rc) return rc;
     } else {
-        void *in[1] = {ctx->d_spec};
-        void *out[1] = {ctx->d_grid};
         const int rc = fft_plans_3d(ctx);
         if (rc) return rc;
-        if (rocfft_execute(ctx->plan_inv, in, out, ctx->info_inv) != rocfft_status_success) {
-            ctx->err = "rocfft inverse failed";
+        if (const char *failed = ctx->fft3.inverse(ctx->d_spec, ctx->d_grid)) {
+            ctx->err = failed;
             return FSD_E_HIP;
         }
     }
@@ -1249,12 +1247,10 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
             const int rc = k_fft_yz_forward(ctx);
             if (rc) return rc;
         } else {
-            void *in[1] = {ctx->d_grid};
-            void *out[1] = {ctx->d_spec};
             const int rc = fft_plans_3d(ctx);
             if (rc) return rc;
-            if (rocfft_execute(ctx->plan_fwd, in, out, ctx->info_fwd) != rocfft_status_success) {
-                ctx->err = "rocfft forward failed";
+            if (const char *failed = ctx->fft3.forward(ctx->d_grid, ctx->d_spec)) {
+                ctx->err = failed;
                 return FSD_E_HIP;
             }
         }

@@ -171,30 +171,14 @@ static void cell_dims(fsd_ctx *ctx)
 // the LDS transforms, and the autotuner's comparison with them
 int fft_plans_3d(fsd_ctx *ctx)
 {
-    if (ctx->plan_fwd && ctx->plan_inv) return 0;
+    if (ctx->fft3.ready()) return 0;
     static std::mutex mu;   // contexts may step from several threads
     std::lock_guard<std::mutex> lk(mu);
     const fsd_pse_info &ps = ctx->pse;
-    size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
-    if (rocfft_plan_create(&ctx->plan_fwd, rocfft_placement_notinplace, rocfft_transform_type_real_forward,
-                           rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success ||
-        rocfft_plan_create(&ctx->plan_inv, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
-                           rocfft_precision_single, 3, lengths, 11, nullptr) != rocfft_status_success) {
-        ctx->err = "rocfft_plan_create failed";
+    const size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
+    if (const char *failed = ctx->fft3.make(3, lengths, 11, ctx->stream)) {
+        ctx->err = failed;
         return FSD_E_HIP;
-    }
-    size_t w1 = 0, w2 = 0;
-    rocfft_plan_get_work_buffer_size(ctx->plan_fwd, &w1);
-    rocfft_plan_get_work_buffer_size(ctx->plan_inv, &w2);
-    ctx->fftwork_size = std::max(w1, w2);
-    if (ctx->fftwork_size) CK(hipMalloc(&ctx->d_fftwork, ctx->fftwork_size));
-    rocfft_execution_info_create(&ctx->info_fwd);
-    rocfft_execution_info_create(&ctx->info_inv);
-    rocfft_execution_info_set_stream(ctx->info_fwd, ctx->stream);
-    rocfft_execution_info_set_stream(ctx->info_inv, ctx->stream);
-    if (ctx->fftwork_size) {
-        rocfft_execution_info_set_work_buffer(ctx->info_fwd, ctx->d_fftwork, ctx->fftwork_size);
-        rocfft_execution_info_set_work_buffer(ctx->info_inv, ctx->d_fftwork, ctx->fftwork_size);
     }
     return 0;
 }
@@ -359,7 +343,7 @@ static void free_all(fsd_ctx *ctx)
     lp_free(ctx);
     void *ptrs[] = {ctx->d_nneigh, ctx->d_nlist, ctx->d_snn, ctx->d_nslot, ctx->d_spos, ctx->d_cell_of, ctx->d_cell_count, ctx->d_cell_start,
                     ctx->d_cell_list, ctx->d_flags, ctx->d_pos_last, ctx->d_lub_n, ctx->d_lub_j, ctx->d_lub_a, ctx->d_lub_b,
-                    ctx->d_lub_self, ctx->d_grid, ctx->d_spec, ctx->d_gridk, ctx->d_fftwork, ctx->d_porig,
+                    ctx->d_lub_self, ctx->d_grid, ctx->d_spec, ctx->d_gridk, ctx->d_porig,
                     ctx->d_ocell, ctx->d_olist, ctx->d_ocount, ctx->d_orank, ctx->d_ostart, ctx->d_scan_tmp, ctx->d_wave, ctx->d_rec,
                     ctx->d_ewald, ctx->d_res_dist, ctx->d_res_vals, ctx->d_pn, ctx->d_plist, ctx->d_pless,
                     ctx->d_perm, ctx->d_iperm, ctx->d_lrow, ctx->d_urow, ctx->d_lcol, ctx->d_ucol, ctx->d_upos,
@@ -381,10 +365,7 @@ static void free_all(fsd_ctx *ctx)
     for (hipEvent_t e : {ctx->gm_ev[0], ctx->gm_ev[1], ctx->chk_ev})
         if (e) hipEventDestroy(e);
     if (ctx->h_lan) hipHostFree(ctx->h_lan);
-    if (ctx->plan_fwd) rocfft_plan_destroy(ctx->plan_fwd);
-    if (ctx->plan_inv) rocfft_plan_destroy(ctx->plan_inv);
-    if (ctx->info_fwd) rocfft_execution_info_destroy(ctx->info_fwd);
-    if (ctx->info_inv) rocfft_execution_info_destroy(ctx->info_inv);
+    ctx->fft3.release();
     for (auto &s : ctx->slots)
         for (auto &pr : s.pending) { hipEventDestroy(pr.b); hipEventDestroy(pr.e); }
 }
