@@ -50,9 +50,7 @@ int time_us(fsd_ctx *ctx, const Scratch &s, Fn &&apply, float *us)
 
 }  // namespace
 
-// The neighbour list, the lubrication pairs and the spreading set-up must be current
-// for pos.  Leaves ctx->tune at the fastest variants (tuned = 1).
-int autotune_run(fsd_ctx *ctx, const float4 *pos)
+static int search(fsd_ctx *ctx, const float4 *pos)
 {
     const int64_t N = ctx->N;
     Scratch s;
@@ -71,11 +69,12 @@ int autotune_run(fsd_ctx *ctx, const float4 *pos)
     RC(time_us(ctx, s, wave, &best));
     const bool can_spread2 = ctx->tile == 8 && ctx->pse.P == 6;
     const bool can_contract_tiled = ctx->contract_lds > 0;
-    const bool can_fx = ctx->fft_lds;
+    // the library's plans are made for this comparison; without the memory for them there is none
+    const bool has_fx = ctx->fft_lds, can_fx = has_fx && fft_plans_3d(ctx) == 0;
     int *knobs[3] = {&t.spread, &t.contract, &t.xpass};
     const bool alt[3] = {can_spread2, can_contract_tiled, can_fx};   // the default (0) is a real choice
     for (int k = 0; k < 3; ++k) {
-        if (!alt[k]) { *knobs[k] = 1; continue; }   // only the general kernel applies
+        if (!alt[k]) { *knobs[k] = k == 2 && has_fx ? 0 : 1; continue; }   // only one kernel applies
         *knobs[k] = 1;
         RC(time_us(ctx, s, wave, &us));
         if (us < best) best = us;
@@ -105,4 +104,15 @@ int autotune_run(fsd_ctx *ctx, const float4 *pos)
     t.tuned = 1;
     FSD_HIP(hipStreamSynchronize(ctx->stream));
     return 0;
+}
+
+// The neighbour list, the lubrication pairs and the spreading set-up must be current
+// for pos.  Leaves ctx->tune at the fastest variants (tuned = 1), after a failure as it was.
+int autotune_run(fsd_ctx *ctx, const float4 *pos)
+{
+    const fsd_tuning before = ctx->tune;
+    ctx->tune = fsd_tuning();
+    const int rc = search(ctx, pos);
+    if (rc < 0) ctx->tune = before;
+    return rc;
 }

@@ -1386,7 +1386,6 @@ int fsd_autotune(fsd_ctx *ctx, const float *d_pos4, int32_t *h_choice8, float *h
     const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
     RC(ensure_lub(ctx, pos));
     ctx->spread_valid = false;
-    ctx->tune = fsd_tuning();
     RC(autotune_run(ctx, pos));
     return fsd_get_tuning(ctx, h_choice8, h_us3);
 }
