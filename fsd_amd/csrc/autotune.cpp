@@ -70,7 +70,7 @@ static int search(fsd_ctx *ctx, const float4 *pos)
     const bool can_spread2 = ctx->tile == 8 && ctx->pse.P == 6;
     const bool can_contract_tiled = ctx->contract_lds > 0;
     // the library's plans are made for this comparison; without the memory for them there is none
-    const bool has_fx = ctx->fft_lds, can_fx = has_fx && fft_plans_3d(ctx) == 0;
+    const bool has_fx = ctx->fft_x, can_fx = has_fx && fft_plans_3d(ctx) == 0;
     int *knobs[3] = {&t.spread, &t.contract, &t.xpass};
     const bool alt[3] = {can_spread2, can_contract_tiled, can_fx};   // the default (0) is a real choice
     for (int k = 0; k < 3; ++k) {

@@ -249,8 +249,9 @@ struct fsd_ctx {
     float *d_grid = nullptr;      // 11 real grids, rows of grid_pitch floats
     float2 *d_spec = nullptr;     // 11*Mh complex
     float4 *d_gridk = nullptr;    // Mh
-    // this library's transforms (k_fft.hip), used unless the grid does not fit them
-    bool fft_lds = false;
+    // this library's transforms (k_fft.hip): along x, and in the (y, z) planes where those fit LDS too
+    bool fft_x = false, fft_yz = false;
+    FftLibrary fft2;              // (y, z) library plans of larger planes
     FftAxis fft_axis[3];
     float2 *d_fft_tw = nullptr;
     unsigned short *d_fft_loc = nullptr;
@@ -439,16 +440,20 @@ int k_ff_noise(fsd_ctx *ctx, const float *noise, float fac);
 int k_wave_to_general(fsd_ctx *ctx, float *out);
 int k_shift_wrap(fsd_ctx *ctx, const float4 *pos, const float *psi6, float scale, float4 *out);
 int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done = false);
-// transforms of the grids (k_fft.hip; the 3-D library plans in stokes.cpp)
+// transforms of the grids (k_fft.hip; the library plans in stokes.cpp)
 int fft_init(fsd_ctx *ctx);
+int fft_plans_2d(fsd_ctx *ctx);
 int fft_plans_3d(fsd_ctx *ctx);
 int k_fft_yz_forward(fsd_ctx *ctx);
 int k_fft_x(fsd_ctx *ctx, bool green);
 int k_fft_yz_inverse(fsd_ctx *ctx);
-inline bool use_fft_lds(const fsd_ctx *ctx) { return ctx->fft_lds && ctx->tune.xpass == 0; }
-// row length of the grids in memory: whole float4s for this library's transforms (16-byte stores
-// and loads for odd lengths too), Nz for the 3-D plans
-inline int grid_pitch(const fsd_ctx *ctx) { return use_fft_lds(ctx) ? (ctx->pse.Nz + 3) / 4 * 4 : ctx->pse.Nz; }
+inline bool use_fft_x(const fsd_ctx *ctx) { return ctx->fft_x && ctx->tune.xpass == 0; }
+// row length of the grids in memory: whole float4s for this library's planes (16-byte stores
+// and loads for odd lengths too), Nz for rocFFT's
+inline int grid_pitch(const fsd_ctx *ctx)
+{
+    return use_fft_x(ctx) && ctx->fft_yz ? (ctx->pse.Nz + 3) / 4 * 4 : ctx->pse.Nz;
+}
 int k_precond_apply2(fsd_ctx *ctx, const float *b0, const float *b1, float *y0, float *y1, int n_rhs);
 int k_export_csr(fsd_ctx *ctx, const float4 *pos, int32_t *h_rowptr, int32_t *h_col, float *h_val,
                  int32_t *h_prow, int32_t *h_pcol, float *h_L, int64_t cap);

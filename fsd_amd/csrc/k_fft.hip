@@ -6,7 +6,9 @@
 //                       transformed along z and y there and written once;
 //   x_green_kernel      one workgroup per ky and XKC consecutive kz of all 11 fields: forward
 //                       along x, Green's function, inverse along x;
-//   yz_inverse_kernel   the planes back to real space.
+//   yz_inverse_kernel   the planes back to real space;
+//
+// with the library's 2-D transforms in the place of the first and the last where a plane exceeds LDS.
 //
 // Bound: HBM for large grids, the barriers between the LDS stages for small ones.  Measured
 // (mobility product, HIP kernel times): 135^3, three passes 251 us where the 3-D library plans of
@@ -332,14 +334,20 @@ hipError_t allow_lds(K kernel, size_t bytes)
 }
 }  // namespace
 
-// tables of the three axes when the grid's planes and x columns fit in LDS (up to about 200 points
-// per axis); otherwise ctx->fft_lds stays false and the 3-D library plans are used
+// Tables of the three axes when the grid's x columns fit in LDS (up to about 450 points); otherwise
+// ctx->fft_x stays false and the 3-D library plans are used.  The planes are a matter of their own:
+// those that fit LDS (up to about 200 points per axis) are transformed there, larger ones by the
+// library's 2-D plans, from X_ALONE points along x on.  Wave part of a product that way and with the 3-D
+// plans, us: 40 x 225 x 240 683 and 716, 48 x 200 x 216 523 and 711, 72 x 225 x 240 1231 and 1410, 80 x 256^2
+// 1323 and 1372, 135 x 216 x 225 3132 and 4435, 200^3 1874 and 2109, 256^3 4618 and 4693, 400 x 200^2 4049 and
+// 5706; shorter axes gain nothing (24 x 225 x 240 473 and 470, 12 x 225 x 240 326 and 333).
+constexpr int X_ALONE = 40;
 int fft_init(fsd_ctx *ctx)
 {
     const int n[3] = {ctx->pse.Nx, ctx->pse.Ny, ctx->pse.Nz};
-    ctx->fft_lds = false;
-    const size_t yz = yz_lds(n[1], n[2]), x = x_lds(n[0]);
-    if (yz > LDS_MAX || x > LDS_MAX) return 0;
+    ctx->fft_x = ctx->fft_yz = false;
+    const bool planes = yz_lds(n[1], n[2]) <= LDS_MAX;
+    if (x_lds(n[0]) > LDS_MAX || (!planes && n[0] < X_ALONE)) return 0;
     const int total = n[0] + n[1] + n[2];
     std::vector<float2> tw(total);
     std::vector<unsigned short> loc(total);
@@ -368,7 +376,12 @@ int fft_init(fsd_ctx *ctx)
         FSD_HIP(allow_lds(k, LDS_MAX));
     FSD_HIP(allow_lds(x_green_kernel<XKC, 256, true>, LDS_MAX));
     FSD_HIP(allow_lds(x_green_kernel<XKC, 256, false>, LDS_MAX));
-    ctx->fft_lds = true;
+    if (!planes) {
+        const int rc = fft_plans_2d(ctx);
+        if (rc) return rc;
+    }
+    ctx->fft_x = true;
+    ctx->fft_yz = planes;
     return 0;
 }
 
@@ -384,9 +397,17 @@ static YzArgs yz_args(const fsd_ctx *ctx)
     return a;
 }
 
+static int library_result(fsd_ctx *ctx, const char *failed)
+{
+    if (!failed) return 0;
+    ctx->err = failed;
+    return FSD_E_HIP;
+}
+
 // (y, z) transform of the 11 grids in d_grid into d_spec
 int k_fft_yz_forward(fsd_ctx *ctx)
 {
+    if (!ctx->fft_yz) return library_result(ctx, ctx->fft2.forward(ctx->d_grid, ctx->d_spec));
     const YzArgs a = yz_args(ctx);
     const size_t lds = yz_lds(a.Ny, a.Nz);
     const dim3 grid(11 * a.Nx);
@@ -401,6 +422,7 @@ int k_fft_yz_forward(fsd_ctx *ctx)
 
 int k_fft_yz_inverse(fsd_ctx *ctx)
 {
+    if (!ctx->fft_yz) return library_result(ctx, ctx->fft2.inverse(ctx->d_spec, ctx->d_grid));
     const YzArgs a = yz_args(ctx);
     const size_t lds = yz_lds(a.Ny, a.Nz);
     const dim3 grid(11 * a.Nx);

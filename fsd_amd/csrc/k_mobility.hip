@@ -1176,7 +1176,7 @@ int k_wave_contract(fsd_ctx *ctx, const float4 *pos, bool x_done)
     const int64_t Mp = (int64_t)ps.Nx * ps.Ny * g.pz;   // grid field stride
     hipEvent_t ev;
     prof_begin(ctx, PROF_FFT, &ev);
-    if (use_fft_lds(ctx)) {
+    if (use_fft_x(ctx)) {
         int rc = x_done ? 0 : k_fft_x(ctx, false);
         if (!rc) rc = k_fft_yz_inverse(ctx);
         if (rc) return rc;
@@ -1241,7 +1241,7 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
                                Mp);
         FSD_HIP(hipGetLastError());
         prof_end(ctx, PROF_SPREAD, ev);
-        const bool fx = use_fft_lds(ctx);
+        const bool fx = use_fft_x(ctx);
         prof_begin(ctx, PROF_FFT, &ev);
         if (fx) {
             const int rc = k_fft_yz_forward(ctx);

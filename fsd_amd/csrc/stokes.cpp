@@ -167,21 +167,26 @@ static void cell_dims(fsd_ctx *ctx)
         if (r_ < 0) return r_;                                                                      \
     } while (0)
 
-// the 3-D library plans (batched over the 11 fields), made on the first use: grids that do not fit
-// the LDS transforms, and the autotuner's comparison with them
-int fft_plans_3d(fsd_ctx *ctx)
+static int library_plans(fsd_ctx *ctx, FftLibrary &lib, size_t dims, size_t batch)
 {
-    if (ctx->fft3.ready()) return 0;
+    if (lib.ready()) return 0;
     static std::mutex mu;   // contexts may step from several threads
     std::lock_guard<std::mutex> lk(mu);
     const fsd_pse_info &ps = ctx->pse;
     const size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
-    if (const char *failed = ctx->fft3.make(3, lengths, 11, ctx->stream)) {
+    if (const char *failed = lib.make(dims, lengths, batch, ctx->stream)) {
         ctx->err = failed;
         return FSD_E_HIP;
     }
     return 0;
 }
+
+// the 3-D library plans (batched over the 11 fields), made on the first use: grids that do not take
+// the x pass of k_fft.hip, and the autotuner's comparison with them
+int fft_plans_3d(fsd_ctx *ctx) { return library_plans(ctx, ctx->fft3, 3, 11); }
+
+// the (y, z) library plans (batched over the fields and the x planes)
+int fft_plans_2d(fsd_ctx *ctx) { return library_plans(ctx, ctx->fft2, 2, 11 * (size_t)ctx->pse.Nx); }
 
 static int alloc_all(fsd_ctx *ctx)
 {
@@ -252,7 +257,7 @@ static int alloc_all(fsd_ctx *ctx)
         // 3-D library plans and the separate Green's function
         const char *f3 = getenv("FSD_FFT_3D");
         if (!(f3 && f3[0] == '1')) RC(fft_init(ctx));
-        if (!ctx->fft_lds) RC(fft_plans_3d(ctx));
+        if (!ctx->fft_x) RC(fft_plans_3d(ctx));
     }
     // Ewald table
     ctx->ewald_nR = ps.ewald_n + 1;
@@ -365,6 +370,7 @@ static void free_all(fsd_ctx *ctx)
     for (hipEvent_t e : {ctx->gm_ev[0], ctx->gm_ev[1], ctx->chk_ev})
         if (e) hipEventDestroy(e);
     if (ctx->h_lan) hipHostFree(ctx->h_lan);
+    ctx->fft2.release();
     ctx->fft3.release();
     for (auto &s : ctx->slots)
         for (auto &pr : s.pending) { hipEventDestroy(pr.b); hipEventDestroy(pr.e); }

@@ -64,7 +64,7 @@ static fsd_ctx *context()
     ctx->pse.P = 6;
     ctx->tile = 8;
     ctx->contract_lds = 1;
-    ctx->fft_lds = true;
+    ctx->fft_x = true;
     return ctx;
 }
 
