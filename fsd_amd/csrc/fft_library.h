@@ -1,5 +1,6 @@
 // Forward and inverse real-to-complex transforms of the grids by rocFFT, with all that an execution
 // needs: both plans, their execution infos on the context's stream and one work buffer for the two.
+// lengths[0] is the fastest; the rows of the real grids are pitch floats apart, everything else is dense.
 #pragma once
 #include <hip/hip_runtime_api.h>
 #include <rocfft/rocfft.h>
@@ -11,10 +12,10 @@ struct FftLibrary {
     // Makes everything or nothing: a failed call leaves no plan, info or memory behind, ready() stays
     // false and a later call starts again, so no execution ever runs without the context's stream
     // (on the default stream, unordered with it).  Returns null, or what failed.
-    const char *make(size_t dims, const size_t *lengths, size_t batch, hipStream_t stream)
+    const char *make(size_t dims, const size_t *lengths, size_t pitch, size_t batch, hipStream_t stream)
     {
         if (ready_) return nullptr;
-        const char *failed = try_make(dims, lengths, batch, stream);
+        const char *failed = try_make(dims, lengths, pitch, batch, stream);
         if (failed) release();
         else ready_ = true;
         return failed;
@@ -40,14 +41,37 @@ struct FftLibrary {
     }
 
 private:
-    const char *try_make(size_t dims, const size_t *lengths, size_t batch, hipStream_t stream)
+    const char *try_make(size_t dims, const size_t *lengths, size_t pitch, size_t batch, hipStream_t stream)
     {
         auto ok = [](rocfft_status s) { return s == rocfft_status_success; };
-        if (!ok(rocfft_plan_create(&fwd_, rocfft_placement_notinplace, rocfft_transform_type_real_forward,
-                                   rocfft_precision_single, dims, lengths, batch, nullptr)) ||
-            !ok(rocfft_plan_create(&inv_, rocfft_placement_notinplace, rocfft_transform_type_real_inverse,
-                                   rocfft_precision_single, dims, lengths, batch, nullptr)))
-            return "rocfft_plan_create failed";
+        for (const bool inverse : {false, true}) {
+            rocfft_plan_description layout = nullptr;
+            if (pitch != lengths[0]) {
+                size_t real[3] = {1, 1, 1}, half[3] = {1, 1, 1}, real_size = pitch, half_size = lengths[0] / 2 + 1;
+                for (size_t d = 1; d < dims; ++d) {
+                    real[d] = real_size;
+                    half[d] = half_size;
+                    real_size *= lengths[d];
+                    half_size *= lengths[d];
+                }
+                const rocfft_array_type r = rocfft_array_type_real, h = rocfft_array_type_hermitian_interleaved;
+                const bool described =
+                    ok(rocfft_plan_description_create(&layout)) &&
+                    ok(rocfft_plan_description_set_data_layout(
+                        layout, inverse ? h : r, inverse ? r : h, nullptr, nullptr, dims, inverse ? half : real,
+                        inverse ? half_size : real_size, dims, inverse ? real : half, inverse ? real_size : half_size));
+                if (!described) {
+                    if (layout) rocfft_plan_description_destroy(layout);
+                    return "rocfft_plan_description failed";
+                }
+            }
+            const bool made = ok(rocfft_plan_create(
+                inverse ? &inv_ : &fwd_, rocfft_placement_notinplace,
+                inverse ? rocfft_transform_type_real_inverse : rocfft_transform_type_real_forward,
+                rocfft_precision_single, dims, lengths, batch, layout));
+            if (layout) rocfft_plan_description_destroy(layout);
+            if (!made) return "rocfft_plan_create failed";
+        }
         size_t w1 = 0, w2 = 0;
         if (!ok(rocfft_plan_get_work_buffer_size(fwd_, &w1)) || !ok(rocfft_plan_get_work_buffer_size(inv_, &w2)))
             return "rocfft_plan_get_work_buffer_size failed";

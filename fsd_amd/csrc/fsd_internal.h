@@ -448,12 +448,9 @@ int k_fft_yz_forward(fsd_ctx *ctx);
 int k_fft_x(fsd_ctx *ctx, bool green);
 int k_fft_yz_inverse(fsd_ctx *ctx);
 inline bool use_fft_x(const fsd_ctx *ctx) { return ctx->fft_x && ctx->tune.xpass == 0; }
-// row length of the grids in memory: whole float4s for this library's planes (16-byte stores
-// and loads for odd lengths too), Nz for rocFFT's
-inline int grid_pitch(const fsd_ctx *ctx)
-{
-    return use_fft_x(ctx) && ctx->fft_yz ? (ctx->pse.Nz + 3) / 4 * 4 : ctx->pse.Nz;
-}
+// row length of the grids in memory, for this library's transforms and for rocFFT's plans: whole float4s
+// (16-byte stores and loads for odd lengths too)
+inline int grid_pitch(const fsd_ctx *ctx) { return (ctx->pse.Nz + 3) / 4 * 4; }
 int k_precond_apply2(fsd_ctx *ctx, const float *b0, const float *b1, float *y0, float *y1, int n_rhs);
 int k_export_csr(fsd_ctx *ctx, const float4 *pos, int32_t *h_rowptr, int32_t *h_col, float *h_val,
                  int32_t *h_prow, int32_t *h_pcol, float *h_L, int64_t cap);

