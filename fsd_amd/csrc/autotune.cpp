@@ -1,9 +1,9 @@
 // Autotuner of launch shapes: times, on the context's own positions and lists,
 // every variant of the kernels that compute the same operator and keeps the
 // fastest (fsd_tuning).  Coordinate search over the wave-space knobs (spreading
-// kernel, contraction kernel, fused or 3-D x transforms), then an exhaustive
-// search over lanes per particle x workgroup size for the real-space sum and
-// for the R_FU product.  Each variant is timed with HIP events on the
+// kernel, contraction kernel, transforms in LDS or 3-D library plans), then an
+// exhaustive search over lanes per particle x workgroup size for the real-space
+// sum and for the R_FU product.  Each variant is timed with HIP events on the
 // context's stream: two untimed applies, then the mean of five.
 #include <hip/hip_runtime.h>
 
@@ -83,9 +83,10 @@ static int search(fsd_ctx *ctx, const float4 *pos)
     t.us[0] = best;
     // real space
     best = FLT_MAX;
-    int bg = t.real_g, bb = t.real_blk;
+    int bg = t.real_g, bb = t.real_blk;      // bb stays where the workgroup size is not a choice
     for (int g : {4, 8, 16})
         for (int b : {128, 256}) {
+            if (real_table_in_lds(ctx) && b != bb) continue;   // one workgroup size: the same launch again
             t.real_g = g; t.real_blk = b;
             RC(time_us(ctx, s, [&]() { return k_mobility(ctx, pos, s.gF, s.gU, 1, nullptr); }, &us));
             if (us < best) { best = us; bg = g; bb = b; }

@@ -198,7 +198,8 @@ struct fsd_tuning {
     int contract = 0;        // 0: tile contraction (contract_tile2/contract_tile, when it fits in LDS),
                              // 1: one wave per particle (contract_kernel)
     int xpass = 0;           // 0: the transforms of k_fft.hip (when the grid fits them), 1: 3-D rocFFT
-    int real_g = 16, real_blk = 256;   // real-space sum: lanes per particle (4, 8, 16), workgroup size
+    int real_g = 16, real_blk = 256;   // real-space sum: lanes per particle (4, 8, 16), workgroup size (of the
+                                       // form that reads the table from global memory)
     int rfu_g = 8, rfu_blk = 256;      // R_FU product: lanes per particle (8, 16), workgroup size
     int tuned = 0;
     float us[3] = {0.f, 0.f, 0.f};     // best time per apply (us): wave part, real part, R_FU
@@ -420,6 +421,7 @@ int k_rse(fsd_ctx *ctx, const float4 *pos, float shear_rate, const float *ori, f
 int k_setup_spread(fsd_ctx *ctx, const float4 *pos, const float *gF = nullptr);   // gF: also its records
 int k_contract_lds(fsd_ctx *ctx);
 int k_real_init(fsd_ctx *ctx);       // LDS limits of the real-space kernels; nonzero on failure
+bool real_table_in_lds(const fsd_ctx *ctx);   // the real-space sum's form for this list (its workgroup is then fixed)
 #define SCAN_CHUNK 4096
 #define SCAN_SELF 1024         // chunks whose offsets a workgroup sums for itself
 int scan_excl_chunks(int n);

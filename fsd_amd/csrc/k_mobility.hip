@@ -1113,9 +1113,18 @@ __global__ void __launch_bounds__(256) realspace_kernel(RealParams rp, const flo
 // and from global memory, by list entries: 0.33 M 12.0 and 11.3 us, 0.50 M 12.3 and 12.8, 0.75 M 14.4 and
 // 16.0, 1.0 M 18.9 and 18.1 (its workgroups end with a short pass), 1.1 M 16.5 and 19.2, 2.7 M 30 and 33,
 // 5.2 M 52 and 61.
-#define RS_RMIN 1.9f
-#define RS_ROWS 5000       // 156 KB of LDS; a longer table (xi below 0.38) stays in global memory
-#define RS_LDS_MIN 700000
+constexpr float RS_DR = 0.001f;          // distance between rows
+constexpr float RS_RMIN = 1.9f;
+constexpr int RS_ROWS = 5000;            // 156 KB of LDS; a longer table (xi below 0.38) stays in global memory
+constexpr int64_t RS_LDS_MIN = 700000;
+static int rs_first_row(const fsd_ctx *ctx)
+{
+    return std::max(0, std::min((int)(RS_RMIN / RS_DR) - 1, ctx->ewald_nR - 2));
+}
+bool real_table_in_lds(const fsd_ctx *ctx)
+{
+    return ctx->nlist_total >= RS_LDS_MIN && ctx->ewald_nR - rs_first_row(ctx) <= RS_ROWS;
+}
 template <int G>
 __global__ void __launch_bounds__(1024) realspace_lds_kernel(RealParams rp, const float4 *rec, const float4 *tab,
                                                              int row0, int nrows, const int *snn, const int *nslot,
@@ -1275,7 +1284,7 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
         }
     }
     RealParams rp;
-    rp.b = ctx->box; rp.rcut = ps.rcut; rp.dr = 0.001f; rp.self_x = ps.self_x; rp.self_y = ps.self_y;
+    rp.b = ctx->box; rp.rcut = ps.rcut; rp.dr = RS_DR; rp.self_x = ps.self_x; rp.self_y = ps.self_y;
     rp.ewald_n = ps.ewald_n;
     rp.x_scale = (float)((double)ps.ewald_n / ((double)ps.rcut - (double)rp.dr));
     rp.inv_dr = 1.0f / rp.dr;
@@ -1289,8 +1298,8 @@ int k_mobility(fsd_ctx *ctx, const float4 *pos, const float *gF, float *gU, int 
     const dim3 rg(nblk((int64_t)N * G, blk)), rb(blk);
     const float4 *tab = reinterpret_cast<const float4 *>(ctx->d_ewald);
     const int ur = (parts & 1) ? 1 : 0;
-    const int row0 = std::max(0, std::min((int)(RS_RMIN / rp.dr) - 1, ctx->ewald_nR - 2)), nrows = ctx->ewald_nR - row0;
-    const bool lds = ur && ctx->nlist_total >= RS_LDS_MIN && nrows <= RS_ROWS;
+    const int row0 = rs_first_row(ctx), nrows = ctx->ewald_nR - row0;
+    const bool lds = ur && real_table_in_lds(ctx);
     auto go = [&](auto plain, auto in_lds) {
         if (lds)
             hipLaunchKernelGGL(in_lds, dim3(256), dim3(1024), 2 * sizeof(float4) * nrows, ctx->stream, rp, rec, tab,

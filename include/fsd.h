@@ -207,7 +207,9 @@ int fsd_build_precond(fsd_ctx *ctx, const float *d_pos4, fsd_solve_stats *stats)
  * h_choice8 (may be null): spread (0 tiled, 1 per-tile), contract (0 tiled, 1 per
  * particle), xpass (0 transforms in LDS, 1 3-D rocFFT), real-space lanes, real-space
  * workgroup, R_FU lanes, R_FU workgroup, tuned; h_us3 (may be null): the best time per
- * apply in microseconds of the wave part, the real part and R_FU.  Allocates scratch. */
+ * apply in microseconds of the wave part, the real part and R_FU.  The real-space workgroup
+ * is that of the form for shorter lists: from 700000 list entries on the sum holds its table
+ * in LDS with a workgroup of 1024 per CU, and the value is kept, not tuned.  Allocates scratch. */
 int fsd_autotune(fsd_ctx *ctx, const float *d_pos4, int32_t *h_choice8, float *h_us3);
 int fsd_get_tuning(fsd_ctx *ctx, int32_t *h_choice8, float *h_us3);
 /* sets the seven choices of fsd_autotune's h_choice8 (tests, or a stored tuning) */

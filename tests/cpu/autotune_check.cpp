@@ -32,7 +32,8 @@ int k_rfu_apply(fsd_ctx *ctx, const float *, float *, const float *, float)
     now_us += ctx->tune.rfu_g == 16 ? 2.f : 3.f;
     return 0;
 }
-static bool no_plans;
+static bool no_plans, in_lds;
+bool real_table_in_lds(const fsd_ctx *) { return in_lds; }
 int fft_plans_3d(fsd_ctx *) { return no_plans ? FSD_E_HIP : 0; }
 int k_fill(fsd_ctx *, int64_t, float, float *) { return 0; }
 
@@ -90,6 +91,13 @@ int main()
         CHECK(same(c->tune, before));
         delete c;
     }
+    // where the workgroup size is not a choice, every lane count is timed once and the size stays
+    fail_product = product = 0;
+    in_lds = true;
+    cost = [](const fsd_tuning &t, int) { return 10.f + t.real_g - (t.real_blk == 128); };
+    ctx = context();
+    CHECK(autotune_run(ctx, nullptr) == 0 && ctx->tune.real_g == 4 && ctx->tune.real_blk == 256);
+    CHECK(product == products - 3 * 7);
     // without the library's plans the transforms in LDS stay, untimed against them
     fail_product = 0;
     no_plans = true;
