@@ -1,4 +1,4 @@
-"""Orthogonalisation kernels of GMRES at the edges of their forms.
+"""Orthogonalisation kernels of GMRES and Lanczos at the edges of their forms.
 
 Vectors of 17 N numbers: 2057 (three blocks, not a multiple of four), 131070 and 131087 (either side
 of the line between the short and the long form, neither a multiple of four), 139264 (16-byte accesses).
@@ -7,6 +7,11 @@ the basis is orthonormal and the coefficients are those of the projections.  The
 estimate of 1e-4 and the residual formed from its solution with FP32 products, whose rounding is of
 the order of 1e-6, may be 10 % above that.  Once or twice projected, the solves take the same number of
 iterations but for the one that rounding may shift.
+
+Lanczos takes one coefficient of each projection only.  Its square roots with vectors of 131087 and 131120
+(11 N), 131082 and 131088 numbers (6 N), just beyond the line and either a multiple of four or not, against
+the same rule in 64 bits over the GPU's own products: equal but for the rounding of the products, or for one
+step more where that shifts the stopping rule (a relative change of 1e-3).
 """
 import numpy as np
 import pytest
@@ -36,3 +41,36 @@ def test_residual_estimate(N):
         assert (r.norm() / b.double().norm()).item() <= 1.1e-4
         its.append(info["iterations"])
     assert abs(its[0] - its[1]) <= 1 and its[0] > 8      # more than one group of eight vectors
+
+
+@pytest.mark.parametrize("field,N", [("far", 11917), ("far", 11920), ("near", 21847), ("near", 21848)])
+def test_long_lanczos(field, N):
+    from fsd_amd.stokes import Stokes
+    from oracle.oracle import lanczos_sqrt_adaptive
+    n = int(np.ceil(N ** (1 / 3)))
+    L = 2.6 * n
+    rng = np.random.default_rng(N)
+    cell = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)[:N]
+    pos = (cell + 0.5) * 2.6 - L / 2 + rng.uniform(-0.25, 0.25, (N, 3))
+    p4 = torch.tensor(np.concatenate([pos, np.zeros((N, 1))], 1).astype(np.float32), device="cuda")
+    T, dt = 1.0, 1e-3
+    st = Stokes(N, L, T=T, dt=dt)
+    st.build_nlist(p4)
+    m = 11 if field == "far" else 6
+    psi = rng.standard_normal(m * N).astype(np.float32)
+    noise = torch.tensor(psi, device="cuda")
+    print("long Lanczos", field, N, flush=True)
+    if field == "far":
+        i = st.pse_info()
+        st.set_noise(noise, torch.zeros(6 * i["Nx"] * i["Ny"] * i["Nz"], device="cuda"), None, None)
+        y = st.brownian_farfield(p4)
+        op = lambda v: st.mobility(p4, torch.tensor(v, dtype=torch.float32, device="cuda"), 1)  # noqa: E731
+    else:
+        st.set_noise(None, None, noise, None)
+        y = st.brownian_nearfield(p4)
+        op = lambda v: st.rfu(p4, torch.tensor(v, dtype=torch.float32, device="cuda"))  # noqa: E731
+    ref, steps = lanczos_sqrt_adaptive(lambda v: op(v).double().cpu().numpy(), np.sqrt(2 * T / dt) * psi.astype(np.float64),
+                                       2, 1e-3)
+    assert steps > 2
+    y = y.double().cpu().numpy()
+    assert np.linalg.norm(y - ref) <= 1e-3 * np.linalg.norm(ref)

@@ -5,6 +5,9 @@ than 0.7 million list entries) takes the table from global memory, its copies fr
 and coordinates are multiples of 2^-12, so every separation is exact in both and the pair terms are
 equal: the two differ in the order of their ~80 terms only.  With that many roundings of a running
 sum at 2^-24 of it, random in sign, the difference is about 1e-6 of the largest entry; 2e-5 is allowed.
+
+The lanes per particle that the autotuner can choose, where the table is in LDS, against the FP64 oracle
+(1e-5, as for every mobility product).
 """
 import numpy as np
 import pytest
@@ -39,3 +42,23 @@ def test_table_in_lds(N, overlap):
         out.append((u[:6 * k * N].reshape(k, N, 6), u[6 * k * N:].reshape(k, N, 5)))
     for a, b in zip(*out):
         assert np.abs(b - a).max() <= 2e-5 * np.abs(a).max()
+
+
+@pytest.mark.parametrize("lanes", [4, 8, 16])
+@pytest.mark.parametrize("N", [13824, 13823])
+def test_lanes_with_table_in_lds(N, lanes):
+    from fsd_amd.stokes import Stokes
+    from oracle.oracle import Oracle
+    n, L = 24, 51.0
+    rng = np.random.default_rng(N)
+    cell = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)[:N]
+    pos = ((cell + 0.5) * (L / n) - L / 2 + rng.uniform(-0.05, 0.05, (N, 3))).astype(np.float32)
+    x = rng.standard_normal(11 * N).astype(np.float32)
+    st = Stokes(N, L)
+    p4 = torch.tensor(np.concatenate([pos, np.zeros((N, 1), np.float32)], 1), device="cuda")
+    st.build_nlist(p4)
+    assert st.get_nlist()[0].sum() >= 700000       # from there on the table is in LDS
+    st.set_tuning(real_lanes=lanes)
+    u = st.mobility(p4, torch.tensor(x, device="cuda"), 1).cpu().numpy().astype(np.float64)
+    ref = Oracle(pos, L).mobility(x, 1)
+    assert np.abs(u - ref).max() <= 1e-5 * np.abs(ref).max()
