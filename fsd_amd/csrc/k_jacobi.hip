@@ -208,10 +208,18 @@ __global__ void __launch_bounds__(256) bj_iter_kernel(int N, const int *row, con
 // each direction's blocks in registers, a block or two per thread.  An iteration is one 6x6 product
 // per block into LDS, a barrier, the sum of every row's products, a barrier: 2 us where a launch with
 // its gap takes 4 (N = 700, phi = 0.4, k = 8: 39 us against 70; the call 95 -> 70 us).  Bound by the one
-// CU's LDS and VALU, so the limits are what fits, not where it would lose.  (Six lanes per block as in
-// bj_iter_kernel read each neighbour's values six times: 54 us.)
+// CU's LDS and VALU.  (Six lanes per block as in bj_iter_kernel read each neighbour's values six times: 54 us.)
 constexpr int BS_NT = 1024, BS_HOLD = 2;
 constexpr int BS_MAXN = 1900;   // two vectors of 24 bytes a row and the products of 2048 blocks: 145 of 160 KB of LDS
+// What it saves per iteration has to pay for its first and last steps, which one CU takes over all rows: k
+// from about N / 300 on, and from 5 on for every size (11 launches take 70 to 90 us a call, by the gap between
+// them, which has two values here).  Calls by one workgroup and by launches, us, at k = 1, 2, 3, 5, 8:
+//   N = 343,  828 blocks   41 44 45 49 54   42 48 55 71 91
+//   N = 700,  1465         48 50 53 58 65   41 47 55 73 90
+//   N = 1000, 1563         52 54 57 63 72   41 48 54 71 89
+//   N = 1500, 1462         57 60 62 67 75   40 46 52 69 87
+//   N = 1900, 2046         63 66 70 78 89   41 46 53 69 88
+inline bool bs_pays(int N, int k) { return k >= 5 || N <= 300 * k + 50; }
 constexpr int BS_SUM = 3;       // products of a row read together
 template <int HOLD>
 __global__ void __launch_bounds__(BS_NT) bj_small_kernel(int N, int nlow, int k, const int *lrow, const int *lcol,
@@ -352,7 +360,7 @@ int k_bj_apply(fsd_ctx *ctx, int k, int prof_slot, const float *R, const float *
     const int64_t n6 = 6 * (int64_t)N;
     hipEvent_t ev, e1;
     const int nlow = (int)ctx->pch.nlow;
-    if (N <= BS_MAXN && nlow <= BS_HOLD * BS_NT) {
+    if (N <= BS_MAXN && nlow <= BS_HOLD * BS_NT && bs_pays(N, k)) {
         const size_t lds = sizeof(float) * (2 * n6 + 6 * (nlow + 1)) + sizeof(unsigned short) * (N + 2);
         const BjPost post{ctx->d_perm, Zpost, bsaddle, x, mode};
         auto go = [&](auto kernel) -> int {
