@@ -58,19 +58,29 @@ int k_fill(fsd_ctx *ctx, int64_t n, float v, float *y)
 // one, two or four chunks).
 //   short: dots | sum, axpy, dots | sum, axpy, norm | sum, scale
 //   long:  dots | sum | axpy | dots | sum | axpy, norm | sum, scale
+// In the short form's second launch a block goes through all K vectors twice, so with two passes it is the
+// shorter one up to about 20 vectors only.  Mean over K = 1 .. R of both forms, us:
+//   two passes      n = 17000     42500     102000    130900    204000    557056
+//     R = 16           20 25     21 26      24 27     23 26     25 28     33 35
+//     R = 32           24 26     26 27      29 30     27 29     33 33     50 47
+//     R = 64           30 29     34 30      43 35     38 35     49 45     84 68
+//   one pass
+//     R = 64           16 18     19 19      21 21     20 21     24 26     45 38
+//     R = 100          19 20     23 22      26 26     25 25     31 31     62 51
 // The short products and the updates read the vectors eight at a time, and the eight sums over a wave's
 // lanes share one butterfly (10 exchanges, 48 one by one).
 #define GS_NT 256
 #define GS_CH (4 * GS_NT)     // numbers of a block, four to a thread
 #define GS_KMAX 256
 #define GS_FUSED (1 << 17)
+#define GS_FUSED_K 20         // with two passes
 #define GS_LONG 4             // chunks of a block of the long products
 
 static int gs_chunks(int64_t n) { return (int)((n + GS_CH - 1) / GS_CH); }
-static int gs_dot_blocks(int64_t n) { return n > GS_FUSED ? (gs_chunks(n) + GS_LONG - 1) / GS_LONG : gs_chunks(n); }
-int64_t gs_part_doubles(int64_t n, int K)      // for every length up to n
+static int gs_dot_blocks(int64_t n, bool lng) { return lng ? (gs_chunks(n) + GS_LONG - 1) / GS_LONG : gs_chunks(n); }
+int64_t gs_part_doubles(int64_t n, int K)      // for every length up to n, in either form
 {
-    const int64_t blocks = n > GS_FUSED ? std::max(gs_dot_blocks(n), GS_FUSED / GS_CH) : gs_chunks(n);
+    const int64_t blocks = n > GS_FUSED ? std::max(gs_dot_blocks(n, true), GS_FUSED / GS_CH) : gs_chunks(n);
     return std::max(std::min(K, GS_KMAX) * blocks, (int64_t)gs_chunks(n));
 }
 
@@ -347,10 +357,10 @@ static int gs_launch(fsd_ctx *ctx, int64_t n, int K, const float *V, const float
     return 0;
 }
 
-static int gs_dots(fsd_ctx *ctx, int64_t n, int K, const float *V, const float *w, double *out)
+static int gs_dots(fsd_ctx *ctx, int64_t n, int K, const float *V, const float *w, double *out, bool lng)
 {
-    const bool vec = vec4_ok(n, n, V, w), lng = n > GS_FUSED;
-    const dim3 grid(gs_dot_blocks(n), lng ? K : (K + 7) / 8);
+    const bool vec = vec4_ok(n, n, V, w);
+    const dim3 grid(gs_dot_blocks(n, lng), lng ? K : (K + 7) / 8);
     if (lng) {
         auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(GS_NT), 0, ctx->stream, n, V, w, out); };
         vec ? go(gs_dots_long_kernel<true>) : go(gs_dots_long_kernel<false>);
@@ -366,22 +376,23 @@ int k_gs_orthonormalise(fsd_ctx *ctx, int64_t n, int K, const float *V, float *w
                         double *h2, double *norm)
 {
     if (K > GS_KMAX) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
+    const bool lng = n > GS_FUSED || (passes == 2 && K > GS_FUSED_K);
     double *a = ctx->d_part[0], *b = ctx->d_part[1];
-    int rc = gs_dots(ctx, n, K, V, w, a);
+    int rc = gs_dots(ctx, n, K, V, w, a, lng);
     for (int pass = 1; pass <= passes && !rc; ++pass) {
         double *h = pass == 1 ? h1 : h2;
         const bool last = pass == passes;
-        int np = gs_dot_blocks(n);
-        if (n > GS_FUSED) {
+        int np = gs_dot_blocks(n, lng);
+        if (lng) {
             hipLaunchKernelGGL(gs_sum_kernel, dim3(K), dim3(GS_NT), 0, ctx->stream, a, np, b, h, kfirst);
             std::swap(a, b);
             np = 1;
             h = nullptr;
         }
         if (last) rc = gs_launch<true, false, true>(ctx, n, K, V, w, a, np, h, kfirst, b);
-        else if (n > GS_FUSED) rc = gs_launch<true, false, false>(ctx, n, K, V, w, a, np, h, kfirst, nullptr);
+        else if (lng) rc = gs_launch<true, false, false>(ctx, n, K, V, w, a, np, h, kfirst, nullptr);
         else rc = gs_launch<true, true, false>(ctx, n, K, V, w, a, np, h, kfirst, b);
-        if (!last && n > GS_FUSED && !rc) rc = gs_dots(ctx, n, K, V, w, b);
+        if (!last && lng && !rc) rc = gs_dots(ctx, n, K, V, w, b, lng);
         std::swap(a, b);
     }
     return rc ? rc : k_gs_scale(ctx, n, w, w, a, norm);

@@ -74,3 +74,46 @@ def test_long_lanczos(field, N):
     assert steps > 2
     y = y.double().cpu().numpy()
     assert np.linalg.norm(y - ref) <= 1e-3 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("N", [1001, 6000])
+def test_two_passes_of_many_vectors(N):
+    """two projections on more than 20 vectors: the residual estimate as above, and (N = 6000, 102000 numbers, up
+    to 60 vectors) they take about 1.6 times as long as one, 34 and 21 us in the mean; where blocks go through
+    all vectors twice, 43 us; 1.8 times is allowed"""
+    from fsd_amd.stokes import Stokes
+    n = int(np.ceil(N ** (1 / 3)))
+    L = 2.6 * n
+    rng = np.random.default_rng(N)
+    cell = np.stack(np.meshgrid(*[np.arange(n)] * 3, indexing="ij"), -1).reshape(-1, 3)[:N]
+    pos = (cell + 0.5) * 2.6 - L / 2 + rng.uniform(-0.25, 0.25, (N, 3))
+    p4 = torch.tensor(np.concatenate([pos, np.zeros((N, 1))], 1).astype(np.float32), device="cuda")
+    b = torch.tensor(rng.standard_normal(17 * N).astype(np.float32), device="cuda")
+    us, its = [], []
+    for passes in (1, 2):
+        st = Stokes(N, L, gmres_true_tol=1e-5, gmres_restart=100, gram_schmidt_passes=passes, precond="ichol_jacobi",
+                    jacobi_iters=1)
+        st.build_nlist(p4)
+        st.build_precond(p4)
+        x, info = st.saddle_solve(p4, b)
+        r = b.double() - st.saddle_multiply(p4, x).double()
+        assert info["converged"] and info["restarts"] == 1
+        assert (r.norm() / b.double().norm()).item() <= 1.1e-5
+        its.append(info["iterations"])
+        st = Stokes(N, L, gmres_tol=1e-12, gmres_maxiter=60, gmres_restart=60, gram_schmidt_passes=passes,
+                    precond="ichol_jacobi", jacobi_iters=1)
+        st.build_nlist(p4)
+        st.build_precond(p4)
+        st.saddle_solve(p4, b)
+        st.profile(True, classes=["gmres_vec"])
+        best = 1e30
+        for _ in range(5):
+            st.profile_reset()
+            st.saddle_solve(p4, b)
+            count, ms = st.profile_get("gmres_vec")
+            best = min(best, 1e3 * ms / count)
+        us.append(best)
+    print("one and two passes", N, its, us)
+    assert abs(its[0] - its[1]) <= 1 and its[0] > 20
+    if N == 6000:
+        assert us[1] < 1.8 * us[0]
