@@ -11,9 +11,9 @@
 // with the library's 2-D transforms in the place of the first and the last where a plane exceeds LDS.
 //
 // Bound: HBM for large grids, the barriers between the LDS stages for small ones.  Measured
-// (mobility product, HIP kernel times): 135^3, three passes 251 us where the 3-D library plans of
-// this odd length and the separate Green's function took 1137 us (product 1820 -> 941 us); 72^3,
-// 66 us against 65 us with the library's 2-D transforms; 40^3, 30 us; 20^3, 22 us (23 us).
+// (mobility product, kernel trace): 135^3, three passes 252 us where the 3-D library plans of this
+// odd length and the separate Green's function took 1113 us; 72^3, 64 us as with the library's 2-D
+// transforms; 40^3, 30 us against 37; 20^3, 22 us against 23 (3-D plans).
 // Each pass reads and writes its data once, so a product moves 6 x 11 x 4 M bytes here
 // whatever the lengths' factors are.  Grid lengths are 2^a 3^b 5^c; fft::split splits
 // them into few large radices, which a thread transforms in registers.
@@ -338,9 +338,9 @@ hipError_t allow_lds(K kernel, size_t bytes)
 // ctx->fft_x stays false and the 3-D library plans are used.  The planes are a matter of their own:
 // those that fit LDS (up to about 200 points per axis) are transformed there, larger ones by the
 // library's 2-D plans, from X_ALONE points along x on.  Wave part of a product that way and with the 3-D
-// plans, us: 40 x 225 x 240 683 and 716, 48 x 200 x 216 523 and 711, 72 x 225 x 240 1231 and 1410, 80 x 256^2
-// 1323 and 1372, 135 x 216 x 225 3132 and 4435, 200^3 1874 and 2109, 256^3 4618 and 4693, 400 x 200^2 4049 and
-// 5706; shorter axes gain nothing (24 x 225 x 240 473 and 470, 12 x 225 x 240 326 and 333).
+// plans, us: 40 x 225 x 240 656 and 706, 48 x 200 x 216 514 and 680, 72 x 225 x 240 1205 and 1373, 80 x 256^2
+// 1254 and 1335, 135 x 216 x 225 2940 and 4246, 200^3 1813 and 2039, 225^3 6879 and 8581, 256^3 4520 and 4642,
+// 400 x 200^2 3934 and 5590; shorter axes gain nothing (24 x 225 x 240 473 and 470, 12 x 225 x 240 326 and 333).
 constexpr int X_ALONE = 40;
 int fft_init(fsd_ctx *ctx)
 {

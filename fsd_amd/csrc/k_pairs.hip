@@ -132,9 +132,9 @@ __global__ void cell_scatter_kernel(const int *cell_of, int N, const int *start,
     list[start[c] + slot] = i;
 }
 
-// deterministic order inside a cell: ascending particle index, one wave per cell.  A cell of up to
-// 256 particles is held in registers (four per lane) and each key stored at its rank, the number of
-// smaller keys (the keys differ); a fuller one (spheres that overlap) is sorted by one lane.
+// deterministic order inside a cell: ascending particle index, one wave per cell.  The keys of a cell of
+// up to 256 particles are staged in LDS; a lane counts the smaller ones of each of its keys (they all
+// differ) and stores the key at that rank.  A fuller cell (spheres that overlap) is sorted by one lane.
 __global__ void __launch_bounds__(64) cell_sort_kernel(const int *start, int ncells, int *list)
 {
     __shared__ int keys[256];

@@ -375,7 +375,7 @@ static int gs_dots(fsd_ctx *ctx, int64_t n, int K, const float *V, const float *
 int k_gs_orthonormalise(fsd_ctx *ctx, int64_t n, int K, const float *V, float *w, int passes, int kfirst, double *h1,
                         double *h2, double *norm)
 {
-    if (K > GS_KMAX) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
+    if (K > GS_KMAX) { ctx->err = "more than 256 vectors to orthogonalise against or to combine"; return FSD_E_PARAM; }
     const bool lng = n > GS_FUSED || (passes == 2 && K > GS_FUSED_K);
     double *a = ctx->d_part[0], *b = ctx->d_part[1];
     int rc = gs_dots(ctx, n, K, V, w, a, lng);
@@ -418,7 +418,7 @@ int k_gs_scale(fsd_ctx *ctx, int64_t n, const float *w, float *v, const double *
 int k_gs_combine(fsd_ctx *ctx, int64_t n, int K, const float *V, const double *c, const float *x0, float *out,
                  const float *prev, double *part, int *nch)
 {
-    if (K > GS_KMAX) { ctx->err = "multi_axpy: more than 256 vectors"; return FSD_E_PARAM; }
+    if (K > GS_KMAX) { ctx->err = "more than 256 vectors to orthogonalise against or to combine"; return FSD_E_PARAM; }
     GsCoef coef;
     for (int k = 0; k < GS_KMAX; ++k) coef.c[k] = k < K ? (float)c[k] : 0.f;
     auto go = [&](auto kernel) {

@@ -1313,6 +1313,9 @@ int fsd_rfd_drift(fsd_ctx *ctx, const float *d_pos4, uint32_t timestep, float *d
 
 // The lubrication operators run behind the list's check without waiting for it; the host looks once,
 // at the end, and runs them again over a new list (or pair records of a larger capacity) if it must.
+// Such a call has run its operator once in vain, about 20 us of 190 at N = 9261; with 30 spheres R_FU takes
+// 148 us in a call that rebuilds the list, 136 where the host waited for the check first, and 53 instead
+// of 70 in one that does not.
 int fsd_rfu(fsd_ctx *ctx, const float *d_pos4, const float *d_U6, float *d_F6)
 {
     const float4 *pos = reinterpret_cast<const float4 *>(d_pos4);
