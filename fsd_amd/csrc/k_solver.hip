@@ -59,7 +59,9 @@ int k_fill(fsd_ctx *ctx, int64_t n, float v, float *y)
 //   short: dots | sum, axpy, dots | sum, axpy, norm | sum, scale
 //   long:  dots | sum | axpy | dots | sum | axpy, norm | sum, scale
 // In the short form's second launch a block goes through all K vectors twice, so with two passes it is the
-// shorter one up to about 20 vectors only.  Mean over K = 1 .. R of both forms, us:
+// shorter one up to about 20 vectors only, 32 below 65536 numbers (the near-field square root of a Brownian
+// step at N = 1000, some 40 steps of 6000 numbers: 813 us a call at 20, 790 at 32).  Mean over K = 1 .. R of both
+// forms, us:
 //   two passes      n = 17000     42500     102000    130900    204000    557056
 //     R = 16           20 25     21 26      24 27     23 26     25 28     33 35
 //     R = 32           24 26     26 27      29 30     27 29     33 33     50 47
@@ -73,8 +75,9 @@ int k_fill(fsd_ctx *ctx, int64_t n, float v, float *y)
 #define GS_CH (4 * GS_NT)     // numbers of a block, four to a thread
 #define GS_KMAX 256
 #define GS_FUSED (1 << 17)
-#define GS_FUSED_K 20         // with two passes
 #define GS_LONG 4             // chunks of a block of the long products
+
+static int gs_fused_k(int64_t n) { return n > (1 << 16) ? 20 : 32; }     // with two passes
 
 static int gs_chunks(int64_t n) { return (int)((n + GS_CH - 1) / GS_CH); }
 static int gs_dot_blocks(int64_t n, bool lng) { return lng ? (gs_chunks(n) + GS_LONG - 1) / GS_LONG : gs_chunks(n); }
@@ -376,7 +379,7 @@ int k_gs_orthonormalise(fsd_ctx *ctx, int64_t n, int K, const float *V, float *w
                         double *h2, double *norm)
 {
     if (K > GS_KMAX) { ctx->err = "more than 256 vectors to orthogonalise against or to combine"; return FSD_E_PARAM; }
-    const bool lng = n > GS_FUSED || (passes == 2 && K > GS_FUSED_K);
+    const bool lng = n > GS_FUSED || (passes == 2 && K > gs_fused_k(n));
     double *a = ctx->d_part[0], *b = ctx->d_part[1];
     int rc = gs_dots(ctx, n, K, V, w, a, lng);
     for (int pass = 1; pass <= passes && !rc; ++pass) {

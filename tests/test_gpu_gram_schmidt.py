@@ -78,9 +78,9 @@ def test_long_lanczos(field, N):
 
 @pytest.mark.parametrize("N", [1001, 6000])
 def test_two_passes_of_many_vectors(N):
-    """two projections on more than 20 vectors: the residual estimate as above, and (N = 6000, 102000 numbers, up
-    to 60 vectors) they take about 1.6 times as long as one, 34 and 21 us in the mean; where blocks go through
-    all vectors twice, 43 us; 1.8 times is allowed"""
+    """two projections on more than 20 vectors, where N = 6000 (102000 numbers) goes from one form to the other
+    on the way: the residual estimate as above, and up to 60 vectors take about 1.6 times as long as one
+    projection, 34 and 21 us in the mean; where blocks go through all vectors twice, 43 us; 1.8 times is allowed"""
     from fsd_amd.stokes import Stokes
     n = int(np.ceil(N ** (1 / 3)))
     L = 2.6 * n
