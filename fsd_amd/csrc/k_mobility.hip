@@ -369,7 +369,7 @@ __global__ void __launch_bounds__(512) spread_kernel(SpreadGeom g, const int *or
 // x 4 nodes), of which 19 count, at twice the VALU's rate.  The same sums on the VALU were bound
 // by lanes that waited for the longest of 36 short runs of spheres (34.6 us per product at N =
 // 32768) or, with those runs merged, by LDS bank conflicts (each lane its own sphere: 34.6 us); this form takes
-// 23 us (13 us at N = 4072), of which half are the dependent loads before the products and the
+// 21 us (13 us at N = 4072), of which half are the dependent loads before the products and the
 // stores after them.
 // The tile's halo of 13^3 origin cells is staged in LDS.  Its spheres are in the order of buckets
 // (x, third of z, y): a wave of the lower nodes needs the first two thirds, one of the upper
